@@ -17,6 +17,7 @@
 // of the workgroup compute the tile's OBS_SPLIT parts per env.
 #pragma once
 #include "policy_bf16.h"
+#include "policy_lane.h"
 #include "policy_split.h"
 #include "sample.h"
 
@@ -304,6 +305,196 @@ __global__ void __launch_bounds__((CollectShape<M, Env::OBS_DIM, WIDE>::NT),
     }
 }
 
+// collect on the row-per-lane-pair forward (policy_lane.h): a workgroup of
+// kLaneTile envs on four waves, two workgroups per CU, lanes 0 .. 31 of a wave
+// its env lanes. Observations pass between the lanes of a wave, so
+// the only barriers are the weight ring's, and a wave's LN, head and env
+// phases run beside the other workgroup's products.
+template <typename Env, int PREC>
+struct CollectLane {
+    using Tr = EnvTraits<Env>;
+    static constexpr int O = Env::OBS_DIM, HD = Env::ACT_DIM + 1;
+    static constexpr int HC = (HD + 3) / 4 * 4;  // head columns, padded
+    // parts of a split observation: lane (n, q) computes the parts p = 2 s + q
+    // of row n, which are its embed operands
+    static constexpr uint32_t KS = Tr::STATE_IN_REGISTERS ? 0 : Tr::OBS_SPLIT;
+    static constexpr int NOB = (O + 1) / 2;
+    static constexpr uint32_t WIN = O <= 16 ? O * kEmbed : 0;  // W_in in LDS
+    // a wave's heads; an fp32 policy's categorical draws near an edge also need
+    // a row's scratch (tile_row_head)
+    static constexpr bool EDGE = PREC == MG_PRECISION_FP32 && !Tr::CONTINUOUS && Env::ACT_DIM > 1;
+    static constexpr uint32_t ROW = (kLaneRows * HD + 3) / 4 * 4;
+    static constexpr uint32_t IO = ROW + (EDGE ? kLaneRowLds : 0);
+    static constexpr bool OK = HD <= 16;  // the head's columns are registers
+};
+
+template <typename Env, int PREC>
+__global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_collect_args a) {
+    using CL = CollectLane<Env, PREC>;
+    using Tr = EnvTraits<Env>;
+    using State = typename Env::State;
+    using Action = typename Env::Action;
+    using Obs = typename Env::Obs;
+    constexpr int O = CL::O, A = Env::ACT_DIM, HD = CL::HD, HC = CL::HC, NOB = CL::NOB;
+    constexpr uint32_t KS = CL::KS;
+    extern __shared__ __align__(16) float lane_lds_f[];
+    const LaneLds L = lane_lds<PREC, HC>(a.policy.layers, CL::WIN, CL::IO);
+    LaneParams<HC> P;
+    LaneRing<PREC> ring;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = lane & 31, q = lane >> 5;
+    const uint32_t n = a.n, T = a.horizon;
+    const uint32_t i0 = blockIdx.x * kLaneTile + (uint32_t)(kLaneRows * wave);
+    // n is a multiple of 64, so a wave's rows are all there or none; a wave of
+    // none still moves its share of the weights, on row 0's values
+    const bool valid = i0 < n;
+    const uint32_t i = valid ? i0 + (uint32_t)row : (uint32_t)row;
+    const bool envLane = valid && q == 0;
+    const bool wide = n >= 64u * 512u;  // the tile height that launch_collect_tiles would take
+    float* ioL = lane_lds_f + L.io + wave * (int)CL::IO;
+    float* headL = ioL + row * HD;
+    State* states = static_cast<State*>(a.state);
+    Action* actSlots = static_cast<Action*>(a.action_slots);
+    const float* logStd = a.policy.params + a.policy.off_log_std;
+
+    uint32_t rng = 0;
+    uint8_t done = 0;
+    std::conditional_t<Tr::STATE_IN_REGISTERS, State, char> sreg;
+    auto S = [&]() -> State& {
+        if constexpr (Tr::STATE_IN_REGISTERS)
+            return sreg;
+        else
+            return states[i];
+    };
+    float ob[NOB];  // this lane's embed operands: observation floats 2 s + q of its row
+    // Steps the env lanes with act and passes the observation on: to its slot
+    // and to the lanes' embed operands.
+    auto env_step = [&](const Action& act, size_t slot, float& r) {
+        if constexpr (KS > 0) {
+            if (envLane) {
+                if (done) Env::reset(S(), rng);
+                Env::stepState(S(), act, r, done);
+            }
+            // the stepped state is read by both lanes of the row
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            const State& s = states[i];
+            Obs o{};
+            Env::observeRest(s, o);
+            const float* of = reinterpret_cast<const float*>(&o);
+#pragma unroll
+            for (int u = 0; u < NOB; ++u) {
+                constexpr int K = (int)KS;
+                float v = 0.0f;
+                if (2 * u + 1 < K) {
+                    v = Env::observePart(s, 2 * u + q);
+                } else {
+                    const float e = 2 * u < K ? 0.0f : of[2 * u];
+                    const float d = 2 * u + 1 < O ? of[2 * u + 1 < O ? 2 * u + 1 : 0] : 0.0f;
+                    v = q ? d : e;
+                    if (2 * u < K) {
+                        if (q == 0) v = Env::observePart(s, 2 * u);
+                    }
+                }
+                ob[u] = v;
+                if (valid && 2 * u + q < O) a.obs_slots[slot * O + 2 * u + q] = v;
+            }
+        } else {
+            float obs[2 * NOB];
+#pragma unroll
+            for (int k = 0; k < 2 * NOB; ++k) obs[k] = 0.0f;
+            if (envLane) {
+                if (done) Env::reset(S(), rng);
+                Obs o{};
+                Env::step(S(), act, o, r, done);
+                const float* of = reinterpret_cast<const float*>(&o);
+#pragma unroll
+                for (int k = 0; k < O; ++k) obs[k] = of[k];
+                store_floats<O>(a.obs_slots + slot * O, obs);
+            }
+#pragma unroll
+            for (int u = 0; u < NOB; ++u) ob[u] = lane_give(obs[2 * u], obs[2 * u + 1]);
+        }
+    };
+
+    lane_start<PREC, HC>(a.policy, lane_lds_f, L, CL::WIN, P, ring);
+    if (envLane) {
+        rng = a.rng[i];
+        done = a.done[i];
+        if constexpr (Tr::STATE_IN_REGISTERS) sreg = states[i];
+    }
+    if (a.first) {  // model/ppo.h:720-722: one step with action 0 into slot 0
+        Action act{};
+        float r = 0.0f;
+        env_step(act, i, r);
+        if (envLane) a.reward_slots[i] = r;
+    } else {  // model/ppo.h:724: obs[T] -> obs[0]
+#pragma unroll
+        for (int u = 0; u < NOB; ++u) {
+            const bool in = 2 * u + q < O;
+            const float v = a.obs_slots[((size_t)T * n + i) * O + (in ? 2 * u + q : 0)];
+            ob[u] = in ? v : 0.0f;
+            if (valid && in) a.obs_slots[(size_t)i * O + 2 * u + q] = v;
+        }
+    }
+
+    for (uint32_t t = 0; t <= T; ++t) {
+        float hv[HC];
+        lane_forward<PREC, HC, O, (CL::WIN > 0)>(a.policy, P, ring, O, ob, hv);
+        if (t == T) {  // bootstrap head for GAE and headValue()
+            if (envLane) {
+#pragma unroll
+                for (int j = 0; j < HD; ++j) a.head_out[(size_t)i * HD + j] = hv[j];
+            }
+            break;
+        }
+        const size_t k = (size_t)t * n + i;
+        Action act{};
+        float r = 0.0f, lp = 0.0f, edge = 1.0f;
+        const uint32_t rng0 = rng;
+        if (envLane) {
+#pragma unroll
+            for (int j = 0; j < HD; ++j) headL[j] = hv[j];  // the samplers index the row
+            if constexpr (Tr::CONTINUOUS)
+                sample_gaussian(headL, logStd, A, rng, reinterpret_cast<float*>(&act), lp);
+            else
+                act = (Action)sample_categorical(headL, A, rng, lp, CL::EDGE ? &edge : nullptr);
+        }
+        if constexpr (CL::EDGE) {
+            for (uint64_t near = __ballot(envLane && edge <= kLaneEdge); near; near &= near - 1) {
+                const int e = __builtin_ctzll(near);
+                const float* ep = a.obs_slots + ((size_t)t * n + i0 + (uint32_t)e) * O;
+                if (wide)
+                    tile_row_head<32, O, HD>(a.policy, ep, ioL + CL::ROW, ioL + e * HD);
+                else
+                    tile_row_head<16, O, HD>(a.policy, ep, ioL + CL::ROW, ioL + e * HD);
+                if (lane == e) {
+                    const float mine = lp;
+                    uint32_t s = rng0;
+                    const Action own = act;
+                    act = (Action)sample_categorical(headL, A, s, lp);
+                    if (act == own) lp = mine;
+                }
+            }
+        }
+        if (envLane) {
+            actSlots[k] = act;
+            a.logp_slots[k] = lp;
+            a.value_slots[k] = hv[A];
+        }
+        env_step(act, k + n, r);
+        if (envLane) {
+            a.reward_slots[k] = r;
+            a.done_slots[k] = done;
+        }
+    }
+    if (envLane) {
+        if constexpr (Tr::STATE_IN_REGISTERS) states[i] = sreg;
+        a.rng[i] = rng;
+        a.done[i] = done;
+    }
+}
+
 // The kernel's static LDS as the compiler laid it out (SIZE_MAX if the
 // runtime cannot tell, which turns the small-parameter staging off).
 template <typename Env, int M, bool BF16, bool WIDE>
@@ -349,9 +540,33 @@ void launch_collect_m(const mg_collect_args* a, hipStream_t st) {
     launch_collect_mw<Env, M, BF16, false>(a, st);
 }
 
+// Runs the collect on collect_lane_kernel where that is the faster: from 16384
+// envs in fp32 and 32768 in bf16 (128 and 256 workgroups), for heads of up to
+// 16 columns. ms a collect of 32 steps, the tiles below against this, CartPole:
+// fp32 2.32 / 1.81 at 16384 envs, 4.26 / 1.81 at 32768, 8.49 / 2.97 at 65536,
+// 33.6 / 11.3 at 262144 (1.15 PFLOP/s of binary16 products, what the library's
+// 8192^3 binary16 product reaches here); bf16 0.58 / 0.77 at 16384, 0.95 / 0.77
+// at 32768, 6.54 / 4.47 at 262144; VoxelNav16 262144: fp32 37.2 / 12.9, bf16
+// 9.35 / 5.96.
+template <typename Env, int PREC>
+bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
+    using CL = CollectLane<Env, PREC>;
+    if constexpr (CL::OK) {
+        if (a->n < (PREC == MG_PRECISION_BF16 ? 32768u : 16384u) || !a->policy.frag_fwd32_bf) return false;
+        const size_t lds = (size_t)lane_lds<PREC, CL::HC>(a->policy.layers, CL::WIN, CL::IO).total * 4;
+        if (lds > 163840 / 2) return false;
+        hipLaunchKernelGGL((collect_lane_kernel<Env, PREC>), dim3((a->n + kLaneTile - 1) / kLaneTile), dim3(kLaneNT),
+                           lds, st, *a);
+        return true;
+    } else {
+        return false;
+    }
+}
+
 template <typename Env, bool BF16>
 int launch_collect_tiles(const mg_collect_args* a) {
     hipStream_t st = static_cast<hipStream_t>(a->stream);
+    if (launch_collect_lane<Env, BF16 ? MG_PRECISION_BF16 : MG_PRECISION_FP32>(a, st)) return (int)hipGetLastError();
     // 64-row tiles reuse each weight fragment across the most rows; they need
     // n / 64 >= 512 workgroups (2 per CU) to fill the chip. Smaller runs use
     // 32-row, then 16-row tiles for more workgroups.

@@ -10,8 +10,11 @@ namespace dev {
 constexpr float kLogSqrt2Pi = 0.9189385332046727f;  // 0.5 * log(2 pi)
 constexpr float kPiF = 3.14159265358979323846f;
 
-// model/sample.metal:18-47: inverse-CDF draw; returns the action.
-__device__ __forceinline__ int sample_categorical(const float* h, int A, uint32_t& rng, float& logp) {
+// model/sample.metal:18-47: inverse-CDF draw; returns the action. edge: also
+// how far the draw fell from the nearest inner edge of the CDF, as a share of
+// the whole.
+__device__ __forceinline__ int sample_categorical(const float* h, int A, uint32_t& rng, float& logp,
+                                                  float* edge = nullptr) {
     float rowMax = -__builtin_huge_valf();
     for (int a = 0; a < A; ++a) rowMax = rowMax < h[a] ? h[a] : rowMax;
     float sum = 0.0f;
@@ -28,6 +31,14 @@ __device__ __forceinline__ int sample_categorical(const float* h, int A, uint32_
         }
     }
     logp = h[chosen] - lse;
+    if (edge) {
+        float e = sum, cdf = 0.0f;
+        for (int a = 0; a + 1 < A; ++a) {
+            cdf += mg::expf(h[a] - rowMax);
+            e = fminf(e, fabsf(u - cdf));
+        }
+        *edge = e / sum;
+    }
     return chosen;
 }
 

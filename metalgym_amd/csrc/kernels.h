@@ -57,8 +57,8 @@ int train_ws_bytes(const mg_policy_view& pv, uint32_t rows, size_t* bytes);
 int train_ws_bind(const mg_policy_view& pv, uint32_t rows, void* base, TrainWs* ws);
 // One minibatch: rows pass, weight-gradient pass, reduce + norm, Adam. Adam
 // rewrites only the fragment-tiled copies the row pass reads (frag_fwd16 and
-// frag_bwd16, or their bf16 versions in bf16 mode); the others (frag_fwd32
-// and, in bf16 mode, the fp32 copies and frag_fwd32_bf, read by collect and
+// frag_bwd16, or their bf16 versions in bf16 mode); the others (frag_fwd32,
+// frag_fwd32_bf and, in bf16 mode, the fp32 copies, read by collect and
 // forward) are stale afterwards until launch_derive_blocks.
 int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hparams& hp, float lr,
                       const TrainWs& ws, const TrainStep& step, const float* obs_slots, const void* action_slots,

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "kernels.h"
+#include "mg/device/policy_lane.h"
 
 struct mg_ppo {
     mg_gym* gym = nullptr;
@@ -115,6 +116,12 @@ void shuffle_blocks(uint64_t& s, std::vector<uint32_t>& order) {
         const uint32_t j = (uint32_t)(splitmix(s) % (uint64_t)i);
         std::swap(order[i - 1], order[j]);
     }
+}
+
+// frag_fwd32_bf: one bfloat16 plane, or an fp32 policy's two binary16 planes
+// and their scales.
+size_t fwd32_bf_bytes(const mg_policy_view& pv) {
+    return 2 * (pv.precision == MG_PRECISION_BF16 ? (size_t)pv.count : dev::split_elems(pv.count));
 }
 
 int ensure_head(mg_ppo* p, uint32_t rows) {
@@ -321,9 +328,9 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
         (rc = device_alloc((void**)&pv.frag_fwd32, (size_t)pv.count * 4, "PPOModel forward matrix tiles")) ||
         (rc = device_alloc((void**)&pv.frag_fwd16, (size_t)pv.count * 4, "PPOModel forward matrix tiles")) ||
         (rc = device_alloc((void**)&pv.frag_bwd16, (size_t)pv.count * 4, "PPOModel backward matrix tiles")) ||
+        (rc = device_alloc((void**)&pv.frag_fwd32_bf, fwd32_bf_bytes(pv), "PPOModel 16-bit matrix tiles")) ||
         (pv.precision == MG_PRECISION_BF16 &&
-         ((rc = device_alloc((void**)&pv.frag_fwd32_bf, (size_t)pv.count * 2, "PPOModel bf16 matrix tiles")) ||
-          (rc = device_alloc((void**)&pv.frag_fwd16_bf, (size_t)pv.count * 2, "PPOModel bf16 matrix tiles")) ||
+         ((rc = device_alloc((void**)&pv.frag_fwd16_bf, (size_t)pv.count * 2, "PPOModel bf16 matrix tiles")) ||
           (rc = device_alloc((void**)&pv.frag_bwd16_bf, (size_t)pv.count * 2, "PPOModel bf16 matrix tiles")))) ||
         (rc = device_alloc((void**)&p->m, (size_t)pv.count * 4, "PPOModel adam m")) ||
         (rc = device_alloc((void**)&p->v, (size_t)pv.count * 4, "PPOModel adam v")) ||
@@ -356,7 +363,8 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
         hipMemsetAsync(pv.frag_fwd32, 0, (size_t)pv.count * 4, st) != hipSuccess ||
         hipMemsetAsync(pv.frag_fwd16, 0, (size_t)pv.count * 4, st) != hipSuccess ||
         hipMemsetAsync(pv.frag_bwd16, 0, (size_t)pv.count * 4, st) != hipSuccess ||
-        (pv.frag_fwd32_bf && hipMemsetAsync(pv.frag_fwd32_bf, 0, (size_t)pv.count * 2, st) != hipSuccess) ||
+        (pv.frag_fwd32_bf &&
+         hipMemsetAsync(pv.frag_fwd32_bf, 0, fwd32_bf_bytes(pv), st) != hipSuccess) ||
         (pv.frag_fwd16_bf && hipMemsetAsync(pv.frag_fwd16_bf, 0, (size_t)pv.count * 2, st) != hipSuccess) ||
         (pv.frag_bwd16_bf && hipMemsetAsync(pv.frag_bwd16_bf, 0, (size_t)pv.count * 2, st) != hipSuccess))
         return fail(set_error(MG_ERR_HIP, "PPOModel: initialisation upload failed"));

@@ -29,6 +29,7 @@
 
 #include "kernels.h"
 #include "mg/device/policy_bf16.h"
+#include "mg/device/policy_lane.h"
 #include "mg/device/sample.h"
 
 namespace mg {
@@ -1214,11 +1215,59 @@ __device__ __forceinline__ void store_tile_frags(const MatTile& m, const float* 
     }
 }
 
-// The fragment-tiled copies from params, one tile per workgroup.
+// Writes the tile held in lds to the binary16 planes of the split forward
+// (policy_lane.h): the transpose in the order of the 32-wide bf16 copy, each
+// element times scale, the hi halves in planes, the lo halves `count` elements
+// later. After a barrier that follows the tile's LDS stores.
+__device__ __forceinline__ void store_tile_split(const MatTile& m, const float* lds, uint16_t* planes, uint32_t count,
+                                                 float scale) {
+    const int t = threadIdx.x;
+    if (t >= 128) return;
+    const int ln = t & 63, nb = ln & 31, kb = 16 * (t >> 6) + 8 * (ln >> 5);
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = scale * lds[(kb + j) * kTileLd + nb];
+    f16x8 p[2];
+    LaneOps<MG_PRECISION_FP32>::pack(x, p);
+    uint16_t* at = planes + m.base + frag_index_b<32>(m.c0 + nb, m.r0 + kb, m.rows);
+    *reinterpret_cast<f16x8*>(at) = p[0];
+    *reinterpret_cast<f16x8*>(at + count) = p[1];
+}
+
+// SplitScale from params: per block matrix (128 hidden floats each, contiguous
+// from float_group), one per workgroup, the exponent of its largest finite
+// magnitude.
+__global__ void __launch_bounds__(1024) split_scale_kernel(const float* __restrict__ param, uint32_t float_group,
+                                                           uint32_t EH, SplitScale* out) {
+    __shared__ float red[16];
+    const f32x4* p = reinterpret_cast<const f32x4*>(param + float_group + (size_t)blockIdx.x * EH);
+    float m = 0.0f;
+#pragma unroll 8
+    for (uint32_t k = threadIdx.x; k < EH / 4; k += 1024) {
+        const f32x4 v = p[k];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float x = fabsf(v[j]);
+            m = x < __builtin_huge_valf() && x > m ? x : m;
+        }
+    }
+    m = group_max<64>(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        m = group_max<16>(red[threadIdx.x]);
+        if (threadIdx.x == 0) ((blockIdx.x & 1) ? out->down : out->up)[blockIdx.x >> 1] = pow2_above(m);
+    }
+}
+
+// The fragment-tiled copies from params, one tile per workgroup. split: an
+// fp32 policy's planes, which take fwd32b's place (SplitScale after them is
+// current).
 __global__ void __launch_bounds__(256) derive_blocks_kernel(const float* __restrict__ param, float* __restrict__ fwd32,
                                                             float* __restrict__ fwd16, float* __restrict__ bwd16,
                                                             uint16_t* fwd32b, uint16_t* fwd16b, uint16_t* bwd16b,
-                                                            uint32_t float_group, uint32_t H) {
+                                                            uint16_t* split, uint32_t count, uint32_t float_group,
+                                                            uint32_t H) {
     __shared__ float lds[kTT * kTileLd];
     const MatTile m = mat_tile(blockIdx.x, float_group, H);
     const int t = threadIdx.x, c = t & (kTT - 1);
@@ -1228,6 +1277,11 @@ __global__ void __launch_bounds__(256) derive_blocks_kernel(const float* __restr
         lds[r * kTileLd + c] = param[m.base + (size_t)(m.r0 + r) * m.cols + m.c0 + c];
     }
     store_tile_frags(m, lds, fwd32, fwd16, bwd16, fwd32b, fwd16b, bwd16b);
+    if (split) {
+        const SplitScale& ss = *split_scale(split, count);
+        const int mat = (int)((m.base - float_group) / (kEmbed * H)), l = mat >> 1;
+        store_tile_split(m, lds, split, count, pow2i((mat & 1) ? split_exp_down(ss, l) : split_exp_up(ss, l)));
+    }
 }
 
 struct AdamArgs {
@@ -1394,9 +1448,16 @@ int check_matrix_layout(const mg_policy_view& pv) {
 int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv) {
     int rc = check_matrix_layout(pv);
     if (rc) return rc;
+    uint16_t* split = pv.precision == MG_PRECISION_FP32 ? pv.frag_fwd32_bf : nullptr;
+    if (split) {
+        hipLaunchKernelGGL(dev::split_scale_kernel, dim3(2 * pv.layers), dim3(1024), 0, st, pv.params, pv.float_group,
+                           (uint32_t)MG_EMBED * pv.hidden,
+                           const_cast<dev::SplitScale*>(dev::split_scale(split, pv.count)));
+        MG_HIP(hipGetLastError(), "split scale launch");
+    }
     hipLaunchKernelGGL(dev::derive_blocks_kernel, dim3(mat_tiles(pv)), dim3(256), 0, st, pv.params, pv.frag_fwd32,
-                       pv.frag_fwd16, pv.frag_bwd16, pv.frag_fwd32_bf, pv.frag_fwd16_bf, pv.frag_bwd16_bf,
-                       pv.float_group, pv.hidden);
+                       pv.frag_fwd16, pv.frag_bwd16, split ? nullptr : pv.frag_fwd32_bf, pv.frag_fwd16_bf,
+                       pv.frag_bwd16_bf, split, pv.count, pv.float_group, pv.hidden);
     MG_HIP(hipGetLastError(), "derive blocks launch");
     return MG_OK;
 }
