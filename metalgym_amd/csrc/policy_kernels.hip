@@ -3,6 +3,7 @@
 // advantage statistics used by the PPO loss.
 #include "kernels.h"
 #include "mg/device/policy_bf16.h"
+#include "mg/device/policy_lane.h"
 #include "mg/device/sample.h"
 
 namespace mg {
@@ -34,6 +35,36 @@ __global__ void __launch_bounds__(256) forward_kernel(const mg_policy_view pv, c
     for (int idx = threadIdx.x; idx < M * HD; idx += 256) {
         const uint32_t r = row0 + idx / HD;
         if (r < rows) head[(size_t)row0 * HD + idx] = headL[idx];
+    }
+}
+
+// The same with a row in a pair of lanes (policy_lane.h), kLaneTile rows per
+// workgroup. HC, OC: bounds of the head's and the observation's width.
+template <int PREC, int HC, int OC>
+__global__ void __launch_bounds__(kLaneNT, 2) forward_lane_kernel(const mg_policy_view pv,
+                                                                  const float* __restrict__ obs, uint32_t rows,
+                                                                  float* __restrict__ head) {
+    extern __shared__ __align__(16) float lane_lds_f[];
+    const LaneLds L = lane_lds<PREC, HC>(pv.layers, 0, 0);
+    LaneParams<HC> P;
+    LaneRing<PREC> ring;
+    const int O = (int)pv.obs_dim, HD = (int)pv.head_dim;
+    const int lane = threadIdx.x & 63, q = lane >> 5;
+    const uint32_t r = blockIdx.x * kLaneTile + (uint32_t)(kLaneRows * (threadIdx.x >> 6) + (lane & 31));
+    const float* o = obs + (size_t)(r < rows ? r : rows - 1) * O;
+    float ob[(OC + 1) / 2];
+#pragma unroll
+    for (int s = 0; s < (OC + 1) / 2; ++s) {
+        const float v = o[2 * s + q < O ? 2 * s + q : 0];
+        ob[s] = 2 * s + q < O ? v : 0.0f;
+    }
+    lane_start<PREC, HC>(pv, lane_lds_f, L, 0, P, ring);
+    float hv[HC];
+    lane_forward<PREC, HC, OC, false>(pv, P, ring, O, ob, hv);
+    if (r < rows && q == 0) {
+#pragma unroll
+        for (int j = 0; j < HC; ++j)
+            if (j < HD) head[(size_t)r * HD + j] = hv[j];
     }
 }
 
@@ -139,11 +170,38 @@ __global__ void __launch_bounds__(256) adv_stats_kernel(const float* __restrict_
 
 }  // namespace dev
 
+namespace {
+template <int PREC, int HC, int OC>
+bool try_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
+    if (pv.head_dim > (uint32_t)HC || pv.obs_dim > (uint32_t)OC) return false;
+    const size_t lds = (size_t)dev::lane_lds<PREC, HC>(pv.layers, 0, 0).total * 4;
+    if (lds > 163840 / 2) return false;
+    hipLaunchKernelGGL((dev::forward_lane_kernel<PREC, HC, OC>), dim3((rows + dev::kLaneTile - 1) / dev::kLaneTile),
+                       dim3(dev::kLaneNT), lds, st, pv, obs, rows, head);
+    return true;
+}
+// From 8192 rows in fp32 and 16384 in bf16 (64 and 128 workgroups): a
+// workgroup takes the time of its chain of stages however few there are, so
+// forward_kernel's 32-row tiles are as fast where they fit the GPU once. us a
+// call, forward_kernel against this, CartPole: fp32 57.5 / 58.2 at 4096 rows,
+// 60.5 / 59.6 at 8192, 97.6 / 61.9 at 16384, 544 / 189 at 100003; bf16 31.2 /
+// 33.8 at 8192, 38.1 / 34.4 at 16384, 162 / 82 at 100003.
+template <int PREC>
+bool launch_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
+    if (rows < (PREC == MG_PRECISION_BF16 ? 16384u : 8192u) || !pv.frag_fwd32_bf) return false;
+    return try_forward_lane<PREC, 4, 4>(st, pv, obs, rows, head) ||
+           try_forward_lane<PREC, 8, 32>(st, pv, obs, rows, head) ||
+           try_forward_lane<PREC, 16, 64>(st, pv, obs, rows, head);
+}
+}  // namespace
+
 int launch_forward(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
     MG_CHECK(pv.obs_dim <= (uint32_t)dev::kMaxObs && pv.head_dim <= (uint32_t)dev::kMaxHead, MG_ERR_INVALID,
              "forward: OBS_DIM must be <= %d and ACT_DIM + 1 <= %d", dev::kMaxObs, dev::kMaxHead);
     if (rows == 0) return MG_OK;
-    if (pv.precision == MG_PRECISION_BF16)
+    if (pv.precision == MG_PRECISION_BF16 ? launch_forward_lane<MG_PRECISION_BF16>(st, pv, obs, rows, head)
+                                          : launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head)) {
+    } else if (pv.precision == MG_PRECISION_BF16)
         hipLaunchKernelGGL((dev::forward_kernel<32, true>), dim3((rows + 31) / 32), dim3(256), 0, st, pv, obs, rows,
                            head);
     else
