@@ -103,6 +103,12 @@ __device__ __forceinline__ float opaque(float v) {
     return v;
 }
 
+// The same in a vector register.
+__device__ __forceinline__ float opaque_v(float v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
 template <int PREC>
 struct LaneOps;
 template <>

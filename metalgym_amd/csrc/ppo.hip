@@ -8,7 +8,7 @@
 #include <vector>
 
 #include "kernels.h"
-#include "mg/device/policy_lane.h"
+#include "mg/device/policy_pair.h"
 
 struct mg_ppo {
     mg_gym* gym = nullptr;
@@ -17,6 +17,7 @@ struct mg_ppo {
     mg_ppo_hparams hp{};
     uint32_t n = 0, T = 0, B = 0, blocks = 0;
     mg_policy_view pv{};
+    void* arenas = nullptr;  // params, their copies, m and v
     float* m = nullptr;
     float* v = nullptr;
     uint32_t step = 0;
@@ -122,6 +123,15 @@ void shuffle_blocks(uint64_t& s, std::vector<uint32_t>& order) {
 // and their scales.
 size_t fwd32_bf_bytes(const mg_policy_view& pv) {
     return 2 * (pv.precision == MG_PRECISION_BF16 ? (size_t)pv.count : dev::split_elems(pv.count));
+}
+
+// frag_fwd16_bf and frag_bwd16_bf: one bfloat16 plane, or an fp32 policy's pair
+// planes (frag_fwd16_bf's with their scales).
+size_t fwd16_bf_bytes(const mg_policy_view& pv) {
+    return 2 * (pv.precision == MG_PRECISION_BF16 ? (size_t)pv.count : dev::pair_elems(pv.count));
+}
+size_t bwd16_bf_bytes(const mg_policy_view& pv) {
+    return (pv.precision == MG_PRECISION_BF16 ? 2 : 4) * (size_t)pv.count;
 }
 
 int ensure_head(mg_ppo* p, uint32_t rows) {
@@ -324,17 +334,31 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
     const size_t slot = T * n;
     int rc;
     if ((rc = check_matrix_layout(pv))) return fail(rc);
-    if ((rc = device_alloc((void**)&pv.params, (size_t)pv.count * 4, "PPOModel params")) ||
-        (rc = device_alloc((void**)&pv.frag_fwd32, (size_t)pv.count * 4, "PPOModel forward matrix tiles")) ||
-        (rc = device_alloc((void**)&pv.frag_fwd16, (size_t)pv.count * 4, "PPOModel forward matrix tiles")) ||
-        (rc = device_alloc((void**)&pv.frag_bwd16, (size_t)pv.count * 4, "PPOModel backward matrix tiles")) ||
-        (rc = device_alloc((void**)&pv.frag_fwd32_bf, fwd32_bf_bytes(pv), "PPOModel 16-bit matrix tiles")) ||
-        (pv.precision == MG_PRECISION_BF16 &&
-         ((rc = device_alloc((void**)&pv.frag_fwd16_bf, (size_t)pv.count * 2, "PPOModel bf16 matrix tiles")) ||
-          (rc = device_alloc((void**)&pv.frag_bwd16_bf, (size_t)pv.count * 2, "PPOModel bf16 matrix tiles")))) ||
-        (rc = device_alloc((void**)&p->m, (size_t)pv.count * 4, "PPOModel adam m")) ||
-        (rc = device_alloc((void**)&p->v, (size_t)pv.count * 4, "PPOModel adam v")) ||
-        (rc = device_alloc((void**)&p->obs_slots, (T + 1) * n * env->obs_dim * 4, "obs slots")) ||
+    // the policy's arenas in one allocation, cleared by one memset
+    const size_t words = (size_t)pv.count * 4;
+    struct {
+        void** at;
+        size_t bytes;
+    } const arenas[] = {
+        {(void**)&pv.params, words},
+        {(void**)&pv.frag_fwd32, words},
+        {(void**)&pv.frag_fwd16, words},
+        {(void**)&pv.frag_bwd16, words},
+        {(void**)&pv.frag_fwd32_bf, fwd32_bf_bytes(pv)},
+        {(void**)&pv.frag_fwd16_bf, fwd16_bf_bytes(pv)},
+        {(void**)&pv.frag_bwd16_bf, bwd16_bf_bytes(pv)},
+        {(void**)&p->m, words},
+        {(void**)&p->v, words},
+    };
+    size_t arena_bytes = 0;
+    for (const auto& s : arenas) arena_bytes += (s.bytes + 255) / 256 * 256;
+    if ((rc = device_alloc(&p->arenas, arena_bytes, "PPOModel params and matrix tiles"))) return fail(rc);
+    arena_bytes = 0;
+    for (const auto& s : arenas) {
+        *s.at = static_cast<char*>(p->arenas) + arena_bytes;
+        arena_bytes += (s.bytes + 255) / 256 * 256;
+    }
+    if ((rc = device_alloc((void**)&p->obs_slots, (T + 1) * n * env->obs_dim * 4, "obs slots")) ||
         (rc = device_alloc(&p->action_slots, slot * env->action_bytes, "action slots")) ||
         (rc = device_alloc((void**)&p->logp, slot * 4, "logp slots")) ||
         (rc = device_alloc((void**)&p->value, slot * 4, "value slots")) ||
@@ -348,9 +372,8 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
     std::vector<float> P;
     init_params(pv, c->seed, P);
     hipStream_t st = gym->stream;
-    if (hipMemcpyAsync(pv.params, P.data(), (size_t)pv.count * 4, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipMemsetAsync(p->m, 0, (size_t)pv.count * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->v, 0, (size_t)pv.count * 4, st) != hipSuccess ||
+    if (hipMemsetAsync(p->arenas, 0, arena_bytes, st) != hipSuccess ||
+        hipMemcpyAsync(pv.params, P.data(), (size_t)pv.count * 4, hipMemcpyHostToDevice, st) != hipSuccess ||
         hipMemsetAsync(p->obs_slots, 0, (T + 1) * n * env->obs_dim * 4, st) != hipSuccess ||
         hipMemsetAsync(p->action_slots, 0, slot * env->action_bytes, st) != hipSuccess ||
         hipMemsetAsync(p->logp, 0, slot * 4, st) != hipSuccess ||
@@ -359,14 +382,7 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
         hipMemsetAsync(p->done_slots, 0, slot, st) != hipSuccess ||
         hipMemsetAsync(p->adv, 0, slot * 4, st) != hipSuccess ||
         hipMemsetAsync(p->ret, 0, slot * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->head, 0, (size_t)p->head_cap * pv.head_dim * 4, st) != hipSuccess ||
-        hipMemsetAsync(pv.frag_fwd32, 0, (size_t)pv.count * 4, st) != hipSuccess ||
-        hipMemsetAsync(pv.frag_fwd16, 0, (size_t)pv.count * 4, st) != hipSuccess ||
-        hipMemsetAsync(pv.frag_bwd16, 0, (size_t)pv.count * 4, st) != hipSuccess ||
-        (pv.frag_fwd32_bf &&
-         hipMemsetAsync(pv.frag_fwd32_bf, 0, fwd32_bf_bytes(pv), st) != hipSuccess) ||
-        (pv.frag_fwd16_bf && hipMemsetAsync(pv.frag_fwd16_bf, 0, (size_t)pv.count * 2, st) != hipSuccess) ||
-        (pv.frag_bwd16_bf && hipMemsetAsync(pv.frag_bwd16_bf, 0, (size_t)pv.count * 2, st) != hipSuccess))
+        hipMemsetAsync(p->head, 0, (size_t)p->head_cap * pv.head_dim * 4, st) != hipSuccess)
         return fail(set_error(MG_ERR_HIP, "PPOModel: initialisation upload failed"));
     if ((rc = launch_derive_blocks(st, pv))) return fail(rc);
     if (hipStreamSynchronize(st) != hipSuccess)
@@ -381,15 +397,7 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
 int mg_ppo_destroy(mg_ppo* p) {
     if (!p) return MG_OK;
     if (p->gym && p->gym->stream) (void)hipStreamSynchronize(p->gym->stream);
-    (void)hipFree(p->pv.params);
-    (void)hipFree(p->pv.frag_fwd32);
-    (void)hipFree(p->pv.frag_fwd16);
-    (void)hipFree(p->pv.frag_bwd16);
-    (void)hipFree(p->pv.frag_fwd32_bf);
-    (void)hipFree(p->pv.frag_fwd16_bf);
-    (void)hipFree(p->pv.frag_bwd16_bf);
-    (void)hipFree(p->m);
-    (void)hipFree(p->v);
+    (void)hipFree(p->arenas);
     (void)hipFree(p->obs_slots);
     (void)hipFree(p->action_slots);
     (void)hipFree(p->logp);

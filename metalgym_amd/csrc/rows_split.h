@@ -5,6 +5,7 @@
 // reduces over the same TPR lanes as LayerNorm. The captures for the weight
 // gradients have the row-major layouts of train_rows_kernel<false>.
 #pragma once
+#include "mg/device/policy_pair.h"
 #include "mg/device/policy_split.h"
 
 namespace mg {
@@ -26,9 +27,16 @@ struct SkShape {
     static constexpr int OBS = 48;
 };
 
-// LDS of one workgroup.
-template <int W>
-struct alignas(16) SkSmem {
+// LDS of one workgroup. F16: the pair kernel's block input planes and scales.
+template <bool F16>
+struct SkPairLds {
+    PairInput in;
+    int exps[2 * MG_MAX_LAYERS];  // the planes' exponents
+};
+template <>
+struct SkPairLds<false> {};
+template <int W, bool F16 = false>
+struct alignas(16) SkSmem : SkPairLds<F16> {
     using Sh = SkShape<W>;
     float xs[kTR * kLds];        // block input broadcast (X or dh); x_f for dW_head; dh0 for dW_in
     float red[W][kTR * kLds];    // the waves' partials of a block output; W_in / b_in at start-up
@@ -48,17 +56,24 @@ struct alignas(16) SkSmem {
 
 // The block output: this wave's partial to LDS, a barrier, then the thread's
 // row and columns summed over the waves in order.
-template <int W>
-__device__ __forceinline__ RowVec<SkShape<W>::NV> sk_reduce(SkSmem<W>& L, const f32x4 (&hp)[8], int wave, int row,
+template <int W, bool F16>
+__device__ __forceinline__ RowVec<SkShape<W>::NV> sk_reduce(SkSmem<W, F16>& L, const f32x4 (&hp)[8], int wave, int row,
                                                             int c0) {
     return sk_reduce_buf<W, SkShape<W>::NV>(&L.red[0][0], hp, wave, row, c0);
+}
+
+// A block output in a scaled row's units back to its own.
+template <int NV>
+__device__ __forceinline__ void pair_unscale(RowVec<NV>& v, int e) {
+#pragma unroll
+    for (int c = 0; c < 4 * NV; ++c) v[c] = __builtin_ldexpf(v[c], e);
 }
 
 // model/layernorm.metal:74-127 on a row: g is the gradient at the LN output,
 // the result the gradient at its input. The row's terms of the dgamma and
 // dbeta sums (xn g and g) go to part.
-template <int W>
-__device__ __forceinline__ RowVec<SkShape<W>::NV> sk_layernorm_bwd(SkSmem<W>& L, const RowVec<SkShape<W>::NV>& g,
+template <int W, bool F16>
+__device__ __forceinline__ RowVec<SkShape<W>::NV> sk_layernorm_bwd(SkSmem<W, F16>& L, const RowVec<SkShape<W>::NV>& g,
                                                                    int lnIdx, int row, int c0) {
     constexpr int NV = SkShape<W>::NV, CPT = SkShape<W>::CPT, TPR = SkShape<W>::TPR;
     const RowVec<NV> xv = rv_load<NV>(L.xn + (lnIdx * kTR + row) * kEmbed + c0);
@@ -111,8 +126,8 @@ __device__ __forceinline__ void sk_layernorm_r(const RowVec<NV>& h, const float*
 
 // The tile's dgamma and dbeta (rows summed in order) from part; after a
 // barrier that follows the LN backward. Threads 0 .. 255.
-template <int W>
-__device__ __forceinline__ void sk_ln_sums(const SkSmem<W>& L, float* tp_gamma, float* tp_beta) {
+template <int W, bool F16>
+__device__ __forceinline__ void sk_ln_sums(const SkSmem<W, F16>& L, float* tp_gamma, float* tp_beta) {
     const int t = threadIdx.x;
     if (t < 2 * kEmbed) {
         const int c = t & (kEmbed - 1), which = t >> 7;
@@ -237,13 +252,14 @@ __device__ __forceinline__ void sk_loss_row(const RowsArgs& a, const float (&hv)
 }
 
 // HC: a compile-time bound on the head width (4, 8 or 16), for the head and
-// loss in registers.
-template <int W, int HC>
+// loss in registers. F16: the block GEMMs on binary16 pairs (policy_pair.h).
+template <int W, int HC, bool F16>
 __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs a) {
     using Sh = SkShape<W>;
     constexpr int M = kTR, NT = Sh::NT, S = Sh::S, TPR = Sh::TPR, CPT = Sh::CPT, NV = Sh::NV;
     static_assert(NT >= 2 * kEmbed, "sk_ln_sums takes one thread per output");
-    __shared__ SkSmem<W> L;
+    static_assert(!F16 || W == kPairW, "the pair stream's waves");
+    __shared__ SkSmem<W, F16> L;
     const mg_policy_view& pv = a.pv;
     const TrainWs& ws = a.ws;
     const int O = (int)pv.obs_dim, HD = (int)pv.head_dim, H = (int)pv.hidden, NL = (int)pv.layers;
@@ -262,11 +278,21 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
     // drop it), then the weight stream's first loads; the staging stores
     // then wait for the small loads alone (vector memory loads complete in
     // order), so the embed and LN0 overlap the arrival of the first weights
-    const int rot = (wave + (int)(blockIdx.x >> 3)) % NC;
-    const SkSeq<S> seq{pv.frag_fwd16 + pv.float_group, pv.frag_bwd16 + pv.float_group, NL, NC, wave, rot,
-                       (uint32_t)kEmbed * (uint32_t)H};
-    SkPos pos{0, 0, 0};
-    SkStream<S> wst;
+    // F16: this wave's groups of 32 units; else its strips of every chunk
+    const int NK = F16 ? ((int)(H / kPairGroup) - wave + W - 1) / W : NC;
+    const int rot = NK > 0 ? (wave + (int)(blockIdx.x >> 3)) % NK : 0;
+    using Seq = std::conditional_t<F16, PairSeq, SkSeq<S>>;
+    using Pos = std::conditional_t<F16, PairPos, SkPos>;
+    Seq seq;
+    if constexpr (F16)
+        seq = Seq{pv.frag_fwd16_bf + 2 * (size_t)pv.float_group, pv.frag_bwd16_bf + 2 * (size_t)pv.float_group, NL, NK,
+                  wave, rot, (uint32_t)kEmbed * (uint32_t)H};
+    else
+        seq = Seq{pv.frag_fwd16 + pv.float_group, pv.frag_bwd16 + pv.float_group, NL, NC, wave, rot,
+                  (uint32_t)kEmbed * (uint32_t)H};
+    Pos pos{0, 0, 0};
+    std::conditional_t<F16, PairStream, SkStream<S>> wst;
+    PairScale* const pairs = F16 ? pair_scale(pv.frag_fwd16_bf, pv.count) : nullptr;
     float* const winL = &L.red[0][0];  // the partial buffer is unused until the first block's reduction
     float* const binL = winL + Sh::OBS * kEmbed;
     const float* lnp = pv.params + pv.off_ln_gamma[0];
@@ -312,7 +338,14 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
             ret = a.ret_slots[gr];
             if (!pv.continuous) act = static_cast<const int*>(a.action_slots)[gr];
         }
-        wst.start(seq, pos);
+        int ex = 0;
+        if constexpr (F16) {
+            ex = pairs->cur[tid & (2 * MG_MAX_LAYERS - 1)];
+            if (NK > 0) wst.start(seq.role(pos, 0), seq.role(pos, 1));
+            if (tid < 2 * MG_MAX_LAYERS) L.exps[tid] = ex;
+        } else {
+            wst.start(seq, pos);
+        }
         if (tid < n_obs) L.obs[tid] = o0;
 #pragma unroll
         for (int u = 0; u < NWH; ++u) {
@@ -360,31 +393,66 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
         rv_store(L.xn + (l * M + row) * kEmbed + c0, xn);
         if (lk == 0) L.rstd[l * M + row] = sd;
         rv_store(cx + ((size_t)l * B + r0 + row) * kEmbed + c0, x);
-        rv_store(L.xs + row * kLds + c0, x);
+        int unit = 0;  // exponent of the row's block output
+        if constexpr (F16)
+            unit = pair_store_input<TPR>(L.in, x, row, lk, L.exps[2 * l]) + L.exps[2 * l] + kHiddenExp +
+                   L.exps[2 * l + 1];
+        else
+            rv_store(L.xs + row * kLds + c0, x);
         __syncthreads();  // X complete; every wave is past its reads of red (and of W_in)
-        f32x4 xb[8];
-        sk_load_input(L.xs, xb);
         f32x4 hp[8];
 #pragma unroll
         for (int ct = 0; ct < 8; ++ct) hp[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        float* vrow = cv + ((size_t)l * B + r0 + n16) * H + 16 * S * wave + q4;
-        for (int k = 0; k < NC; ++k) {  // model/mlp.metal:18-86 for this wave's units of a chunk
-            const SkPos nx = seq.next(pos);
-            f32x4 v[S];
+        if constexpr (F16) {
+            f16x8 xb[4][2];
+            pair_load_input(L.in, xb);
+            const int vexp = -L.in.unit[n16];
+            float* vrow = cv + ((size_t)l * B + r0 + n16) * H + 2 * q4;
+            for (int k = 0; k < NK; ++k) {  // model/mlp.metal:18-86 for one of this wave's groups
+                const PairPos nx = seq.next(pos);
+                f32x4 v[2] = {};
+                wst.gemm0(v, xb, seq.role(nx, 0));
+                float t[8];
+                f32x4 cap[2];
 #pragma unroll
-            for (int s = 0; s < S; ++s) v[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            wst.gemm0(v, xb, seq.role0(nx));
-            const int c = seq.chunk(pos);
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[s][r] = v[s][r] > 0.0f ? v[s][r] : 0.0f;
-                *reinterpret_cast<f32x4*>(vrow + kChunk * c + 16 * s) = v[s];
+                    for (int r = 0; r < 4; ++r) {
+                        t[4 * s + r] = v[s][r];
+                        cap[s][r] = __builtin_ldexpf(v[s][r] > 0.0f ? v[s][r] : 0.0f, vexp);
+                    }
+                float* vp = vrow + kPairGroup * seq.group(pos);
+                *reinterpret_cast<f32x4*>(vp) = cap[0];
+                *reinterpret_cast<f32x4*>(vp + 4) = cap[1];
+                f16x8 vb[2];
+                LaneOps<MG_PRECISION_FP32>::pack_hidden(t, vb);
+                wst.gemm1(hp, vb, seq.role(nx, 1));
+                pos = nx;
             }
-            wst.gemm1(hp, v, seq.role1(nx), seq.stride1());
-            pos = nx;
+        } else {
+            f32x4 xb[8];
+            sk_load_input(L.xs, xb);
+            float* vrow = cv + ((size_t)l * B + r0 + n16) * H + 16 * S * wave + q4;
+            for (int k = 0; k < NC; ++k) {  // model/mlp.metal:18-86 for this wave's units of a chunk
+                const SkPos nx = seq.next(pos);
+                f32x4 v[S];
+#pragma unroll
+                for (int s = 0; s < S; ++s) v[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                wst.gemm0(v, xb, seq.role0(nx));
+                const int c = seq.chunk(pos);
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[s][r] = v[s][r] > 0.0f ? v[s][r] : 0.0f;
+                    *reinterpret_cast<f32x4*>(vrow + kChunk * c + 16 * s) = v[s];
+                }
+                wst.gemm1(hp, v, seq.role1(nx), seq.stride1());
+                pos = nx;
+            }
         }
-        h = rv_add(h, sk_reduce<W>(L, hp, wave, row, c0));  // model/elementwise.metal:4-13
+        RowVec<NV> dx = sk_reduce<W, F16>(L, hp, wave, row, c0);
+        if constexpr (F16) pair_unscale(dx, -unit);
+        h = rv_add(h, dx);  // model/elementwise.metal:4-13
     }
     // ---- final LN, head, loss and the head's backward, each row in its lanes'
     // registers (model/ppo.h:616-625, then model/ppo.h:793-806) ----
@@ -427,7 +495,7 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
                 for (int i = 0; i < 4; ++i) g[c] += dz[4 * q + i] * w[i];
             }
         }
-        D = sk_layernorm_bwd<W>(L, g, NL, row, c0);
+        D = sk_layernorm_bwd<W, F16>(L, g, NL, row, c0);
     }
     __syncthreads();  // dhead, dls, the LossStats terms and the LN's part terms written
 
@@ -453,39 +521,77 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
     int lnDone = NL;  // the LN whose dgamma / dbeta terms are in part
     for (int l = NL - 1; l >= 0; --l) {  // model/mlp.metal:88-153 + model/ppo.h:851-852
         rv_store(cdh + ((size_t)l * B + r0 + row) * kEmbed + c0, D);
-        rv_store(L.xs + row * kLds + c0, D);
+        int unit = 0;
+        if constexpr (F16)
+            unit = pair_store_input<TPR>(L.in, D, row, lk, L.exps[2 * l + 1]) + L.exps[2 * l + 1] + kHiddenExp +
+                   L.exps[2 * l];
+        else
+            rv_store(L.xs + row * kLds + c0, D);
         __syncthreads();  // dh complete; red read; part holds LN lnDone's terms
-        sk_ln_sums<W>(L, tp + pv.off_ln_gamma[lnDone], tp + pv.off_ln_beta[lnDone]);
-        f32x4 xb[8];
-        sk_load_input(L.xs, xb);
+        sk_ln_sums<W, F16>(L, tp + pv.off_ln_gamma[lnDone], tp + pv.off_ln_beta[lnDone]);
         f32x4 hp[8];
 #pragma unroll
         for (int ct = 0; ct < 8; ++ct) hp[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        const float* vrow = cv + ((size_t)l * B + r0 + n16) * H + 16 * S * wave + q4;
-        float* dvrow = cdv + ((size_t)l * B + r0 + n16) * H + 16 * S * wave + q4;
-        for (int k = 0; k < NC; ++k) {
-            const SkPos nx = seq.next(pos);
-            const int c = seq.chunk(pos);
-            // this lane's hidden values of the forward: the relu mask (loaded
-            // before the GEMM issues its weight refills)
-            f32x4 m[S], dv[S];
+        if constexpr (F16) {
+            f16x8 xb[4][2];
+            pair_load_input(L.in, xb);
+            const int vexp = -L.in.unit[n16];
+            const float* vrow = cv + ((size_t)l * B + r0 + n16) * H + 2 * q4;
+            float* dvrow = cdv + ((size_t)l * B + r0 + n16) * H + 2 * q4;
+            for (int k = 0; k < NK; ++k) {
+                const PairPos nx = seq.next(pos);
+                const int u0 = kPairGroup * seq.group(pos);
+                // this lane's hidden values of the forward: the relu mask
+                const f32x4 m[2] = {*reinterpret_cast<const f32x4*>(vrow + u0),
+                                    *reinterpret_cast<const f32x4*>(vrow + u0 + 4)};
+                f32x4 dv[2] = {};
+                wst.gemm0(dv, xb, seq.role(nx, 0));  // dV^T = Down strips . dh^T
+                float t[8];
+                f32x4 cap[2];
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                m[s] = *reinterpret_cast<const f32x4*>(vrow + kChunk * c + 16 * s);
-                dv[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        t[4 * s + r] = m[s][r] > 0.0f ? dv[s][r] : 0.0f;
+                        cap[s][r] = __builtin_ldexpf(t[4 * s + r], vexp);
+                    }
+                *reinterpret_cast<f32x4*>(dvrow + u0) = cap[0];
+                *reinterpret_cast<f32x4*>(dvrow + u0 + 4) = cap[1];
+                f16x8 vb[2];
+                pair_pack(t, vb);
+                wst.gemm1(hp, vb, seq.role(nx, 1));  // dx += dV Up^T
+                pos = nx;
             }
-            wst.gemm0(dv, xb, seq.role0(nx));  // dV^T = Down strip . dh^T
+        } else {
+            f32x4 xb[8];
+            sk_load_input(L.xs, xb);
+            const float* vrow = cv + ((size_t)l * B + r0 + n16) * H + 16 * S * wave + q4;
+            float* dvrow = cdv + ((size_t)l * B + r0 + n16) * H + 16 * S * wave + q4;
+            for (int k = 0; k < NC; ++k) {
+                const SkPos nx = seq.next(pos);
+                const int c = seq.chunk(pos);
+                // this lane's hidden values of the forward: the relu mask (loaded
+                // before the GEMM issues its weight refills)
+                f32x4 m[S], dv[S];
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
+                for (int s = 0; s < S; ++s) {
+                    m[s] = *reinterpret_cast<const f32x4*>(vrow + kChunk * c + 16 * s);
+                    dv[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+                wst.gemm0(dv, xb, seq.role0(nx));  // dV^T = Down strip . dh^T
 #pragma unroll
-                for (int r = 0; r < 4; ++r) dv[s][r] = m[s][r] > 0.0f ? dv[s][r] : 0.0f;
-                *reinterpret_cast<f32x4*>(dvrow + kChunk * c + 16 * s) = dv[s];
+                for (int s = 0; s < S; ++s) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) dv[s][r] = m[s][r] > 0.0f ? dv[s][r] : 0.0f;
+                    *reinterpret_cast<f32x4*>(dvrow + kChunk * c + 16 * s) = dv[s];
+                }
+                wst.gemm1(hp, dv, seq.role1(nx), seq.stride1());  // dx += dV Up^T
+                pos = nx;
             }
-            wst.gemm1(hp, dv, seq.role1(nx), seq.stride1());  // dx += dV Up^T
-            pos = nx;
         }
-        const RowVec<NV> dx = sk_reduce<W>(L, hp, wave, row, c0);
-        D = rv_add(D, sk_layernorm_bwd<W>(L, dx, l, row, c0));  // residualAdd(dBranch, dStream)
+        RowVec<NV> dx = sk_reduce<W, F16>(L, hp, wave, row, c0);
+        if constexpr (F16) pair_unscale(dx, -unit);
+        D = rv_add(D, sk_layernorm_bwd<W, F16>(L, dx, l, row, c0));  // residualAdd(dBranch, dStream)
         lnDone = l;
     }
     // model/input.metal:38-60 on this tile: dW_in[k][c] = sum_r obs[r][k] dh0[r][c], db_in = sum_r dh0
@@ -493,9 +599,20 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
     __syncthreads();
     // LN0's sums on threads 0 .. 255 and db_in's on the waves past them (on 8
     // waves: 256 .. 383), so no wave adds two of the tail's column sums
-    sk_ln_sums<W>(L, tp + pv.off_ln_gamma[0], tp + pv.off_ln_beta[0]);
+    sk_ln_sums<W, F16>(L, tp + pv.off_ln_gamma[0], tp + pv.off_ln_beta[0]);
     tile_colsum2<M>(L.xs, nullptr, tp + pv.off_in_b, nullptr, NT >= 3 * kEmbed ? 2 * kEmbed : 0);
     tile_outer<M, NT>(L.obs, O, O, L.xs, tp + pv.off_in_w, kEmbed, 1);
+    if constexpr (F16) {  // the exponents for the coming Adam step's planes (PairScale), one wave per matrix
+        if (wave == W - 1) {
+            const int tiles = H / 8;  // 32 x 32 tiles of a matrix: at most kPairTiles
+            for (int m = (int)blockIdx.x; m < 2 * NL; m += (int)gridDim.x) {
+                const float t0 = lane < tiles ? pairs->tilemax[m][lane] : 0.0f;
+                const float t1 = lane + 64 < tiles ? pairs->tilemax[m][lane + 64] : 0.0f;
+                const float most = group_max<64>(fmaxf(t0, t1)) + kAdamReach * a.lr;
+                if (lane == 0) pairs->next[m] = pair_exp(most);
+            }
+        }
+    }
 }
 
 // The split row pass's wave count for a policy: 8 (two waves per SIMD, the

@@ -30,6 +30,7 @@
 #include "kernels.h"
 #include "mg/device/policy_bf16.h"
 #include "mg/device/policy_lane.h"
+#include "mg/device/policy_pair.h"
 #include "mg/device/sample.h"
 
 namespace mg {
@@ -139,6 +140,7 @@ struct RowsArgs {
     const float* logp_slots;
     const float* adv_stats;
     float* head_out;
+    float lr;
 };
 
 // LDS arrays of the loss phase: head [16][HD] in; dhead [16][HD], the
@@ -1234,11 +1236,43 @@ __device__ __forceinline__ void store_tile_split(const MatTile& m, const float* 
     *reinterpret_cast<f16x8*>(at + count) = p[1];
 }
 
+// Writes the tile held in lds to the pair kernel's planes (policy_pair.h), each
+// element times 2^e: an up tile in role 0 to fwd and in role 1 to bwd, a down
+// tile the other way round. Threads 0 .. 127 write role 0 (one k-group of both
+// strips), the others role 1 (two column strips). After a barrier that follows
+// the tile's LDS stores.
+__device__ __forceinline__ void store_tile_pair(const MatTile& m, const float* lds, uint16_t* fwd, uint16_t* bwd,
+                                                bool down, int e) {
+    const int t = threadIdx.x & 127, half = threadIdx.x >> 7, s = t >> 6, r = t & 15, q = (t >> 4) & 3;
+    // the tile's (row, column) of the eight elements and the index they start at
+    int r0, c0, dr, dc;
+    uint32_t at;
+    if (half == 0) {
+        const int u = 8 * (r >> 2) + 4 * s + (r & 3);
+        r0 = down ? u : 8 * q, c0 = down ? 8 * q : u, dr = down ? 0 : 1, dc = down ? 1 : 0;
+        at = down ? pair_index0(m.r0 + u, m.c0 + 8 * q) : pair_index0(m.c0 + u, m.r0 + 8 * q);
+    } else {
+        const int c = 16 * s + r;
+        r0 = down ? 8 * q : c, c0 = down ? c : 8 * q, dr = down ? 1 : 0, dc = down ? 0 : 1;
+        at = down ? pair_index1(m.r0 + 8 * q, m.c0 + c) : pair_index1(m.c0 + 8 * q, m.r0 + c);
+    }
+    const float f = pow2i(e < -126 ? -126 : e);
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = f * lds[(r0 + j * dr) * kTileLd + c0 + j * dc];
+    f16x8 p[2];
+    LaneOps<MG_PRECISION_FP32>::pack(x, p);
+    uint16_t* out = (half == (down ? 1 : 0) ? fwd : bwd) + 2 * (size_t)m.base + at;
+    *reinterpret_cast<f16x8*>(out) = p[0];
+    *reinterpret_cast<f16x8*>(out + 512) = p[1];
+}
+
 // SplitScale from params: per block matrix (128 hidden floats each, contiguous
 // from float_group), one per workgroup, the exponent of its largest finite
-// magnitude.
+// magnitude. pairs: also the pair planes' exponents and their tiles' magnitudes
+// (the matrix's for each), one entry per workgroup.
 __global__ void __launch_bounds__(1024) split_scale_kernel(const float* __restrict__ param, uint32_t float_group,
-                                                           uint32_t EH, SplitScale* out) {
+                                                           uint32_t EH, SplitScale* out, PairScale* pairs) {
     __shared__ float red[16];
     const f32x4* p = reinterpret_cast<const f32x4*>(param + float_group + (size_t)blockIdx.x * EH);
     float m = 0.0f;
@@ -1254,20 +1288,24 @@ __global__ void __launch_bounds__(1024) split_scale_kernel(const float* __restri
     m = group_max<64>(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x < 16) {
-        m = group_max<16>(red[threadIdx.x]);
-        if (threadIdx.x == 0) ((blockIdx.x & 1) ? out->down : out->up)[blockIdx.x >> 1] = pow2_above(m);
+    if (threadIdx.x < kPairTiles) {
+        m = group_max<16>(red[threadIdx.x & 15]);
+        if (threadIdx.x == 0) {
+            ((blockIdx.x & 1) ? out->down : out->up)[blockIdx.x >> 1] = pow2_above(m);
+            if (pairs) pairs->cur[blockIdx.x] = pairs->next[blockIdx.x] = pair_exp(m);
+        }
+        if (pairs) pairs->tilemax[blockIdx.x][threadIdx.x] = m;
     }
 }
 
 // The fragment-tiled copies from params, one tile per workgroup. split: an
-// fp32 policy's planes, which take fwd32b's place (SplitScale after them is
-// current).
+// fp32 policy's planes, which take fwd32b's place, pfwd and pbwd: its pair
+// planes, in fwd16b's and bwd16b's (the scales after them are current).
 __global__ void __launch_bounds__(256) derive_blocks_kernel(const float* __restrict__ param, float* __restrict__ fwd32,
                                                             float* __restrict__ fwd16, float* __restrict__ bwd16,
                                                             uint16_t* fwd32b, uint16_t* fwd16b, uint16_t* bwd16b,
-                                                            uint16_t* split, uint32_t count, uint32_t float_group,
-                                                            uint32_t H) {
+                                                            uint16_t* split, uint16_t* pfwd, uint16_t* pbwd,
+                                                            uint32_t count, uint32_t float_group, uint32_t H) {
     __shared__ float lds[kTT * kTileLd];
     const MatTile m = mat_tile(blockIdx.x, float_group, H);
     const int t = threadIdx.x, c = t & (kTT - 1);
@@ -1281,6 +1319,7 @@ __global__ void __launch_bounds__(256) derive_blocks_kernel(const float* __restr
         const SplitScale& ss = *split_scale(split, count);
         const int mat = (int)((m.base - float_group) / (kEmbed * H)), l = mat >> 1;
         store_tile_split(m, lds, split, count, pow2i((mat & 1) ? split_exp_down(ss, l) : split_exp_up(ss, l)));
+        if (pfwd) store_tile_pair(m, lds, pfwd, pbwd, mat & 1, pair_scale(pfwd, count)->cur[mat]);
     }
 }
 
@@ -1292,6 +1331,8 @@ struct AdamArgs {
     uint16_t* frag_fwd32_bf;
     uint16_t* frag_fwd16_bf;
     uint16_t* frag_bwd16_bf;
+    uint16_t* pair_fwd;  // the pair planes in the place of frag_fwd16 / frag_bwd16, or NULL
+    uint16_t* pair_bwd;
     const float* grad;
     float* mom;
     float* var;
@@ -1343,6 +1384,7 @@ __device__ __forceinline__ float adam_clip_scale(const AdamArgs& a) {
 // group and the head elementwise. Workgroup 0 also records the pre-clip norm.
 __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
     __shared__ float lds[kTT * kTileLd];
+    __shared__ float wmax[4];
     constexpr int PER = kTT * kTT / 256;  // tile elements per thread
     const int t = threadIdx.x;
     if (blockIdx.x < a.mat_tiles) {
@@ -1356,11 +1398,28 @@ __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
             idx[e] = m.base + (m.r0 + r) * m.cols + m.c0 + c;
             in[e] = adam_load(a, idx[e]);
         }
+        const uint32_t per = a.hidden * kEmbed / (kTT * kTT), mat = blockIdx.x / per;
+        PairScale* const pairs = a.pair_fwd ? pair_scale(a.pair_fwd, a.count) : nullptr;
+        const int exp = pairs ? pairs->next[mat] : 0;
         const float scale = adam_clip_scale(a);
+        float most = 0.0f;
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
             const int r = (256 / kTT) * e + t / kTT;
-            lds[r * kTileLd + c] = adam_elem(a, idx[e], in[e], scale);
+            const float p = adam_elem(a, idx[e], in[e], scale);
+            lds[r * kTileLd + c] = p;
+            most = fmaxf(most, fabsf(p));
+        }
+        if (pairs) {  // this tile's planes, and what the next step's exponent needs (PairScale)
+            most = group_max<64>(most);
+            if ((t & 63) == 0) wmax[t >> 6] = most;
+            __syncthreads();
+            if (t == 0) {
+                pairs->tilemax[mat][blockIdx.x % per] = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+                if (blockIdx.x % per == 0) pairs->cur[mat] = exp;
+            }
+            store_tile_pair(m, lds, a.pair_fwd, a.pair_bwd, mat & 1, exp);
+            return;
         }
         store_tile_frags(m, lds, a.frag_fwd32, a.frag_fwd16, a.frag_bwd16, a.frag_fwd32_bf, a.frag_fwd16_bf,
                          a.frag_bwd16_bf);
@@ -1445,19 +1504,32 @@ int check_matrix_layout(const mg_policy_view& pv) {
     return MG_OK;
 }
 
+namespace {
+// Whether the fp32 row pass runs on binary16 pairs: wherever the 8-wave split
+// layout holds the policy and the planes are there.
+bool rows_on_pairs(const mg_policy_view& pv) {
+    return pv.precision == MG_PRECISION_FP32 && pv.frag_fwd16_bf && pv.frag_bwd16_bf &&
+           dev::rows_split_waves(pv) == dev::kPairW;
+}
+}  // namespace
+
 int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv) {
     int rc = check_matrix_layout(pv);
     if (rc) return rc;
-    uint16_t* split = pv.precision == MG_PRECISION_FP32 ? pv.frag_fwd32_bf : nullptr;
+    const bool bf = pv.precision == MG_PRECISION_BF16, pairs = rows_on_pairs(pv);
+    uint16_t* split = bf ? nullptr : pv.frag_fwd32_bf;
     if (split) {
         hipLaunchKernelGGL(dev::split_scale_kernel, dim3(2 * pv.layers), dim3(1024), 0, st, pv.params, pv.float_group,
                            (uint32_t)MG_EMBED * pv.hidden,
-                           const_cast<dev::SplitScale*>(dev::split_scale(split, pv.count)));
+                           const_cast<dev::SplitScale*>(dev::split_scale(split, pv.count)),
+                           pairs ? dev::pair_scale(pv.frag_fwd16_bf, pv.count) : nullptr);
         MG_HIP(hipGetLastError(), "split scale launch");
     }
     hipLaunchKernelGGL(dev::derive_blocks_kernel, dim3(mat_tiles(pv)), dim3(256), 0, st, pv.params, pv.frag_fwd32,
-                       pv.frag_fwd16, pv.frag_bwd16, split ? nullptr : pv.frag_fwd32_bf, pv.frag_fwd16_bf,
-                       pv.frag_bwd16_bf, split, pv.count, pv.float_group, pv.hidden);
+                       pv.frag_fwd16, pv.frag_bwd16, bf ? pv.frag_fwd32_bf : nullptr,
+                       bf ? pv.frag_fwd16_bf : nullptr, bf ? pv.frag_bwd16_bf : nullptr, split,
+                       pairs ? pv.frag_fwd16_bf : nullptr, pairs ? pv.frag_bwd16_bf : nullptr, pv.count,
+                       pv.float_group, pv.hidden);
     MG_HIP(hipGetLastError(), "derive blocks launch");
     return MG_OK;
 }
@@ -1496,14 +1568,14 @@ dev::DwArgsT<T> dw_args(const mg_policy_view& pv, const TrainWs& ws, uint32_t B,
 }
 
 // The split row pass with the head width's compile-time bound.
-template <int W>
+template <int W, bool F16 = false>
 void launch_rows_split(hipStream_t st, uint32_t B, const mg_policy_view& pv, const dev::RowsArgs& ra) {
     if (pv.head_dim <= 4)
-        hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 4>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
+        hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 4, F16>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
     else if (pv.head_dim <= 8)
-        hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 8>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
+        hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 8, F16>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
     else
-        hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 16>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
+        hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 16, F16>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
 }
 
 int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hparams& hp, float lr,
@@ -1543,8 +1615,11 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         ra.logp_slots = logp_slots;
         ra.adv_stats = adv_stats;
         ra.head_out = head_out;
+        ra.lr = lr;
         if (bf)
             hipLaunchKernelGGL(dev::train_rows_kernel<true>, dim3(B / dev::kTR), dim3(dev::kTNT), 0, st, ra);
+        else if (rows_on_pairs(pv))
+            launch_rows_split<dev::kPairW, true>(st, B, pv, ra);
         else if (dev::rows_split_waves(pv) == 8)
             launch_rows_split<8>(st, B, pv, ra);
         else if (dev::rows_split_waves(pv) == 4)
@@ -1622,8 +1697,11 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         // only the copies the next minibatch's row pass reads; the others are
         // derived once before the next collect or forward
         aa.frag_fwd32 = nullptr;
-        aa.frag_fwd16 = bf ? nullptr : pv.frag_fwd16;
-        aa.frag_bwd16 = bf ? nullptr : pv.frag_bwd16;
+        const bool pairs = rows_on_pairs(pv);
+        aa.frag_fwd16 = bf || pairs ? nullptr : pv.frag_fwd16;
+        aa.frag_bwd16 = bf || pairs ? nullptr : pv.frag_bwd16;
+        aa.pair_fwd = pairs ? pv.frag_fwd16_bf : nullptr;
+        aa.pair_bwd = pairs ? pv.frag_bwd16_bf : nullptr;
         aa.frag_fwd32_bf = nullptr;
         aa.frag_fwd16_bf = bf ? pv.frag_fwd16_bf : nullptr;
         aa.frag_bwd16_bf = bf ? pv.frag_bwd16_bf : nullptr;
