@@ -730,124 +730,15 @@ __device__ __forceinline__ void write_norm_part(float sq, float* out) {
     }
 }
 
-constexpr int kDwRows = 64;             // rows staged in LDS per step
-constexpr int kDwTileM = 128;           // output tile: 128 x 64
-constexpr int kDwTileN = 64;
-constexpr int kDwLdX = kDwTileM + 4;    // LDS row strides of the staged slabs
-constexpr int kDwLdY = kDwTileN + 4;
-constexpr int kDwWaves = 8;             // two per SIMD
-
-// One 128 x 64 tile of a block matrix's gradient C = X^T Y over one row split:
-// 8 waves, wave w owning the 32 x 32 sub-tile at (32 (w / 2), 32 (w % 2)) as
-// one accumulator (v_mfma_f32_32x32x2_f32: A = X[k][m], B = Y[k][n] straight
-// from the staged slab, k = the rows). 64-row slabs of X (32 KB) and Y (16 KB)
-// are double-buffered in LDS, and each slab's loads are issued two slabs
-// before it is written there (two register sets), so one workgroup per CU
-// keeps two slabs of loads in flight; one barrier per slab. The next slab's
-// LDS writes and the loads after them are issued between the current slab's
-// MFMAs (written after them, the last wave of a SIMD ran them alone before the
-// barrier: 23.6 -> 22.1 us at 4096 rows, hidden 512). Workgroup id =
-// tile * splits + split: workgroups go to the 8 XCDs round robin, so with 8
-// or 16 splits all tiles of one row split run on the same XCD and share its
-// rows through that XCD's L2.
-__global__ void __launch_bounds__(64 * kDwWaves) train_dw_kernel(const DwArgsT<float> a) {
-    __shared__ float xs[2][kDwRows * kDwLdX];
-    __shared__ float ys[2][kDwRows * kDwLdY];
-    const uint32_t split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
-    const uint32_t rowsPer = a.rows / a.splits;
-    const uint32_t rb = split * rowsPer;
-    float* out = a.partial + (size_t)split * a.count;
-    const int tid = threadIdx.x;
-    uint32_t t = tile, m = 0;  // the grid is big_tiles * splits: every workgroup has a tile
-    while (t >= a.tiles_per_big[m]) t -= a.tiles_per_big[m], ++m;
-    const BigMatT<float>& bm = a.big[m];
-    const uint32_t ntn = bm.ndim / kDwTileN;
-    const uint32_t tm = t / ntn, tn = t % ntn;
-    const int w = tid >> 6, lane = tid & 63;
-    const int wm = 32 * (w >> 1), wn = 32 * (w & 1);
-    // staging: X rows t / 32 + 16 i (i < 4) at column 4 (t % 32); Y rows
-    // t / 16 + 32 i (i < 2) at column 4 (t % 16)
-    const int xr = tid >> 5, xc = 4 * (tid & 31), yr = tid >> 4, yc = 4 * (tid & 15);
-    // slab indices past the split's last slab reload the last one, so every
-    // step issues the same loads
-    f32x4 px[2][4], py[2][2];
-    const uint32_t steps = rowsPer / kDwRows;
-    // staging item it < 4: X rows xr + 16 it; it >= 4: Y rows yr + 32 (it - 4),
-    // of the slab's 64 rows; buffer loads from the matrices' bases with this
-    // thread's byte offset in a VGPR and the row offset in an SGPR.
-    // With 8 splits, split s takes the rows of the row pass's 16-row tiles
-    // s, s + 8, s + 16, ...: the row-pass workgroups that wrote them ran on the
-    // same XCD as this split (workgroups go to the XCDs round robin), so part of
-    // the slabs still sit in that XCD's L2 (22.2 -> 21.9 us at 4096 rows);
-    // otherwise a split's rows are contiguous. Slab row q is then row
-    // 16 s + q % 16 + 128 (q / 16) of the minibatch.
-    const bool xcd = a.splits == 8;
-    const uint32_t xrow = xcd ? 16 * split + xr : rb + xr;
-    const uint32_t yrow = xcd ? 16 * split + (yr & 15) + 128 * (yr >> 4) : rb + yr;
-    const uint32_t rstep = xcd ? 8 : 1;  // minibatch rows per slab row, in 16-row groups
-    const uint32_t xv = 4 * (xrow * bm.ldx + tm * kDwTileM + xc);
-    const uint32_t yv = 4 * (yrow * bm.ldy + tn * kDwTileN + yc);
-    auto load_item = [&](int set, int it, uint32_t sl) {
-        const uint32_t r0 = (sl < steps ? sl : steps - 1) * kDwRows;
-        if (it < 4)
-            px[set][it] = buffer_load16(bm.x, xv, 4 * rstep * (r0 + 16 * it) * bm.ldx);
-        else
-            py[set][it - 4] = buffer_load16(bm.y, yv, 4 * rstep * (r0 + 32 * (it - 4)) * bm.ldy);
-    };
-    auto put_item = [&](int set, int buf, int it) {
-        if (it < 4)
-            *reinterpret_cast<f32x4*>(&xs[buf][(xr + 16 * it) * kDwLdX + xc]) = px[set][it];
-        else
-            *reinterpret_cast<f32x4*>(&ys[buf][(yr + 32 * (it - 4)) * kDwLdY + yc]) = py[set][it - 4];
-    };
-    f32x16 acc = f32x16{};
-    // lane (i = l % 32, k = l / 32) supplies X[k][wm + i] and Y[k][wn + i]
-    const int ox = (lane >> 5) * kDwLdX + wm + (lane & 31), oy = (lane >> 5) * kDwLdY + wn + (lane & 31);
-    // The MFMAs of the slab in LDS buffer buf, with the next slab's staging
-    // interleaved: after MFMA 4 it + 3, register set s's item it goes to
-    // buffer buf ^ 1 (last read before the previous barrier) and is reloaded
-    // with slab nx's item, so the staging runs in the MFMAs' shadow.
-    auto slab = [&](int buf, int s, uint32_t nx) {
-        const float* xp = xs[buf] + ox;
-        const float* yp = ys[buf] + oy;
-#pragma unroll
-        for (int kk = 0; kk < kDwRows / 2; ++kk) {
-            acc = mfma32x32x2(xp[2 * kk * kDwLdX], yp[2 * kk * kDwLdY], acc);
-            if (kk % 4 == 3 && kk / 4 < 6) {
-                put_item(s, buf ^ 1, kk / 4);
-                load_item(s, kk / 4, nx);
-            }
-        }
-    };
-    // slab 0 in LDS buffer 0, slab 1 in set 1, slab 2 in set 0
-#pragma unroll
-    for (int it = 0; it < 6; ++it) load_item(0, it, 0);
-#pragma unroll
-    for (int it = 0; it < 6; ++it) load_item(1, it, 1);
-#pragma unroll
-    for (int it = 0; it < 6; ++it) put_item(0, 0, it);
-#pragma unroll
-    for (int it = 0; it < 6; ++it) load_item(0, it, 2);
-    __syncthreads();
-    for (uint32_t sl = 0; sl + 1 < steps; sl += 2) {
-        slab(0, 1, sl + 3);  // slab sl; stages slab sl + 1, loads slab sl + 3
-        __syncthreads();
-        slab(1, 0, sl + 4);  // slab sl + 1; stages slab sl + 2, loads slab sl + 4
-        __syncthreads();
-    }
-    if (steps & 1) slab(0, 1, steps);  // the last slab (its staging is not read)
-    float* o = out + bm.off + (size_t)(tm * kDwTileM + wm) * bm.ndim + tn * kDwTileN + wn + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[(size_t)c32_row(r, lane) * bm.ndim] = acc[r];
-}
-
 // The weight gradients with bf16 operands (MG_PRECISION_BF16). X and Y are
 // row-group-packed (element (r, c) at ((r / 8) C + c) 8 + r % 8), so the
 // operand of lane l of a v_mfma_f32_32x32x16_bf16 contracting over rows (rows
 // 8 (l / 32) .. + 7 of column l % 32) is 16 contiguous bytes, and a half-wave
 // reads 512 contiguous bytes: operands go from memory straight into
 // registers, no LDS staging. A workgroup computes one 64 x 64 tile over its
-// row split (workgroup id = tile * splits + split, as in train_dw_kernel);
+// row split (workgroup id = tile * splits + split: workgroups go to the 8 XCDs
+// round robin, so with 8 or 16 splits all tiles of one row split run on the
+// same XCD and share its rows through that XCD's L2);
 // each of its NW waves takes every NW-th 16-row step, with the whole tile as
 // 2 x 2 MFMAs per step, and the NW partial tiles are added in LDS in wave
 // order. U steps are loaded while the previous U run their MFMAs. (Measured at
@@ -1127,6 +1018,173 @@ __global__ void __launch_bounds__(64 * NW) train_dw_fused_kernel(const DwFusedAr
 }
 constexpr int kDwf32Waves = 8, kDwf32U = 8, kDwf32Sets = 2;
 
+// ---- fp32 weight gradients on three bfloat16 planes -----------------------------
+// x = hi + mid + lo exactly, each a bfloat16 (hi truncated, so it never
+// overflows; the rest is exact in fp32): no scale is needed whatever the
+// gradients' range. Six products, hi hi + hi mid + mid hi + hi lo + lo hi + mid
+// mid, leave out terms of at most 2^-24 of a product, and a sum is rounded 6
+// times per 16 rows instead of 16 times (v_mfma_f32_32x32x2_f32).
+struct Planes3 {
+    bf16x8 p[3];
+};
+__device__ __forceinline__ Planes3 split3(const float (&x)[8]) {
+    u32x4 hi, mid, lo;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t b0 = __builtin_bit_cast(uint32_t, x[2 * j]), b1 = __builtin_bit_cast(uint32_t, x[2 * j + 1]);
+        hi[j] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+        const float r0 = x[2 * j] - __builtin_bit_cast(float, b0 & 0xFFFF0000u);
+        const float r1 = x[2 * j + 1] - __builtin_bit_cast(float, b1 & 0xFFFF0000u);
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const bf16x2 m = {(__bf16)r0, (__bf16)r1};
+        mid[j] = __builtin_bit_cast(uint32_t, m);
+        const float s0 = r0 - __builtin_bit_cast(float, mid[j] << 16);
+        const float s1 = r1 - __builtin_bit_cast(float, mid[j] & 0xFFFF0000u);
+        const bf16x2 l = {(__bf16)s0, (__bf16)s1};
+        lo[j] = __builtin_bit_cast(uint32_t, l);
+    }
+    return Planes3{{__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, mid), __builtin_bit_cast(bf16x8, lo)}};
+}
+// acc[m][n] += a[m]^T b[n], the small products first, each product of all four
+// tiles before the next, so no MFMA waits for the one before it.
+__device__ __forceinline__ void mma3(const Planes3 (&a)[2], const Planes3 (&b)[2], f32x16 (&acc)[2][2]) {
+    constexpr int kA[6] = {1, 0, 2, 0, 1, 0}, kB[6] = {1, 2, 0, 1, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+                acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m].p[kA[k]], b[n].p[kB[k]], acc[m][n], 0, 0, 0);
+}
+
+// One 64 x 64 tile (tm, tn) of C = X^T Y over rows [rb, rb + 16 steps), the
+// sums of the NW waves in red ([NW][64 x 64], LDS), after its barrier. Wave w
+// takes the 16-row steps w, w + NW, ...; of a step, lane (i, q) loads rows 8 q
+// .. + 7 of its columns i and i + 32 of both operands as dwords straight from
+// the row-major captures (a half-wave reads one row's 128 bytes), one step
+// ahead.
+template <int NW>
+__device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, uint32_t tn, uint32_t rb,
+                                         uint32_t steps, float* red) {
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const uint32_t i = lane & 31, q = lane >> 5;
+    const uint32_t xv = 4 * (8 * q * bm.ldx + tm * 64 + i), yv = 4 * (8 * q * bm.ldy + tn * 64 + i);
+    auto load = [&](float (&x)[2][8], float (&y)[2][8], uint32_t s) {
+        const uint32_t r = rb + 16 * (s < steps ? s : steps - 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                x[h][j] = buffer_load4(bm.x, xv + 128 * h, 4 * (r + j) * bm.ldx);
+                y[h][j] = buffer_load4(bm.y, yv + 128 * h, 4 * (r + j) * bm.ldy);
+            }
+    };
+    f32x16 acc[2][2] = {};
+    float x[2][2][8], y[2][2][8];
+    auto step = [&](int b) {
+        Planes3 px[2], py[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) px[h] = split3(x[b][h]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) py[h] = split3(y[b][h]);
+        mma3(px, py, acc);
+    };
+    load(x[0], y[0], w);
+    for (uint32_t s = w; s < steps; s += 2 * NW) {
+        load(x[1], y[1], s + NW);
+        __builtin_amdgcn_sched_barrier(0);
+        step(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + NW < steps) {
+            load(x[0], y[0], s + 2 * NW);
+            __builtin_amdgcn_sched_barrier(0);
+            step(1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    float* rw = red + w * 4096;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) rw[(32 * m + c32_row(r, lane)) * 64 + 32 * n + i] = acc[m][n][r];
+    __syncthreads();
+}
+
+// Workgroup b of T on XCD b % 8 takes the b / 8-th of that XCD's run of T / 8
+// work items, so an XCD's tiles share their captures' columns in its L2.
+__device__ __forceinline__ uint32_t xcd_item(uint32_t b, uint32_t T) {
+    return T % 8 ? b : (b % 8) * (T / 8) + b / 8;
+}
+
+// Tile t of the block matrices in order (matrix, hidden block, embed block).
+__device__ __forceinline__ void dw3_locate(uint32_t t, uint32_t per, uint32_t& mi, uint32_t& hb, uint32_t& eb) {
+    mi = t / per, eb = (t % per) % (kEmbed / 64), hb = (t % per) / (kEmbed / 64);
+}
+
+// The weight gradients over row splits: one tile and split per workgroup, to
+// the splits' partial arenas (grad_reduce_kernel adds them). Next to
+// train_dw_fused_kernel a 64 x 64 tile reads half the captures per product,
+// but writes partial sums for a further launch (6.5 us): us for both at hidden
+// 512, 53.0 + 8.8 against 71.7 with 2 blocks at 16384 rows, 30.2 + 6.5 against
+// 44.5 with 4 at 4096, 19.1 + 6.4 against 21.5 with 2 at 4096; hence the line at
+// twice the work of 2 blocks at 4096 rows (launch_train_step).
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) train_dw3_kernel(const DwArgsT<float> a) {
+    __shared__ float red[NW * 4096];
+    const uint32_t item = xcd_item(blockIdx.x, gridDim.x), split = item / a.big_tiles, t = item % a.big_tiles;
+    uint32_t mi, hb, eb;
+    dw3_locate(t, a.tiles_per_big[0], mi, hb, eb);
+    const BigMatT<float>& bm = a.big[mi];
+    const bool up = bm.mdim == (uint32_t)kEmbed;
+    const uint32_t tm = up ? eb : hb, tn = up ? hb : eb, per = a.rows / a.splits;
+    dw3_tile<NW>(bm, tm, tn, split * per, per / 16, red);
+    float* out = a.partial + (size_t)split * a.count + bm.off + (size_t)tm * 64 * bm.ndim + tn * 64;
+    for (int e = threadIdx.x; e < 4096; e += 64 * NW) {
+        float v = red[e];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) v += red[k * 4096 + e];
+        out[(size_t)(e >> 6) * bm.ndim + (e & 63)] = v;
+    }
+}
+
+// The same over all rows, with the tile-partial columns and the norm parts, as
+// train_dw_fused_kernel: where the tiles alone fill the GPU. 4 blocks, hidden
+// 1024, 16384 rows: 368 -> 190 us. The captures' 604 MB take 116 us from HBM and
+// the products 85 us; a wave's splits (176 vector instructions per 24 MFMAs)
+// overlap its SIMD's other wave's MFMAs only in part.
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) train_dw3_fused_kernel(const DwFusedArgs<float> a) {
+    __shared__ float red[NW * 4096];
+    float sq = 0.0f;
+    const uint32_t T = a.dw.big_tiles;
+    if (blockIdx.x >= T) {
+        sq = reduce_tile_partials<64 * NW>(a.red, blockIdx.x - T, gridDim.x - T);
+    } else {
+        uint32_t mi, hb, eb;
+        dw3_locate(xcd_item(blockIdx.x, T), a.dw.tiles_per_big[0], mi, hb, eb);
+        const BigMatT<float>& bm = a.dw.big[mi];
+        const bool up = bm.mdim == (uint32_t)kEmbed;
+        const uint32_t tm = up ? eb : hb, tn = up ? hb : eb;
+        dw3_tile<NW>(bm, tm, tn, 0, a.dw.rows / 16, red);
+        float* out = a.red.grad + bm.off + (size_t)tm * 64 * bm.ndim + tn * 64;
+        for (int e = threadIdx.x; e < 4096; e += 64 * NW) {
+            float v = red[e];
+#pragma unroll
+            for (int k = 1; k < NW; ++k) v += red[k * 4096 + e];
+            out[(size_t)(e >> 6) * bm.ndim + (e & 63)] = v;
+            sq += v * v;
+        }
+        if (gridDim.x == T) sq += reduce_tile_partials<64 * NW>(a.red, blockIdx.x, gridDim.x);
+    }
+    write_norm_part<NW>(sq, a.red.normpart + blockIdx.x);
+    if (blockIdx.x == 0)
+        for (uint32_t k = gridDim.x + threadIdx.x; k < (uint32_t)kReduceBlocks; k += 64 * NW) a.red.normpart[k] = 0.0f;
+}
+constexpr int kDw3Waves = 8;
+
 // The block matrices are contiguous from float_group: per block up [128 x H]
 // then down [H x 128]. Both matrix kinds split into (128 x H) / 1024 tiles of
 // 32 x 32; tile t's matrix, its row/column extents and the tile's origin.
@@ -1382,9 +1440,11 @@ __device__ __forceinline__ float adam_clip_scale(const AdamArgs& a) {
 // Workgroups [0, mat_tiles) update one 32 x 32 block-matrix tile each and
 // write it to the fragment-tiled copies as well; the rest update the vector
 // group and the head elementwise. Workgroup 0 also records the pre-clip norm.
+// PAIRS: the tiles go to the pair planes instead (policy_pair.h).
+template <bool PAIRS>
 __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
     __shared__ float lds[kTT * kTileLd];
-    __shared__ float wmax[4];
+    __shared__ float wmax[PAIRS ? 4 : 1];
     constexpr int PER = kTT * kTT / 256;  // tile elements per thread
     const int t = threadIdx.x;
     if (blockIdx.x < a.mat_tiles) {
@@ -1399,8 +1459,8 @@ __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
             in[e] = adam_load(a, idx[e]);
         }
         const uint32_t per = a.hidden * kEmbed / (kTT * kTT), mat = blockIdx.x / per;
-        PairScale* const pairs = a.pair_fwd ? pair_scale(a.pair_fwd, a.count) : nullptr;
-        const int exp = pairs ? pairs->next[mat] : 0;
+        PairScale* const pairs = PAIRS ? pair_scale(a.pair_fwd, a.count) : nullptr;
+        const int exp = PAIRS ? pairs->next[mat] : 0;
         const float scale = adam_clip_scale(a);
         float most = 0.0f;
 #pragma unroll
@@ -1408,9 +1468,9 @@ __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
             const int r = (256 / kTT) * e + t / kTT;
             const float p = adam_elem(a, idx[e], in[e], scale);
             lds[r * kTileLd + c] = p;
-            most = fmaxf(most, fabsf(p));
+            if (PAIRS) most = fmaxf(most, fabsf(p));
         }
-        if (pairs) {  // this tile's planes, and what the next step's exponent needs (PairScale)
+        if constexpr (PAIRS) {  // this tile's planes, and what the next step's exponent needs (PairScale)
             most = group_max<64>(most);
             if ((t & 63) == 0) wmax[t >> 6] = most;
             __syncthreads();
@@ -1588,13 +1648,13 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
              "train: OBS_DIM <= 64 and ACT_DIM + 1 <= 64 required");
     const uint32_t E = MG_EMBED, L = pv.layers, H = pv.hidden;
     const bool bf = pv.precision == MG_PRECISION_BF16;
-    // weight-gradient tiles over all block matrices: 128 x 64 (fp32) or 64 x 64 (bf16)
-    const uint32_t dw_tiles = bf ? 2 * L * (E / 64) * (H / 64) : 2 * L * (E * H / (dev::kDwTileM * dev::kDwTileN));
-    // row splits of the block-matrix gradient sums: fp32, each split covers a
-    // multiple of 32 rows and about one workgroup per CU in all; bf16, a
-    // multiple of 64 rows and about two workgroups per CU (fewer splits, fewer
-    // partial sums to write and add)
-    const uint32_t split_rows = bf ? 16 * dev::kDwbWaves : dev::kDwRows;
+    // 64 x 64 weight-gradient tiles over all block matrices
+    const uint32_t tiles64 = 2 * L * (E / 64) * (H / 64);
+    const uint32_t dw_tiles = tiles64;
+    // row splits of the block-matrix gradient sums: each split covers a
+    // multiple of 64 rows, in fp32 about one workgroup per CU in all, in bf16
+    // about two (fewer splits, fewer partial sums to write and add)
+    const uint32_t split_rows = 64;
     const uint32_t max_wgs = bf ? 512 : 256;
     uint32_t splits = kSplits;
     while (splits > 1 && (B % (splits * split_rows) != 0 || dw_tiles * splits > max_wgs)) splits /= 2;
@@ -1649,7 +1709,18 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
     // fused with the tile-partial sums (one launch instead of two; fp32 at
     // 4096 rows, 2 blocks, hidden 512: 71.8 -> 67.9 us per minibatch)
     const uint32_t tiles32 = 2 * L * (E / 32) * (H / 32);
-    if (bf && tiles32 >= 128 && tiles32 <= (uint32_t)kReduceBlocks && B % (16 * dev::kDwfWaves) == 0) {
+    // enough work for dw3's partial sums to pay (train_dw3_kernel)
+    const bool wide = (uint64_t)tiles64 * B >= 2u * 64u * 4096u;
+    if (!bf && tiles64 >= 256 && tiles64 <= (uint32_t)kReduceBlocks) {
+        TimedLaunch tl(MG_K_TRAIN_DW, st);
+        dev::DwFusedArgs<float> fa;
+        fa.dw = dw_args<float>(pv, ws, B, 1, 64);
+        fa.red = ga;
+        const uint32_t grid = tiles64 + ga.small_wgs <= (uint32_t)kReduceBlocks ? tiles64 + ga.small_wgs : tiles64;
+        hipLaunchKernelGGL((dev::train_dw3_fused_kernel<dev::kDw3Waves>), dim3(grid), dim3(64 * dev::kDw3Waves), 0, st,
+                           fa);
+        MG_HIP(hipGetLastError(), "train dW launch");
+    } else if (bf && tiles32 >= 128 && tiles32 <= (uint32_t)kReduceBlocks && B % (16 * dev::kDwfWaves) == 0) {
         TimedLaunch tl(MG_K_TRAIN_DW, st);
         dev::DwFusedArgs<uint16_t> fa;
         fa.dw = dw_args<uint16_t>(pv, ws, B, 1, 32);
@@ -1658,7 +1729,7 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         hipLaunchKernelGGL((dev::train_dw_bf16_fused_kernel<dev::kDwfWaves, 4>), dim3(grid),
                            dim3(64 * dev::kDwfWaves), 0, st, fa);
         MG_HIP(hipGetLastError(), "train dW launch");
-    } else if (!bf && tiles32 >= 128 && tiles32 <= (uint32_t)kReduceBlocks &&
+    } else if (!bf && !wide && tiles32 >= 128 && tiles32 <= (uint32_t)kReduceBlocks &&
                B % (2 * dev::kDwf32Waves * dev::kDwf32U * dev::kDwf32Sets) == 0) {
         TimedLaunch tl(MG_K_TRAIN_DW, st);
         dev::DwFusedArgs<float> fa;
@@ -1678,9 +1749,9 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
                 hipLaunchKernelGGL((dev::train_dw_bf16_kernel<dev::kDwbWaves, 2>), dim3(dw_tiles * splits),
                                    dim3(64 * dev::kDwbWaves), 0, st, da);
             } else {
-                const auto da = dw_args<float>(pv, ws, B, splits, dev::kDwTileM, dev::kDwTileN);
-                hipLaunchKernelGGL(dev::train_dw_kernel, dim3(dw_tiles * splits), dim3(64 * dev::kDwWaves), 0, st,
-                                   da);
+                const auto da = dw_args<float>(pv, ws, B, splits, 64);
+                hipLaunchKernelGGL((dev::train_dw3_kernel<dev::kDw3Waves>), dim3(dw_tiles * splits),
+                                   dim3(64 * dev::kDw3Waves), 0, st, da);
             }
             MG_HIP(hipGetLastError(), "train dW launch");
         }
@@ -1720,7 +1791,11 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         aa.beta2_pow = step.beta2_pow;
         aa.max_grad_norm = hp.max_grad_norm;
         const uint32_t lin = pv.float_group + (pv.count - pv.off_head);
-        hipLaunchKernelGGL(dev::adam_kernel, dim3(aa.mat_tiles + (lin + 255) / 256), dim3(256), 0, st, aa);
+        const dim3 grid(aa.mat_tiles + (lin + 255) / 256);
+        if (pairs)
+            hipLaunchKernelGGL(dev::adam_kernel<true>, grid, dim3(256), 0, st, aa);
+        else
+            hipLaunchKernelGGL(dev::adam_kernel<false>, grid, dim3(256), 0, st, aa);
         MG_HIP(hipGetLastError(), "adam launch");
     }
     return MG_OK;

@@ -1,0 +1,49 @@
+"""The fp32 PPO minibatch on binary16 pairs (policy_pair.h) and its weight
+gradients on three bfloat16 planes, at the edges of their shapes: one minibatch
+against the oracle's train step, and the operand copies that Adam keeps against
+the parameters they stand for after many large steps."""
+import numpy as np
+import pytest
+
+from parity import ENVS, check_minibatch
+from test_gpu_lane import network64
+from test_gpu_train import block_rows, setup
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("env,n,B,layers,scale", [
+    ("cartpole", 64, 64, 1, 1),               # 4 groups of hidden units for 8 waves; 4 steps for 8 waves
+    ("cartpole", 640, 320, 2, 3),             # 12 groups: waves of one and of two
+    ("cartpole_continuous", 192, 192, 3, 5),  # 20 groups
+    ("voxelnav16", 128, 128, 2, 2),           # one group per wave, 30 observation floats
+    ("cartpole", 64, 64, 4, 8),               # gradient tiles that fill the GPU, fewer steps than waves
+    ("cartpole_continuous", 320, 320, 4, 8),  # 20 steps of 16 rows over 8 waves
+    ("cartpole", 4096, 4096, 4, 4),           # the first work of the row-split gradients
+    ("cartpole", 128, 128, 5, 1),             # past the pair layout's LDS: the fp32 row pass
+])
+def test_minibatch(mg, orc, env, n, B, layers, scale):
+    gym, model, d = setup(mg, orc, env, n, 2, B, layers=layers, scale=scale)
+    s, p0 = model.download_slots(), model.params()
+    model.train_block(1)
+    check_minibatch(model, orc, d, orc.hparams(), p0, block_rows(s, n, B, 1), B)
+
+
+@pytest.mark.parametrize("lr,epochs", [(3e-4, 2), (0.05, 5), (1.0, 3)])
+def test_copies_follow_the_parameters(mg, lr, epochs):
+    """Adam writes its planes with exponents made before the step, from the
+    largest weight and from how far one step can move it. After training, the
+    head that the next minibatch's row pass computes from them must be the
+    parameters' (relative to the row's largest: 1e-4 as the policy heads
+    elsewhere)."""
+    n = 1024
+    gym = mg.Gym(ENVS["cartpole"][1], n, 0)
+    model = mg.PPOModel(gym, horizon=4, minibatch=256, lr=lr)
+    model.collect()
+    model.train(epochs)
+    p, obs = model.params(), model.download_slots()["obs"]
+    assert np.isfinite(p).all()
+    model.train_block(5)  # slot 1, rows 256 .. 511
+    want = network64(model.pv, p, obs[1][256:512])
+    err = np.abs(model.head() - want) / np.maximum(1.0, np.abs(want).max(1, keepdims=True))
+    assert float(err.max()) <= 1e-4, float(err.max())
