@@ -18,6 +18,7 @@
 #pragma once
 #include "policy_bf16.h"
 #include "policy_lane.h"
+#include "policy_pair.h"
 #include "policy_split.h"
 #include "sample.h"
 
@@ -495,6 +496,175 @@ __global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_colle
     }
 }
 
+// collect of 16-row tiles with the forward on pairs (pair_forward): eight
+// waves, one workgroup per CU, env lanes 0 .. 15 of wave 0.
+template <typename Env>
+struct CollectPair {
+    static constexpr int O = Env::OBS_DIM, HD = Env::ACT_DIM + 1;
+    static constexpr bool OK = O <= 16 && HD <= 16 && EnvTraits<Env>::STATE_IN_REGISTERS;
+    static constexpr bool EDGE = !EnvTraits<Env>::CONTINUOUS && Env::ACT_DIM > 1;
+    // floats of the small parameters, each array a multiple of 4
+    __host__ __device__ static constexpr uint32_t small(uint32_t layers) {
+        return O * kEmbed + kEmbed + (layers + 1) * 2 * kEmbed + kEmbed * HD;
+    }
+};
+
+template <typename Env>
+__global__ void __launch_bounds__(64 * kPairW, 1) collect_pair_kernel(const mg_collect_args a) {
+    using CP = CollectPair<Env>;
+    using Tr = EnvTraits<Env>;
+    using State = typename Env::State;
+    using Action = typename Env::Action;
+    using Obs = typename Env::Obs;
+    constexpr int M = kSplitRows, NT = 64 * kPairW, O = CP::O, A = Env::ACT_DIM, HD = CP::HD;
+    __shared__ PairFwdSmem sm;
+    __shared__ float obsL[M * O];
+    __shared__ float headL[M * HD];
+    __shared__ float edgeHead[HD];
+    __shared__ uint32_t near;  // env lanes whose draw fell near an edge
+    extern __shared__ __align__(16) float small_lds[];
+
+    const int tid = threadIdx.x;
+    const uint32_t n = a.n, T = a.horizon, i = blockIdx.x * M + (uint32_t)tid;
+    const bool envLane = tid < M;
+    State* states = static_cast<State*>(a.state);
+    Action* actSlots = static_cast<Action*>(a.action_slots);
+    const float* logStd = a.policy.params + a.policy.off_log_std;
+
+    PairFwd F;
+    F.start(a.policy);
+    SmallParams sp = small_params(a.policy);
+    {
+        const int lnf = (int)(a.policy.layers + 1) * 2 * kEmbed;
+        float* win = small_lds;
+        float* bin = win + O * kEmbed;
+        float* ln = bin + kEmbed;
+        float* wh = ln + lnf;
+        for (int k = tid; k < O * kEmbed; k += NT) win[k] = sp.win[k];
+        for (int k = tid; k < kEmbed; k += NT) bin[k] = sp.bin[k];
+        for (int k = tid; k < lnf; k += NT) ln[k] = sp.ln[k];
+        for (int k = tid; k < kEmbed * HD; k += NT) wh[k] = sp.wh[k];
+        sp = {win, bin, ln, wh};
+        if (tid < 2 * MG_MAX_LAYERS) sm.exps[tid] = pair_scale(a.policy.frag_fwd16_bf, a.policy.count)->cur[tid];
+    }
+    uint32_t rng = 0;
+    uint8_t done = 0;
+    State st;
+    auto env_step = [&](const Action& act, size_t slot, float& r) {
+        if (done) Env::reset(st, rng);
+        Obs o{};
+        Env::step(st, act, o, r, done);
+        const float* of = reinterpret_cast<const float*>(&o);
+        float obs[O];
+#pragma unroll
+        for (int k = 0; k < O; ++k) obs[k] = of[k];
+        store_floats<O>(a.obs_slots + slot * O, obs);
+#pragma unroll
+        for (int k = 0; k < O; ++k) obsL[tid * O + k] = obs[k];
+    };
+    if (envLane) {
+        rng = a.rng[i];
+        done = a.done[i];
+        st = states[i];
+        if (a.first) {  // model/ppo.h:720-722: one step with action 0 into slot 0
+            Action act{};
+            float r = 0.0f;
+            env_step(act, i, r);
+            a.reward_slots[i] = r;
+        } else {  // model/ppo.h:724: obs[T] -> obs[0]
+            float obs[O];
+            load_floats<O>(obs, a.obs_slots + ((size_t)T * n + i) * O);
+            store_floats<O>(a.obs_slots + (size_t)i * O, obs);
+#pragma unroll
+            for (int k = 0; k < O; ++k) obsL[tid * O + k] = obs[k];
+        }
+    }
+    __syncthreads();
+
+    for (uint32_t t = 0; t <= T; ++t) {
+        pair_forward<O>(a.policy, sp, sm, F, obsL, O, headL, HD);
+        if (t == T) {  // bootstrap head for GAE and headValue()
+            if (envLane) {
+#pragma unroll
+                for (int j = 0; j < HD; ++j) a.head_out[(size_t)i * HD + j] = headL[tid * HD + j];
+            }
+            break;
+        }
+        const size_t k = (size_t)t * n + i;
+        const uint32_t rng0 = rng;
+        Action act{};
+        float r = 0.0f, lp = 0.0f, edge = 1.0f;
+        if (envLane) {
+            const float* h = headL + tid * HD;
+            if constexpr (Tr::CONTINUOUS)
+                sample_gaussian(h, logStd, A, rng, reinterpret_cast<float*>(&act), lp);
+            else
+                act = (Action)sample_categorical(h, A, rng, lp, CP::EDGE ? &edge : nullptr);
+        }
+        if constexpr (CP::EDGE) {
+            // draws near an edge take the action of the fp32 tiles' arithmetic
+            // (policy_lane.h): of the 32-row tile from 8192 envs, else of
+            // split_forward16
+            if (tid < 64) {
+                const uint64_t b = __ballot(envLane && edge <= kLaneEdge);
+                if (tid == 0) near = (uint32_t)b;
+            }
+            __syncthreads();
+            for (uint32_t rest = near; rest; rest &= rest - 1) {
+                const int e = __builtin_ctz(rest);
+                if (n >= 32u * 256u) {
+                    if (tid < 64) tile_row_head<16, O, HD>(a.policy, obsL + e * O, &sm.red[0][0], edgeHead);
+                    __syncthreads();
+                } else {
+                    split_row_head<O, HD>(a.policy, sp, obsL + e * O, blockIdx.x, &sm.red[0][0], edgeHead);
+                }
+                if (tid == e) {
+                    const float mine = lp;
+                    uint32_t s = rng0;
+                    const Action own = act;
+                    act = (Action)sample_categorical(edgeHead, A, s, lp);
+                    if (act == own) lp = mine;
+                }
+                __syncthreads();  // edgeHead and red are free again
+            }
+        }
+        if (envLane) {
+            actSlots[k] = act;
+            a.logp_slots[k] = lp;
+            a.value_slots[k] = headL[tid * HD + A];
+            env_step(act, k + n, r);
+            a.reward_slots[k] = r;
+            a.done_slots[k] = done;
+        }
+        __syncthreads();
+    }
+    if (envLane) {
+        states[i] = st;
+        a.rng[i] = rng;
+        a.done[i] = done;
+    }
+}
+
+// Runs the collect on collect_pair_kernel where that is the faster: under 16384
+// envs (up to four workgroups per CU, one after the other) of an env with at most
+// 16 observation floats and a register-held State. ms a collect of 32 steps,
+// CartPole, split_forward16 or the 32-row tiles against this: 0.63 / 0.40 at 64
+// envs, 0.65 / 0.46 at 4096, 1.34 / 0.83 at 8192, 2.32 / 1.22 at 12288, 2.32 /
+// 1.73 at 16384 (collect_lane_kernel 1.71). A step takes 14 us at 4096 envs, of
+// which the weights' 1 MB through each CU's L1 is about 11.
+template <typename Env>
+bool launch_collect_pair(const mg_collect_args* a, hipStream_t st) {
+    using CP = CollectPair<Env>;
+    if constexpr (CP::OK) {
+        if (a->policy.precision != MG_PRECISION_FP32 || a->n >= 16384u || !a->policy.frag_fwd16_bf) return false;
+        hipLaunchKernelGGL((collect_pair_kernel<Env>), dim3(a->n / kSplitRows), dim3(64 * kPairW),
+                           CP::small(a->policy.layers) * 4, st, *a);
+        return true;
+    } else {
+        return false;
+    }
+}
+
 // The kernel's static LDS as the compiler laid it out (SIZE_MAX if the
 // runtime cannot tell, which turns the small-parameter staging off).
 template <typename Env, int M, bool BF16, bool WIDE>
@@ -566,6 +736,7 @@ bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
 template <typename Env, bool BF16>
 int launch_collect_tiles(const mg_collect_args* a) {
     hipStream_t st = static_cast<hipStream_t>(a->stream);
+    if (launch_collect_pair<Env>(a, st)) return (int)hipGetLastError();
     if (launch_collect_lane<Env, BF16 ? MG_PRECISION_BF16 : MG_PRECISION_FP32>(a, st)) return (int)hipGetLastError();
     // 64-row tiles reuse each weight fragment across the most rows; they need
     // n / 64 >= 512 workgroups (2 per CU) to fill the chip. Smaller runs use

@@ -56,10 +56,12 @@ __host__ __device__ __forceinline__ PairScale* pair_scale(uint16_t* planes, uint
 // The exponent of a matrix whose largest magnitude is m.
 __device__ __forceinline__ int pair_exp(float m) { return split_min(kMatTarget - pow2_above(m), 40); }
 
-// A wave's position in the forward's blocks and then the backward's.
+// A wave's position in the forward's blocks and then the backward's (FWD_ONLY:
+// the forward's, again and again).
 struct PairPos {
     int bwd, l, k;
 };
+template <bool FWD_ONLY = false>
 struct PairSeq {
     const uint16_t* fwd;  // frag_fwd16_bf + 2 float_group: up in role 0, down in role 1
     const uint16_t* bwd;  // frag_bwd16_bf + 2 float_group: up in role 1, down in role 0
@@ -78,6 +80,7 @@ struct PairSeq {
         p.k = 0;
         if (!p.bwd) {
             if (++p.l < L) return p;
+            if (FWD_ONLY) return PairPos{0, 0, 0};
             p.bwd = 1;
             p.l = L - 1;
             return p;
@@ -194,6 +197,191 @@ __device__ __forceinline__ void pair_pack(const float (&x)[8], f16x8 (&p)[2]) {
         p[0][2 * j] = hi[0], p[0][2 * j + 1] = hi[1];
         p[1][2 * j] = lo[0], p[1][2 * j + 1] = lo[1];
     }
+}
+
+// LDS of pair_forward: the block input, the waves' partials of a block output
+// (scratch for split_row_head between the forwards) and the planes' exponents.
+struct alignas(16) PairFwdSmem {
+    PairInput in;
+    float red[kPairW][kSplitRows * kLds];
+    int exps[2 * MG_MAX_LAYERS];
+};
+
+// A wave's weight stream, carried from one forward to the next: the last
+// group's refills are the next forward's first operands.
+struct PairFwd {
+    PairStream wst;
+    PairSeq<true> seq;
+    PairPos pos;
+    __device__ __forceinline__ void start(const mg_policy_view& pv) {
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        const int nk = ((int)(pv.hidden / kPairGroup) - wave + kPairW - 1) / kPairW;
+        const int rot = nk > 0 ? (wave + (int)(blockIdx.x >> 3)) % nk : 0;
+        seq = PairSeq<true>{pv.frag_fwd16_bf + 2 * (size_t)pv.float_group, nullptr, (int)pv.layers, nk, wave, rot,
+                            (uint32_t)kEmbed * pv.hidden};
+        pos = PairPos{0, 0, 0};
+        if (nk > 0) wst.start(seq.role(pos, 0), seq.role(pos, 1));
+    }
+};
+
+// split_forward16 (policy_split.h) with the block GEMMs on pairs: obs staged in
+// obsL ([16][O], LDS) -> head in headL ([16][HD], LDS), ending with a barrier.
+// OC: O where it is known at compile time, else 0.
+template <int OC>
+__device__ __forceinline__ void pair_forward(const mg_policy_view& pv, const SmallParams& sp, PairFwdSmem& sm,
+                                             PairFwd& F, const float* obsL, int O, float* headL, int HD) {
+    constexpr int TPR = 64 * kPairW / kSplitRows;  // 32 threads per row, four columns each
+    constexpr int kUnroll = OC > 0 ? OC : 4;
+    const int tid = threadIdx.x, wave = F.seq.wave, On = OC > 0 ? OC : O;
+    const int row = tid / TPR, lk = tid % TPR, c0 = 4 * lk, NL = (int)pv.layers;
+    RowVec<1> h = rv_load<1>(sp.bin + c0);  // model/input.metal:11-27
+#pragma unroll kUnroll
+    for (int k = 0; k < On; ++k) {
+        const float ok = obsL[row * On + k];
+        const RowVec<1> w = rv_load<1>(sp.win + k * kEmbed + c0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) h[c] = __builtin_fmaf(ok, w[c], h[c]);
+    }
+    RowVec<1> x, xn;
+    float sd;
+    for (int l = 0; l < NL; ++l) {
+        sk_layernorm<TPR>(h, sp.ln + l * 2 * kEmbed, sp.ln + l * 2 * kEmbed + kEmbed, c0, x, xn, sd);
+        const int unit = pair_store_input<TPR>(sm.in, x, row, lk, 0) + sm.exps[2 * l] + kHiddenExp + sm.exps[2 * l + 1];
+        __syncthreads();  // X complete; every wave is past its reads of red
+        f16x8 xb[4][2];
+        pair_load_input(sm.in, xb);
+        f32x4 hp[8];
+#pragma unroll
+        for (int ct = 0; ct < 8; ++ct) hp[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k = 0; k < F.seq.nk; ++k) {  // model/mlp.metal:18-86 for one of this wave's groups
+            const PairPos nx = F.seq.next(F.pos);
+            f32x4 v[2] = {};
+            F.wst.gemm0(v, xb, F.seq.role(nx, 0));
+            float t[8];
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) t[4 * s + r] = v[s][r];
+            f16x8 vb[2];
+            LaneOps<MG_PRECISION_FP32>::pack_hidden(t, vb);
+            F.wst.gemm1(hp, vb, F.seq.role(nx, 1));
+            F.pos = nx;
+        }
+        RowVec<1> d = sk_reduce_buf<kPairW, 1>(&sm.red[0][0], hp, wave, row, c0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) h[c] += __builtin_ldexpf(d[c], -unit);  // model/elementwise.metal:4-13
+    }
+    sk_layernorm<TPR>(h, sp.ln + NL * 2 * kEmbed, sp.ln + NL * 2 * kEmbed + kEmbed, c0, x, xn, sd);
+    for (int j = 0; j < HD; ++j) {  // model/linear.metal:17-37
+        float acc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc = __builtin_fmaf(x[c], sp.wh[(c0 + c) * HD + j], acc);
+        acc = group_sum<TPR>(acc);
+        if (lk == 0) headL[row * HD + j] = acc;
+    }
+    __syncthreads();
+}
+
+// One row's head as split_forward16 computes it, bit for bit, by the whole
+// workgroup of 8 waves (policy_lane.h says what for): V one unit per thread,
+// then wave w adds its units' products into its partial, two columns per lane.
+// Orders: an MFMA's k = 16 g + 4 q + j over g, j, q; the second GEMM's units 4
+// q + j of a strip over j, q, the wave's chunks from its rotation; a row's sums
+// over four columns, then 32 threads as group_sum does; the partials in wave
+// order. block: the tile's workgroup index there. lds: scratch of (hidden + 8 *
+// 128 + 2 * 128 + 32) floats, dead otherwise. Starts and ends with a barrier.
+template <int OC, int HD>
+__device__ __forceinline__ void split_row_head(const mg_policy_view& pv, const SmallParams& sp, const float* obs,
+                                               uint32_t block, float* lds, float* head) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int H = (int)pv.hidden, NC = H / kChunk;
+    float* vs = lds;               // [hidden]
+    float* part = lds + H;         // [8][128]
+    float* hs = part + 8 * kEmbed;  // [128] residual stream
+    float* xs = hs + kEmbed;       // [128] LN output
+    float* rs = xs + kEmbed;       // [32]
+    __syncthreads();
+    if (tid < kEmbed) {
+        float h = sp.bin[tid];
+        for (int k = 0; k < OC; ++k) h += obs[k] * sp.win[k * kEmbed + tid];
+        hs[tid] = h;
+    }
+    // sum over the row of f(column): four columns per thread in order, then the
+    // 32 threads' pairing of group_sum<32>; every thread computes it
+    auto row_sum = [&](auto f) {
+        __syncthreads();
+        if (tid < 32) {
+            float s = f(4 * tid);
+#pragma unroll
+            for (int c = 1; c < 4; ++c) s += f(4 * tid + c);
+            rs[tid] = s;
+        }
+        __syncthreads();
+        float q[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q[i] = (rs[4 * i] + rs[4 * i + 1]) + (rs[4 * i + 2] + rs[4 * i + 3]);
+        return ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+    };
+    auto layernorm = [&](int l) {
+        const float mean = row_sum([&](int c) { return hs[c]; }) / (float)kEmbed;
+        const float q = row_sum([&](int c) {
+            const float d = hs[c] - mean;
+            return d * d;
+        });
+        const float rstd = 1.0f / sqrtf(q / (float)kEmbed + 1e-5f);
+        if (tid < kEmbed) {
+            const float xn = (hs[tid] - mean) * rstd;
+            xs[tid] = sp.ln[2 * kEmbed * l + tid] * xn + sp.ln[2 * kEmbed * l + kEmbed + tid];
+        }
+        __syncthreads();
+    };
+    for (int l = 0; l < (int)pv.layers; ++l) {
+        layernorm(l);
+        for (int u = tid; u < H; u += 64 * kPairW) {
+            const float* up = pv.params + pv.off_up[l] + u;
+            float v = 0.0f;
+#pragma unroll 1
+            for (int g = 0; g < 8; ++g) {
+                float w[16];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) w[k] = up[(size_t)(16 * g + k) * H];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v = __builtin_fmaf(w[4 * q + j], xs[16 * g + 4 * q + j], v);
+            }
+            vs[u] = v > 0.0f ? v : 0.0f;
+        }
+        __syncthreads();
+        float p[2] = {0.0f, 0.0f};
+        const int rot = (wave + (int)(block >> 3)) % NC;
+#pragma unroll 1
+        for (int k = 0; k < NC; ++k) {
+            const int c = k + rot < NC ? k + rot : k + rot - NC;
+            const int u0 = kChunk * c + 16 * wave;
+            const float* dn = pv.params + pv.off_down[l] + (size_t)u0 * kEmbed + lane;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        p[i] = __builtin_fmaf(vs[u0 + 4 * q + j], dn[(4 * q + j) * kEmbed + 64 * i], p[i]);
+        }
+        part[wave * kEmbed + lane] = p[0], part[wave * kEmbed + 64 + lane] = p[1];
+        __syncthreads();
+        if (tid < kEmbed) {
+            float s = part[tid];
+            for (int w = 1; w < kPairW; ++w) s += part[w * kEmbed + tid];
+            hs[tid] = hs[tid] + s;
+        }
+    }
+    layernorm((int)pv.layers);
+    for (int j = 0; j < HD; ++j) {
+        const float s = row_sum([&](int c) { return xs[c] * sp.wh[c * HD + j]; });
+        if (tid == 0) head[j] = s;
+    }
+    __syncthreads();
 }
 
 // Where element (unit u of a matrix's hidden index, column k of the embed) of a

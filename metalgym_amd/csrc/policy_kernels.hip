@@ -4,6 +4,7 @@
 #include "kernels.h"
 #include "mg/device/policy_bf16.h"
 #include "mg/device/policy_lane.h"
+#include "mg/device/policy_pair.h"
 #include "mg/device/sample.h"
 
 namespace mg {
@@ -66,6 +67,45 @@ __global__ void __launch_bounds__(kLaneNT, 2) forward_lane_kernel(const mg_polic
         for (int j = 0; j < HC; ++j)
             if (j < HD) head[(size_t)r * HD + j] = hv[j];
     }
+}
+
+// The same in 16-row tiles with the fp32 products on pairs (policy_pair.h), one
+// workgroup per CU. Dynamic LDS: the small parameters, the observations and the
+// heads.
+__host__ __device__ __forceinline__ uint32_t forward_pair_floats(uint32_t O, uint32_t HD, uint32_t layers) {
+    return O * kEmbed + kEmbed + (layers + 1) * 2 * kEmbed + kEmbed * HD + kSplitRows * (O + HD);
+}
+__global__ void __launch_bounds__(64 * kPairW, 1) forward_pair_kernel(const mg_policy_view pv,
+                                                                      const float* __restrict__ obs, uint32_t rows,
+                                                                      float* __restrict__ head) {
+    constexpr int NT = 64 * kPairW, M = kSplitRows;
+    __shared__ PairFwdSmem sm;
+    extern __shared__ __align__(16) float pair_lds[];
+    const int tid = threadIdx.x, O = (int)pv.obs_dim, HD = (int)pv.head_dim;
+    const int lnf = (int)(pv.layers + 1) * 2 * kEmbed;
+    PairFwd F;
+    F.start(pv);
+    SmallParams sp = small_params(pv);
+    float* win = pair_lds;
+    float* bin = win + O * kEmbed;
+    float* ln = bin + kEmbed;
+    float* wh = ln + lnf;
+    float* obsL = wh + kEmbed * HD;
+    float* headL = obsL + M * O;
+    const uint32_t row0 = blockIdx.x * M;
+#pragma unroll 4
+    for (int k = tid; k < O * kEmbed; k += NT) win[k] = sp.win[k];
+    for (int k = tid; k < kEmbed; k += NT) bin[k] = sp.bin[k];
+    for (int k = tid; k < lnf; k += NT) ln[k] = sp.ln[k];
+#pragma unroll 4
+    for (int k = tid; k < kEmbed * HD; k += NT) wh[k] = sp.wh[k];
+    for (int k = tid; k < M * O; k += NT) obsL[k] = row0 + k / O < rows ? obs[(size_t)row0 * O + k] : 0.0f;
+    if (tid < 2 * MG_MAX_LAYERS) sm.exps[tid] = pair_scale(pv.frag_fwd16_bf, pv.count)->cur[tid];
+    sp = {win, bin, ln, wh};
+    __syncthreads();
+    pair_forward<0>(pv, sp, sm, F, obsL, O, headL, HD);
+    for (int k = tid; k < M * HD; k += NT)
+        if (row0 + k / HD < rows) head[(size_t)row0 * HD + k] = headL[k];
 }
 
 // model/sample.metal:18-47 / model/gaussian.metal:42-71, one thread per row.
@@ -180,18 +220,27 @@ bool try_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs
                        dim3(dev::kLaneNT), lds, st, pv, obs, rows, head);
     return true;
 }
-// From 8192 rows in fp32 and 16384 in bf16 (64 and 128 workgroups): a
+// From 12288 rows in fp32 and 16384 in bf16 (96 and 128 workgroups): a
 // workgroup takes the time of its chain of stages however few there are, so
-// forward_kernel's 32-row tiles are as fast where they fit the GPU once. us a
-// call, forward_kernel against this, CartPole: fp32 57.5 / 58.2 at 4096 rows,
-// 60.5 / 59.6 at 8192, 97.6 / 61.9 at 16384, 544 / 189 at 100003; bf16 31.2 /
-// 33.8 at 8192, 38.1 / 34.4 at 16384, 162 / 82 at 100003.
+// smaller tiles are as fast where they fit the GPU once. us a call, CartPole:
+// fp32, forward_kernel / this, 97.6 / 61.9 at 16384 rows, 544 / 189 at 100003
+// (forward_pair_kernel below 12288); bf16 31.2 / 33.8 at 8192, 38.1 / 34.4 at
+// 16384, 162 / 82 at 100003.
 template <int PREC>
 bool launch_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
-    if (rows < (PREC == MG_PRECISION_BF16 ? 16384u : 8192u) || !pv.frag_fwd32_bf) return false;
+    if (rows < (PREC == MG_PRECISION_BF16 ? 16384u : 12288u) || !pv.frag_fwd32_bf) return false;
     return try_forward_lane<PREC, 4, 4>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 8, 32>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 16, 64>(st, pv, obs, rows, head);
+}
+// An fp32 forward of fewer rows, in the place of forward_kernel's 32-row tiles.
+bool launch_forward_pair(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
+    if (pv.precision != MG_PRECISION_FP32 || rows >= 12288u || !pv.frag_fwd16_bf) return false;
+    const size_t lds = (size_t)dev::forward_pair_floats(pv.obs_dim, pv.head_dim, pv.layers) * 4;
+    if (lds + sizeof(dev::PairFwdSmem) > 163840) return false;
+    hipLaunchKernelGGL(dev::forward_pair_kernel, dim3((rows + dev::kSplitRows - 1) / dev::kSplitRows),
+                       dim3(64 * dev::kPairW), lds, st, pv, obs, rows, head);
+    return true;
 }
 }  // namespace
 
@@ -200,7 +249,8 @@ int launch_forward(hipStream_t st, const mg_policy_view& pv, const float* obs, u
              "forward: OBS_DIM must be <= %d and ACT_DIM + 1 <= %d", dev::kMaxObs, dev::kMaxHead);
     if (rows == 0) return MG_OK;
     if (pv.precision == MG_PRECISION_BF16 ? launch_forward_lane<MG_PRECISION_BF16>(st, pv, obs, rows, head)
-                                          : launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head)) {
+                                          : launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head) ||
+                                                launch_forward_pair(st, pv, obs, rows, head)) {
     } else if (pv.precision == MG_PRECISION_BF16)
         hipLaunchKernelGGL((dev::forward_kernel<32, true>), dim3((rows + 31) / 32), dim3(256), 0, st, pv, obs, rows,
                            head);

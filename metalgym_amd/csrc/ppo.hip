@@ -18,6 +18,7 @@ struct mg_ppo {
     uint32_t n = 0, T = 0, B = 0, blocks = 0;
     mg_policy_view pv{};
     void* arenas = nullptr;  // params, their copies, m and v
+    void* slots = nullptr;   // the rollout slots and the advantage statistics
     float* m = nullptr;
     float* v = nullptr;
     uint32_t step = 0;
@@ -334,12 +335,22 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
     const size_t slot = T * n;
     int rc;
     if ((rc = check_matrix_layout(pv))) return fail(rc);
-    // the policy's arenas in one allocation, cleared by one memset
-    const size_t words = (size_t)pv.count * 4;
-    struct {
+    // the policy's arenas in one allocation and the rollout slots in another,
+    // each cleared by one memset
+    struct Part {
         void** at;
         size_t bytes;
-    } const arenas[] = {
+    };
+    auto carve = [](const Part* parts, size_t count, void* base) {
+        size_t at = 0;
+        for (size_t k = 0; k < count; ++k) {
+            if (base) *parts[k].at = static_cast<char*>(base) + at;
+            at += (parts[k].bytes + 255) / 256 * 256;
+        }
+        return at;
+    };
+    const size_t words = (size_t)pv.count * 4;
+    const Part arenas[] = {
         {(void**)&pv.params, words},
         {(void**)&pv.frag_fwd32, words},
         {(void**)&pv.frag_fwd16, words},
@@ -350,38 +361,30 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
         {(void**)&p->m, words},
         {(void**)&p->v, words},
     };
-    size_t arena_bytes = 0;
-    for (const auto& s : arenas) arena_bytes += (s.bytes + 255) / 256 * 256;
-    if ((rc = device_alloc(&p->arenas, arena_bytes, "PPOModel params and matrix tiles"))) return fail(rc);
-    arena_bytes = 0;
-    for (const auto& s : arenas) {
-        *s.at = static_cast<char*>(p->arenas) + arena_bytes;
-        arena_bytes += (s.bytes + 255) / 256 * 256;
-    }
-    if ((rc = device_alloc((void**)&p->obs_slots, (T + 1) * n * env->obs_dim * 4, "obs slots")) ||
-        (rc = device_alloc(&p->action_slots, slot * env->action_bytes, "action slots")) ||
-        (rc = device_alloc((void**)&p->logp, slot * 4, "logp slots")) ||
-        (rc = device_alloc((void**)&p->value, slot * 4, "value slots")) ||
-        (rc = device_alloc((void**)&p->reward, slot * 4, "reward slots")) ||
-        (rc = device_alloc((void**)&p->done_slots, slot, "done slots")) ||
-        (rc = device_alloc((void**)&p->adv, slot * 4, "advantage slots")) ||
-        (rc = device_alloc((void**)&p->ret, slot * 4, "return slots")) ||
-        (rc = device_alloc((void**)&p->adv_stats, (size_t)p->blocks * 2 * 4, "advantage stats")) ||
-        (rc = ensure_head(p, std::max(p->n, p->B))))
+    const Part slots[] = {
+        {(void**)&p->obs_slots, (T + 1) * n * env->obs_dim * 4},
+        {&p->action_slots, slot * env->action_bytes},
+        {(void**)&p->logp, slot * 4},
+        {(void**)&p->value, slot * 4},
+        {(void**)&p->reward, slot * 4},
+        {(void**)&p->done_slots, slot},
+        {(void**)&p->adv, slot * 4},
+        {(void**)&p->ret, slot * 4},
+        {(void**)&p->adv_stats, (size_t)p->blocks * 2 * 4},
+    };
+    constexpr size_t kArenas = sizeof(arenas) / sizeof(Part), kSlots = sizeof(slots) / sizeof(Part);
+    const size_t arena_bytes = carve(arenas, kArenas, nullptr), slot_bytes = carve(slots, kSlots, nullptr);
+    if ((rc = device_alloc(&p->arenas, arena_bytes, "PPOModel params and matrix tiles")) ||
+        (rc = device_alloc(&p->slots, slot_bytes, "rollout slots")) || (rc = ensure_head(p, std::max(p->n, p->B))))
         return fail(rc);
+    carve(arenas, kArenas, p->arenas);
+    carve(slots, kSlots, p->slots);
     std::vector<float> P;
     init_params(pv, c->seed, P);
     hipStream_t st = gym->stream;
     if (hipMemsetAsync(p->arenas, 0, arena_bytes, st) != hipSuccess ||
         hipMemcpyAsync(pv.params, P.data(), (size_t)pv.count * 4, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipMemsetAsync(p->obs_slots, 0, (T + 1) * n * env->obs_dim * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->action_slots, 0, slot * env->action_bytes, st) != hipSuccess ||
-        hipMemsetAsync(p->logp, 0, slot * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->value, 0, slot * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->reward, 0, slot * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->done_slots, 0, slot, st) != hipSuccess ||
-        hipMemsetAsync(p->adv, 0, slot * 4, st) != hipSuccess ||
-        hipMemsetAsync(p->ret, 0, slot * 4, st) != hipSuccess ||
+        hipMemsetAsync(p->slots, 0, slot_bytes, st) != hipSuccess ||
         hipMemsetAsync(p->head, 0, (size_t)p->head_cap * pv.head_dim * 4, st) != hipSuccess)
         return fail(set_error(MG_ERR_HIP, "PPOModel: initialisation upload failed"));
     if ((rc = launch_derive_blocks(st, pv))) return fail(rc);
@@ -398,16 +401,8 @@ int mg_ppo_destroy(mg_ppo* p) {
     if (!p) return MG_OK;
     if (p->gym && p->gym->stream) (void)hipStreamSynchronize(p->gym->stream);
     (void)hipFree(p->arenas);
-    (void)hipFree(p->obs_slots);
-    (void)hipFree(p->action_slots);
-    (void)hipFree(p->logp);
-    (void)hipFree(p->value);
-    (void)hipFree(p->reward);
-    (void)hipFree(p->done_slots);
-    (void)hipFree(p->adv);
-    (void)hipFree(p->ret);
+    (void)hipFree(p->slots);
     (void)hipFree(p->head);
-    (void)hipFree(p->adv_stats);
     (void)hipFree(p->ws_base);
     (void)hipFree(p->mb_stats);
     delete p;

@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(64 * W) train_rows_split_kernel(const RowsArgs
     // F16: this wave's groups of 32 units; else its strips of every chunk
     const int NK = F16 ? ((int)(H / kPairGroup) - wave + W - 1) / W : NC;
     const int rot = NK > 0 ? (wave + (int)(blockIdx.x >> 3)) % NK : 0;
-    using Seq = std::conditional_t<F16, PairSeq, SkSeq<S>>;
+    using Seq = std::conditional_t<F16, PairSeq<>, SkSeq<S>>;
     using Pos = std::conditional_t<F16, PairPos, SkPos>;
     Seq seq;
     if constexpr (F16)

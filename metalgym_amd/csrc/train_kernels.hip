@@ -1576,7 +1576,7 @@ bool rows_on_pairs(const mg_policy_view& pv) {
 int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv) {
     int rc = check_matrix_layout(pv);
     if (rc) return rc;
-    const bool bf = pv.precision == MG_PRECISION_BF16, pairs = rows_on_pairs(pv);
+    const bool bf = pv.precision == MG_PRECISION_BF16, pairs = !bf && pv.frag_fwd16_bf && pv.frag_bwd16_bf;
     uint16_t* split = bf ? nullptr : pv.frag_fwd32_bf;
     if (split) {
         hipLaunchKernelGGL(dev::split_scale_kernel, dim3(2 * pv.layers), dim3(1024), 0, st, pv.params, pv.float_group,

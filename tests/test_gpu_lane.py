@@ -1,4 +1,5 @@
-"""The row-per-lane-pair forward (policy_lane.h) at the edges of its range:
+"""The forwards on binary16 pairs (policy_lane.h, policy_pair.h) at the edges of
+their range:
 partial last workgroups, shapes at the ends, and weights whose size would leave
 binary16's range without the stored scales. Head values against a float64
 network, collect teacher-forced against the oracle."""
@@ -31,17 +32,28 @@ def network64(pv, P, obs):
 
 
 @pytest.mark.parametrize("env,rows,layers,scale,how", [
-    ("cartpole", 8192, 2, 4, "init"),         # the first row count of the path
-    ("cartpole", 8193, 2, 4, "init"),         # one row in the last workgroup
-    ("cartpole", 128 * 66 + 33, 1, 1, "init"),  # a wave and a row; the least hidden width
-    ("cartpole_continuous", 8200, 4, 8, "init"),
-    ("voxelnav16", 8320, 2, 4, "init"),
-    ("voxelnav", 8321, 8, 1, "init"),         # the deepest, 40 observation floats
-    ("cartpole", 8200, 2, 4, "large"),        # up x 2^40, down x 2^-40, gamma x 300
-    ("cartpole", 8200, 2, 4, "small"),        # up x 2^-30, gamma x 2^-12
-    ("cartpole", 8200, 2, 4, "outlier"),      # one weight 2^12 times the others
-    ("cartpole", 8200, 2, 4, "zero"),         # a block's matrices all zero
-    ("cartpole", 8200, 2, 4, "far"),          # observations of 1e6
+    ("cartpole", 12288, 2, 4, "init"),        # the first row count of the path
+    ("cartpole", 12289, 2, 4, "init"),         # one row in the last workgroup
+    ("cartpole", 128 * 97 + 33, 1, 1, "init"),  # a wave and a row; the least hidden width
+    ("cartpole_continuous", 12300, 4, 8, "init"),
+    ("voxelnav16", 12416, 2, 4, "init"),
+    ("voxelnav", 12417, 8, 1, "init"),         # the deepest, 40 observation floats
+    ("cartpole", 12300, 2, 4, "large"),        # up x 2^40, down x 2^-40, gamma x 300
+    ("cartpole", 12300, 2, 4, "small"),        # up x 2^-30, gamma x 2^-12
+    ("cartpole", 12300, 2, 4, "outlier"),      # one weight 2^12 times the others
+    ("cartpole", 12300, 2, 4, "zero"),         # a block's matrices all zero
+    ("cartpole", 12300, 2, 4, "far"),          # observations of 1e6
+    # 16-row tiles on pairs (policy_pair.h)
+    ("cartpole", 1, 2, 4, "init"),
+    ("cartpole", 12287, 2, 4, "init"),
+    ("voxelnav16", 17, 3, 3, "init"),          # groups of hidden units uneven over the waves
+    ("voxelnav", 1000, 8, 8, "init"),          # the largest policy
+    ("cartpole_continuous", 100, 1, 1, "init"),  # waves without a group
+    ("cartpole", 1000, 2, 4, "large"),
+    ("cartpole", 1000, 2, 4, "small"),
+    ("cartpole", 1000, 2, 4, "outlier"),
+    ("cartpole", 1000, 2, 4, "zero"),
+    ("cartpole", 1000, 2, 4, "far"),
 ])
 def test_forward_lane(mg, orc, env, rows, layers, scale, how):
     """As far from float64 as fp32 sums are on the same rows. The oracle adds a
@@ -84,8 +96,8 @@ def test_forward_lane(mg, orc, env, rows, layers, scale, how):
 
 
 @pytest.mark.parametrize("env,n,T,layers,scale,bf16", [
-    ("cartpole", 16384, 2, 2, 4, False),             # the first env count of the path
-    ("cartpole", 16384 + 64, 3, 2, 4, False),        # half a workgroup at the end
+    ("cartpole", 16384, 2, 2, 4, False),             # the last env count of the 16-row tiles on pairs
+    ("cartpole", 16384 + 64, 3, 2, 4, False),        # lane pairs: half a workgroup at the end
     ("cartpole_continuous", 16448, 2, 1, 8, False),
     ("cartpole_continuous_clamp", 16384, 2, 8, 1, False),
     ("voxelnav16", 16448, 2, 2, 4, False),
@@ -108,18 +120,21 @@ def test_collect_lane(mg, orc, env, n, T, layers, scale, bf16):
     run_collect_parity(Mg, orc, env, n, T, layers=layers, scale=scale, bf16=bf16)
 
 
-@pytest.mark.parametrize("env,T", [("cartpole", 96), ("voxelnav16", 32)])
-def test_collect_lane_takes_the_tiles_actions(mg, env, T):
-    """The first 8192 of 16384 envs (this path) and 8192 envs (32-row tiles) start
-    from the same seeds. Draws within rounding of a CDF edge are decided by the
-    tiles' arithmetic, so the rollouts must be the same step for step."""
+@pytest.mark.parametrize("env,n0,n1,T", [
+    ("voxelnav16", 8192, 16384, 32),   # 32-row tiles against lane pairs, both in the 32-row tiles' arithmetic
+    ("cartpole", 8192, 16448, 96),     # 16-row tiles on pairs against lane pairs, the same
+])
+def test_collects_take_the_same_actions(mg, env, n0, n1, T):
+    """The first n0 of n1 envs and n0 envs alone start from the same seeds. Draws
+    within rounding of a CDF edge are decided by the fp32 tiles' arithmetic in
+    every kernel, so the rollouts must be the same step for step."""
     runs = []
-    for n in (8192, 16384):
+    for n in (n0, n1):
         gym = mg.Gym(ENVS[env][1], n, 3)
-        model = mg.PPOModel(gym, horizon=T, seed=3)
+        model = mg.PPOModel(gym, horizon=T, seed=3, minibatch=64)
         model.collect()
         runs.append(model.download_slots())
     small, large = runs
     for key in ("actions", "obs", "reward", "done"):
-        assert np.array_equal(small[key], large[key][:, :8192]), f"{env} {key}"
-    np.testing.assert_allclose(large["logp"][:, :8192], small["logp"], rtol=0, atol=1e-5)
+        assert np.array_equal(small[key], large[key][:, :n0]), f"{env} {key}"
+    np.testing.assert_allclose(large["logp"][:, :n0], small["logp"], rtol=0, atol=1e-5)
