@@ -167,6 +167,13 @@ void launch_split_rollout(const mg_rollout_args* a, hipStream_t st) {
     launch_split_e<Env, MODE, E>(a, st);
 }
 
+// An env may bring a rollout kernel of its own (a specialisation with OK true,
+// seen before MG_DEFINE_ENV) that gives the same results as rollout_kernel.
+template <typename Env>
+struct PackedRollout {
+    static constexpr bool OK = false;
+};
+
 // Returns 0, a positive hipError_t on a launch failure, or MG_ERR_INVALID.
 template <typename Env>
 int launch_rollout(const mg_rollout_args* a) {
@@ -176,19 +183,21 @@ int launch_rollout(const mg_rollout_args* a) {
     // one lane per env: below 64 K envs one-wave workgroups spread the waves
     // over more CUs (4096 envs are 64 waves: 64 CUs instead of 16)
     hipStream_t st = static_cast<hipStream_t>(a->stream);
-    if constexpr (SplitRollout<Env>::OK) {
+    if constexpr (PackedRollout<Env>::OK) {
+        PackedRollout<Env>::launch(a, st);
+    } else if constexpr (SplitRollout<Env>::OK) {
         if (a->mode == MG_ACTIONS_RANDOM)
             launch_split_rollout<Env, MG_ACTIONS_RANDOM>(a, st);
         else
             launch_split_rollout<Env, MG_ACTIONS_GIVEN>(a, st);
-        return (int)hipGetLastError();
+    } else {
+        const uint32_t bs = a->n >= 65536u ? 256u : 64u;
+        dim3 block(bs), grid((a->n + bs - 1) / bs);
+        if (a->mode == MG_ACTIONS_RANDOM)
+            hipLaunchKernelGGL((rollout_kernel<Env, MG_ACTIONS_RANDOM>), grid, block, 0, st, *a);
+        else
+            hipLaunchKernelGGL((rollout_kernel<Env, MG_ACTIONS_GIVEN>), grid, block, 0, st, *a);
     }
-    const uint32_t bs = a->n >= 65536u ? 256u : 64u;
-    dim3 block(bs), grid((a->n + bs - 1) / bs);
-    if (a->mode == MG_ACTIONS_RANDOM)
-        hipLaunchKernelGGL((rollout_kernel<Env, MG_ACTIONS_RANDOM>), grid, block, 0, st, *a);
-    else
-        hipLaunchKernelGGL((rollout_kernel<Env, MG_ACTIONS_GIVEN>), grid, block, 0, st, *a);
     return (int)hipGetLastError();
 }
 
