@@ -306,12 +306,13 @@ __global__ void __launch_bounds__((CollectShape<M, Env::OBS_DIM, WIDE>::NT),
     }
 }
 
-// collect on the row-per-lane-pair forward (policy_lane.h): a workgroup of
-// kLaneTile envs on four waves, two workgroups per CU, lanes 0 .. 31 of a wave
-// its env lanes. Observations pass between the lanes of a wave, so
-// the only barriers are the weight ring's, and a wave's LN, head and env
-// phases run beside the other workgroup's products.
-template <typename Env, int PREC>
+// collect on the row-per-lane-pair forward (policy_lane.h): four waves, lanes
+// 0 .. 31 of a wave of share 0 its env lanes. With one share a workgroup has 128
+// envs and two of them a CU; observations pass between the lanes of a wave, so
+// the only barriers are the weight ring's, and a wave's LN, head and env phases
+// run beside the other workgroup's products. With two shares a workgroup has 64
+// envs and a CU to itself; share 1 gets the observations through LDS.
+template <typename Env, int PREC, int HS>
 struct CollectLane {
     using Tr = EnvTraits<Env>;
     static constexpr int O = Env::OBS_DIM, HD = Env::ACT_DIM + 1;
@@ -320,7 +321,7 @@ struct CollectLane {
     // of row n, which are its embed operands
     static constexpr uint32_t KS = Tr::STATE_IN_REGISTERS ? 0 : Tr::OBS_SPLIT;
     static constexpr int NOB = (O + 1) / 2;
-    static constexpr uint32_t WIN = O <= 16 ? O * kEmbed : 0;  // W_in in LDS
+    static constexpr uint32_t WIN = O <= 16 * HS ? O * kEmbed : 0;  // W_in in LDS
     // a wave's heads; an fp32 policy's categorical draws near an edge also need
     // a row's scratch (tile_row_head)
     static constexpr bool EDGE = PREC == MG_PRECISION_FP32 && !Tr::CONTINUOUS && Env::ACT_DIM > 1;
@@ -329,9 +330,11 @@ struct CollectLane {
     static constexpr bool OK = HD <= 16;  // the head's columns are registers
 };
 
-template <typename Env, int PREC>
-__global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_collect_args a) {
-    using CL = CollectLane<Env, PREC>;
+template <typename Env, int PREC, int HS>
+__global__ void __launch_bounds__(kLaneNT, LaneShape<HS>::WG) collect_lane_kernel(const mg_collect_args a) {
+    using CL = CollectLane<Env, PREC, HS>;
+    using Ring = LaneRing<PREC, HS>;
+    constexpr int RG = LaneShape<HS>::RG;
     using Tr = EnvTraits<Env>;
     using State = typename Env::State;
     using Action = typename Env::Action;
@@ -339,20 +342,22 @@ __global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_colle
     constexpr int O = CL::O, A = Env::ACT_DIM, HD = CL::HD, HC = CL::HC, NOB = CL::NOB;
     constexpr uint32_t KS = CL::KS;
     extern __shared__ __align__(16) float lane_lds_f[];
-    const LaneLds L = lane_lds<PREC, HC>(a.policy.layers, CL::WIN, CL::IO);
+    const LaneLds L = lane_lds<PREC, HC, HS>(a.policy.layers, CL::WIN, CL::IO);
     LaneParams<HC> P;
-    LaneRing<PREC> ring;
+    Ring ring;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = lane & 31, q = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave % RG, row = lane & 31, q = lane >> 5;
+    const bool lead = HS == 1 || wave < RG;  // share 0, which has the envs
     const uint32_t n = a.n, T = a.horizon;
-    const uint32_t i0 = blockIdx.x * kLaneTile + (uint32_t)(kLaneRows * wave);
+    const uint32_t i0 = blockIdx.x * LaneShape<HS>::TILE + (uint32_t)(kLaneRows * rg);
     // n is a multiple of 64, so a wave's rows are all there or none; a wave of
     // none still moves its share of the weights, on row 0's values
     const bool valid = i0 < n;
     const uint32_t i = valid ? i0 + (uint32_t)row : (uint32_t)row;
-    const bool envLane = valid && q == 0;
+    const bool envLane = valid && q == 0 && lead;
     const bool wide = n >= 64u * 512u;  // the tile height that launch_collect_tiles would take
-    float* ioL = lane_lds_f + L.io + wave * (int)CL::IO;
+    float* ioL = lane_lds_f + L.io + rg * (int)CL::IO;
     float* headL = ioL + row * HD;
     State* states = static_cast<State*>(a.state);
     Action* actSlots = static_cast<Action*>(a.action_slots);
@@ -424,7 +429,22 @@ __global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_colle
         done = a.done[i];
         if constexpr (Tr::STATE_IN_REGISTERS) sreg = states[i];
     }
-    if (a.first) {  // model/ppo.h:720-722: one step with action 0 into slot 0
+    // the observations to share 1
+    auto share = [&]() {
+        if constexpr (HS > 1) {
+            static_assert(NOB * 64 <= 2048 * LaneEx<PREC>::N, "a row group's observations fit");
+            float* at = reinterpret_cast<float*>(LaneEx<PREC>::at(ring, rg)) + lane;
+            if (lead)
+#pragma unroll
+                for (int u = 0; u < NOB; ++u) at[64 * u] = ob[u];
+            Ring::barrier();
+            if (!lead)
+#pragma unroll
+                for (int u = 0; u < NOB; ++u) ob[u] = at[64 * u];
+        }
+    };
+    if (!lead) {
+    } else if (a.first) {  // model/ppo.h:720-722: one step with action 0 into slot 0
         Action act{};
         float r = 0.0f;
         env_step(act, i, r);
@@ -439,6 +459,8 @@ __global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_colle
         }
     }
 
+    share();
+
     for (uint32_t t = 0; t <= T; ++t) {
         float hv[HC];
         lane_forward<PREC, HC, O, (CL::WIN > 0)>(a.policy, P, ring, O, ob, hv);
@@ -449,45 +471,48 @@ __global__ void __launch_bounds__(kLaneNT, 2) collect_lane_kernel(const mg_colle
             }
             break;
         }
-        const size_t k = (size_t)t * n + i;
-        Action act{};
-        float r = 0.0f, lp = 0.0f, edge = 1.0f;
-        const uint32_t rng0 = rng;
-        if (envLane) {
-#pragma unroll
-            for (int j = 0; j < HD; ++j) headL[j] = hv[j];  // the samplers index the row
-            if constexpr (Tr::CONTINUOUS)
-                sample_gaussian(headL, logStd, A, rng, reinterpret_cast<float*>(&act), lp);
-            else
-                act = (Action)sample_categorical(headL, A, rng, lp, CL::EDGE ? &edge : nullptr);
-        }
-        if constexpr (CL::EDGE) {
-            for (uint64_t near = __ballot(envLane && edge <= kLaneEdge); near; near &= near - 1) {
-                const int e = __builtin_ctzll(near);
-                const float* ep = a.obs_slots + ((size_t)t * n + i0 + (uint32_t)e) * O;
-                if (wide)
-                    tile_row_head<32, O, HD>(a.policy, ep, ioL + CL::ROW, ioL + e * HD);
+        if (lead) {
+            const size_t k = (size_t)t * n + i;
+            Action act{};
+            float r = 0.0f, lp = 0.0f, edge = 1.0f;
+            const uint32_t rng0 = rng;
+            if (envLane) {
+    #pragma unroll
+                for (int j = 0; j < HD; ++j) headL[j] = hv[j];  // the samplers index the row
+                if constexpr (Tr::CONTINUOUS)
+                    sample_gaussian(headL, logStd, A, rng, reinterpret_cast<float*>(&act), lp);
                 else
-                    tile_row_head<16, O, HD>(a.policy, ep, ioL + CL::ROW, ioL + e * HD);
-                if (lane == e) {
-                    const float mine = lp;
-                    uint32_t s = rng0;
-                    const Action own = act;
-                    act = (Action)sample_categorical(headL, A, s, lp);
-                    if (act == own) lp = mine;
+                    act = (Action)sample_categorical(headL, A, rng, lp, CL::EDGE ? &edge : nullptr);
+            }
+            if constexpr (CL::EDGE) {
+                for (uint64_t near = __ballot(envLane && edge <= kLaneEdge); near; near &= near - 1) {
+                    const int e = __builtin_ctzll(near);
+                    const float* ep = a.obs_slots + ((size_t)t * n + i0 + (uint32_t)e) * O;
+                    if (wide)
+                        tile_row_head<32, O, HD>(a.policy, ep, ioL + CL::ROW, ioL + e * HD);
+                    else
+                        tile_row_head<16, O, HD>(a.policy, ep, ioL + CL::ROW, ioL + e * HD);
+                    if (lane == e) {
+                        const float mine = lp;
+                        uint32_t s = rng0;
+                        const Action own = act;
+                        act = (Action)sample_categorical(headL, A, s, lp);
+                        if (act == own) lp = mine;
+                    }
                 }
             }
+            if (envLane) {
+                actSlots[k] = act;
+                a.logp_slots[k] = lp;
+                a.value_slots[k] = hv[A];
+            }
+            env_step(act, k + n, r);
+            if (envLane) {
+                a.reward_slots[k] = r;
+                a.done_slots[k] = done;
+            }
         }
-        if (envLane) {
-            actSlots[k] = act;
-            a.logp_slots[k] = lp;
-            a.value_slots[k] = hv[A];
-        }
-        env_step(act, k + n, r);
-        if (envLane) {
-            a.reward_slots[k] = r;
-            a.done_slots[k] = done;
-        }
+        share();
     }
     if (envLane) {
         if constexpr (Tr::STATE_IN_REGISTERS) states[i] = sreg;
@@ -645,18 +670,18 @@ __global__ void __launch_bounds__(64 * kPairW, 1) collect_pair_kernel(const mg_c
     }
 }
 
-// Runs the collect on collect_pair_kernel where that is the faster: under 16384
-// envs (up to four workgroups per CU, one after the other) of an env with at most
-// 16 observation floats and a register-held State. ms a collect of 32 steps,
+// Runs the collect on collect_pair_kernel where that is the faster: to 8192 envs
+// (two workgroups per CU, one after the other) of an env with at most 16
+// observation floats and a register-held State. ms a collect of 32 steps,
 // CartPole, split_forward16 or the 32-row tiles against this: 0.63 / 0.40 at 64
-// envs, 0.65 / 0.46 at 4096, 1.34 / 0.83 at 8192, 2.32 / 1.22 at 12288, 2.32 /
-// 1.73 at 16384 (collect_lane_kernel 1.71). A step takes 14 us at 4096 envs, of
+// envs, 0.65 / 0.46 at 4096, 1.34 / 0.83 at 8192 (collect_lane_kernel 1.06),
+// 2.32 / 1.22 at 12288 (1.10). A step takes 14 us at 4096 envs, of
 // which the weights' 1 MB through each CU's L1 is about 11.
 template <typename Env>
 bool launch_collect_pair(const mg_collect_args* a, hipStream_t st) {
     using CP = CollectPair<Env>;
     if constexpr (CP::OK) {
-        if (a->policy.precision != MG_PRECISION_FP32 || a->n >= 16384u || !a->policy.frag_fwd16_bf) return false;
+        if (a->policy.precision != MG_PRECISION_FP32 || a->n > 8192u || !a->policy.frag_fwd16_bf) return false;
         hipLaunchKernelGGL((collect_pair_kernel<Env>), dim3(a->n / kSplitRows), dim3(64 * kPairW),
                            CP::small(a->policy.layers) * 4, st, *a);
         return true;
@@ -710,27 +735,48 @@ void launch_collect_m(const mg_collect_args* a, hipStream_t st) {
     launch_collect_mw<Env, M, BF16, false>(a, st);
 }
 
-// Runs the collect on collect_lane_kernel where that is the faster: from 16384
-// envs in fp32 and 32768 in bf16 (128 and 256 workgroups), for heads of up to
-// 16 columns. ms a collect of 32 steps, the tiles below against this, CartPole:
-// fp32 2.32 / 1.81 at 16384 envs, 4.26 / 1.81 at 32768, 8.49 / 2.97 at 65536,
-// 33.6 / 11.3 at 262144 (1.15 PFLOP/s of binary16 products, what the library's
-// 8192^3 binary16 product reaches here); bf16 0.58 / 0.77 at 16384, 0.95 / 0.77
-// at 32768, 6.54 / 4.47 at 262144; VoxelNav16 262144: fp32 37.2 / 12.9, bf16
-// 9.35 / 5.96.
-template <typename Env, int PREC>
-bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
-    using CL = CollectLane<Env, PREC>;
+template <typename Env, int PREC, int HS>
+bool launch_collect_lane_as(const mg_collect_args* a, hipStream_t st) {
+    using CL = CollectLane<Env, PREC, HS>;
+    using Sh = LaneShape<HS>;
     if constexpr (CL::OK) {
-        if (a->n < (PREC == MG_PRECISION_BF16 ? 32768u : 16384u) || !a->policy.frag_fwd32_bf) return false;
-        const size_t lds = (size_t)lane_lds<PREC, CL::HC>(a->policy.layers, CL::WIN, CL::IO).total * 4;
-        if (lds > 163840 / 2) return false;
-        hipLaunchKernelGGL((collect_lane_kernel<Env, PREC>), dim3((a->n + kLaneTile - 1) / kLaneTile), dim3(kLaneNT),
+        const size_t lds = (size_t)lane_lds<PREC, CL::HC, HS>(a->policy.layers, CL::WIN, CL::IO).total * 4;
+        if (!a->policy.frag_fwd32_bf || lds > 163840 / Sh::WG) return false;
+        hipLaunchKernelGGL((collect_lane_kernel<Env, PREC, HS>), dim3((a->n + Sh::TILE - 1) / Sh::TILE), dim3(kLaneNT),
                            lds, st, *a);
         return true;
     } else {
         return false;
     }
+}
+
+// Runs the collect on collect_lane_kernel where that is the faster, for heads of
+// up to 16 columns. With 128 envs a workgroup (one share) a step takes the time
+// of one workgroup's stages up to 32768 envs, one per CU, and 1.15 PFLOP/s of
+// binary16 products from 65536 (what the library's 8192^3 binary16 product
+// reaches here); at 16384 half the CUs have none, so there two shares take 64
+// envs a workgroup. ms a collect of 32 steps, CartPole, fp32, the tiles below (to
+// 8192 envs the 16-row tiles on pairs) / two shares / one: 0.87 / 1.06 / 1.32 at
+// 8192 envs, 1.22 / 1.10 / 1.37 at 12288, 2.30 / 1.14 / 1.38 at 16384, 3.26 /
+// 2.08 / 1.43 at 24576, 8.44 / 4.18 / 2.86 at 65536. VoxelNav16, 16 steps: 0.83 /
+// 0.75 / 0.98 at 8192, 1.34 / 0.80 / 1.02 at 16384. bf16, 0.56 / 0.62 / 0.62 at
+// 16384, 0.71 / 1.20 / 0.63 at 20480, 0.87 / 1.21 / 0.68 at 32768: one share only.
+// An env of more than 32 observation floats spends its step on computing them
+// (VoxelNav's 32 ray marches), which the tiles spread over more threads, until
+// the grid is full: 16 steps, tiles / one share, fp32 2.37 / 3.16 at 16384 and 4.09 / 3.32 at 32768;
+// bf16 2.34 / 2.93 at 32768, and 8 steps of 65536 2.48 / 1.92.
+template <typename Env, int PREC>
+bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
+    constexpr bool F32 = PREC == MG_PRECISION_FP32;
+    if constexpr (Env::OBS_DIM > 32) {
+        if (a->n < (F32 ? 32768u : 65536u)) return false;
+    }
+    if (a->n > 16384u) return launch_collect_lane_as<Env, PREC, 1>(a, st);
+    if constexpr (F32) {
+        if (a->n >= 8192u && launch_collect_lane_as<Env, PREC, 2>(a, st)) return true;
+        if (a->n == 16384u) return launch_collect_lane_as<Env, PREC, 1>(a, st);
+    }
+    return false;
 }
 
 template <typename Env, bool BF16>

@@ -10,7 +10,17 @@
 // lane. What the waves share is the weights: a stage of one 32-unit hidden
 // tile (its Up^T strip and its Down^T columns) is staged in LDS once per
 // workgroup of 128 rows, double-buffered, with one barrier per stage, the
-// stage after next already in flight in registers.
+// stage after next already in flight in registers. A stage is bound by the
+// matrix instructions (48 of 32 cycles in fp32) where a SIMD has two waves; with
+// one, everything a wave does between them counts, so each operand is read one
+// step ahead of its product and the next stage's LDS writes and loads are spread
+// over the first eight: 1.47 -> 1.12 us a stage at one wave per SIMD (16384
+// rows), a step of 65536 envs 93 -> 86 us.
+//
+// Where 128 rows a workgroup leave CUs idle the four waves are two row groups of
+// two waves each (shares): a wave does half of the hidden units of its 32 rows,
+// the two sums meet in LDS after a block (LaneEx), and LN, embed and head are
+// done by both. A step of 16384 envs (hidden 512, 2 blocks) 42 -> 34 us.
 //
 // Precision MG_PRECISION_FP32: each fp32 operand as two binary16 halves, x =
 // hi + lo (22 bits and the sign of lo), and hi hi + hi lo + lo hi accumulated
@@ -42,10 +52,18 @@ namespace dev {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kLaneRows = 32;   // rows of a wave
-constexpr int kLaneWaves = 4;   // waves of a workgroup
+constexpr int kLaneRows = 32;  // rows of a wave
+
+constexpr int kLaneWaves = 4;  // waves of a workgroup
 constexpr int kLaneNT = 64 * kLaneWaves;
-constexpr int kLaneTile = kLaneRows * kLaneWaves;  // rows of a workgroup
+// HS waves share the hidden units of 32 rows: wave h RG + g is share h of row
+// group g of RG = 4 / HS.
+template <int HS>
+struct LaneShape {
+    static constexpr int RG = kLaneWaves / HS, TILE = kLaneRows * RG;
+    static constexpr int WG = HS == 1 ? 2 : 1;  // workgroups per CU: the ring is 64 HS KB
+};
+constexpr int kLaneTile = LaneShape<1>::TILE;
 
 // The binary16 planes of an fp32 policy (mg_policy_view.frag_fwd32_bf with
 // MG_PRECISION_FP32): up^T and down^T in the order of the bf16 copies, each
@@ -171,62 +189,75 @@ struct LaneOps<MG_PRECISION_BF16> {
 // it is row 16 b + 8 q + j of the matrix, the K order of the weight copies.
 __device__ __forceinline__ int lane_pi(int m) { return (m & 0x13) | ((m & 4) << 1) | ((m & 8) >> 1); }
 
-// The weights of one forward as a cycle of stages (layer l, hidden tile ht)
-// through two LDS buffers of 32 (fp32) or 16 KB (bf16).
-template <int PREC>
+// The weights of one forward as a cycle of stages (layer l, hidden tile ht of
+// each share) through two LDS buffers of 32 (fp32) or 16 KB (bf16) per share.
+template <int PREC, int HS>
 struct LaneRing {
     using Ops = LaneOps<PREC>;
     static constexpr int PL = Ops::PL;
-    static constexpr int F4 = 1024 * PL;          // float4s of a stage
-    static constexpr int NL = F4 / kLaneNT;       // loads per thread
+    static constexpr int T4 = 1024 * PL;   // float4s of a hidden tile
+    static constexpr int F4 = T4 * HS;     // of a stage
+    static constexpr int NL = F4 / kLaneNT;  // loads per thread
     const uint16_t* planes;
     f32x4* buf;  // LDS, 2 F4
     uint32_t count, group, EH, H;
-    int tiles, layers;  // hidden tiles per layer
+    int tiles, layers;  // hidden tiles per layer and share
     int nl, nt;         // the stage in flight
     f32x4 st[NL];
 
-    // Stage (nl, nt) from memory into st: up^T's strip of 32 hidden units (8
-    // KB a plane, contiguous) and the two k-groups of down^T's four strips (2
-    // KB each).
-    __device__ __forceinline__ void load() {
-        const int tid = threadIdx.x;
-        const uint32_t up = group + 2u * (uint32_t)nl * EH + 4096u * (uint32_t)nt;
-        const uint32_t dn = group + (2u * (uint32_t)nl + 1u) * EH + 1024u * (uint32_t)nt;
-        const uint32_t vd = (uint32_t)(tid >> 7) * 64u * H + 16u * (uint32_t)(tid & 127);
-#pragma unroll
-        for (int p = 0; p < PL; ++p)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                st[2 * p + u] = buffer_load16(planes, 16u * tid, 2u * (up + p * count + 2048u * u));
-                st[2 * PL + 2 * p + u] = buffer_load16(planes, vd, 2u * (dn + p * count + 64u * u * H));
-            }
+    // Load k of stage (nl, nt) into st[k]: of each share's tile (h tiles + nt)
+    // up^T's strip of 32 hidden units (8 KB a plane, contiguous) and the two
+    // k-groups of down^T's four strips (2 KB each).
+    __device__ __forceinline__ void load(int k) {
+        const int tid = threadIdx.x, h = k / (4 * PL), r = k % (4 * PL), p = r / 2 % PL, u = r % 2;
+        const uint32_t t = (uint32_t)(nt + h * tiles);
+        const uint32_t up = group + 2u * (uint32_t)nl * EH + 4096u * t;
+        const uint32_t dn = group + (2u * (uint32_t)nl + 1u) * EH + 1024u * t;
+        if (r < 2 * PL) {
+            st[k] = buffer_load16(planes, 16u * tid, 2u * (up + p * count + 2048u * u));
+        } else {
+            const uint32_t vd = (uint32_t)(tid >> 7) * 64u * H + 16u * (uint32_t)(tid & 127);
+            st[k] = buffer_load16(planes, vd, 2u * (dn + p * count + 64u * u * H));
+        }
+    }
+    __device__ __forceinline__ void store(int b, int k) { buf[b * F4 + kLaneNT * k + threadIdx.x] = st[k]; }
+    __device__ __forceinline__ void next() {
         if (++nt == tiles) {
             nt = 0;
             if (++nl == layers) nl = 0;
         }
-    }
-    __device__ __forceinline__ void store(int b) {
-#pragma unroll
-        for (int u = 0; u < NL; ++u) buf[b * F4 + u * kLaneNT + threadIdx.x] = st[u];
     }
     // Stage 0 in buffer 0 and stage 1 in flight; the caller's next barrier
     // makes buffer 0 readable.
     __device__ __forceinline__ void start(const mg_policy_view& pv, f32x4* lds) {
         planes = pv.frag_fwd32_bf, buf = lds;
         count = pv.count, group = pv.float_group, H = pv.hidden, EH = (uint32_t)kEmbed * H;
-        tiles = (int)H / 32, layers = (int)pv.layers;
+        tiles = (int)H / (32 * HS), layers = (int)pv.layers;
         nl = nt = 0;
-        load();
-        store(0);
-        load();
+#pragma unroll
+        for (int k = 0; k < NL; ++k) load(k);
+        next();
+#pragma unroll
+        for (int k = 0; k < NL; ++k) store(0, k);
+#pragma unroll
+        for (int k = 0; k < NL; ++k) load(k);
+        next();
     }
-    // After the reads of buffer b: the stage in flight goes to the other
-    // buffer, which every wave finished reading before the last barrier, and
-    // the next one leaves.
-    __device__ __forceinline__ void advance(int b) {
-        store(b ^ 1);
-        load();
+    // Beside the products of buffer b's stage, part i of 8: the stage in flight
+    // goes to the other buffer, which every wave finished reading before the
+    // last barrier, and the one after it leaves; then finish().
+    __device__ __forceinline__ void pass(int b, int i) {
+#pragma unroll
+        for (int k = i; k < NL; k += 8) {
+            store(b ^ 1, k);
+            load(k);
+        }
+    }
+    __device__ __forceinline__ void finish() {
+        next();
+        barrier();
+    }
+    __device__ static __forceinline__ void barrier() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -310,19 +341,61 @@ __device__ __forceinline__ void lane_read8(const float* p, float (&v)[8]) {
     for (int j = 0; j < 4; ++j) v[j] = a[j], v[4 + j] = b[j];
 }
 
+// What passes between the two shares of a row group, in ring buffer 1, which is
+// free from the last stage of a block to the first of the next: N of a wave's
+// tiles a time, 4 KB each.
+template <int PREC>
+struct LaneEx {
+    using Ring = LaneRing<PREC, 2>;
+    static constexpr int N = PREC == MG_PRECISION_FP32 ? 4 : 2;
+    static_assert(LaneShape<2>::RG * 2 * 256 * N <= Ring::F4, "fits the buffer");
+    __device__ static __forceinline__ f32x4* at(const Ring& ring, int rg) { return ring.buf + Ring::F4 + 512 * N * rg; }
+    // The two shares' sums, in both. Starts and ends where every wave has
+    // finished with the memory.
+    __device__ static __forceinline__ void join(LaneRows& R, f32x4* ex, int half, int lane) {
+        f32x4 *mine = ex + 256 * N * half + lane, *other = ex + 256 * N * (half ^ 1) + lane;
+#pragma unroll
+        for (int m0 = 0; m0 < 4; m0 += N) {
+#pragma unroll
+            for (int m = 0; m < N; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const f32x16 h = R.h[m0 + m];
+                    mine[64 * (4 * m + r)] = f32x4{h[4 * r], h[4 * r + 1], h[4 * r + 2], h[4 * r + 3]};
+                }
+            Ring::barrier();
+#pragma unroll
+            for (int m = 0; m < N; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const f32x4 v = other[64 * (4 * m + r)];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) R.h[m0 + m][4 * r + j] += v[j];
+                    if (r == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+            Ring::barrier();
+        }
+    }
+};
+
 // model/ppo.h:575-626 for the wave's 32 rows. ob[s]: this lane's embed
-// operand, observation float 2 s + q of row n (0 past the last). The head (HC columns, both lanes of a row) goes to hv.
+// operand, observation float 2 s + q of row n (0 past the last). The head (HC
+// columns, both lanes of a row) goes to hv, of share 0 where there are two.
 // O <= OC: the observation width (OC itself where it is known at compile
 // time); WINL: W_in is in LDS.
-template <int PREC, int HC, int OC, bool WINL>
-__device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const LaneParams<HC>& P, LaneRing<PREC>& ring,
-                                             int O, const float (&ob)[(OC + 1) / 2], float (&hv)[HC]) {
+template <int PREC, int HC, int OC, bool WINL, int HS>
+__device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const LaneParams<HC>& P,
+                                             LaneRing<PREC, HS>& ring, int O, const float (&ob)[(OC + 1) / 2],
+                                             float (&hv)[HC]) {
+    using Ring = LaneRing<PREC, HS>;
     constexpr int NOB = (OC + 1) / 2;
     using Ops = LaneOps<PREC>;
     using V = typename Ops::V;
     constexpr int PL = Ops::PL;
     const int lane = threadIdx.x & 63, q = lane >> 5;
-    const int slot = lane_pi(lane & 31) + 32 * q;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int half = HS > 1 ? wave / LaneShape<HS>::RG : 0;
+    const int slot = lane_pi(lane & 31) + 32 * q + half * Ring::T4;
     LaneRows R;
     // model/input.metal:11-27 on v_mfma_f32_32x32x2_f32
 #pragma unroll
@@ -354,6 +427,7 @@ __device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const Lan
         // at most 16 weights in flight: all 60 of VoxelNav16's spill
         if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (HS > 1) Ring::barrier();  // the observations' LDS is read
     float inv = 1.0f;
     for (uint32_t l = 0; l < pv.layers; ++l) {
         float mean, rstd;
@@ -372,23 +446,36 @@ __device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const Lan
         }
         if constexpr (PREC == MG_PRECISION_FP32) {
             // the stream to this block's units
-            const float f = P.scale[2 * l] * inv;
+            // (in share 0's sum)
+            const float f = half ? 0.0f : P.scale[2 * l] * inv;
             inv = P.scale[2 * l + 1];
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) R.h[mt][r] *= f;
+        } else if constexpr (HS > 1) {
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) R.h[mt][r] = half ? 0.0f : R.h[mt][r];
         }
         for (int ht = 0; ht < ring.tiles; ++ht) {  // tiles is even: hidden is a multiple of 128
-            const f32x4* w = ring.buf + (ht & 1) * LaneRing<PREC>::F4 + slot;
+            const f32x4* w = ring.buf + (ht & 1) * Ring::F4 + slot;
             // model/mlp.metal:18-86: V^T = relu(Up^T x^T) for 32 units, then h^T += Down^T V^T
             f32x16 v = f32x16{};
+            V a[2][PL];
+            auto fetch = [&](int i) {  // operand i of 8 + 8
+                const int at = i < 8 ? 64 * i : 512 * PL + 128 * (i & 3) + 64 * ((i - 8) >> 2);
+#pragma unroll
+                for (int p = 0; p < PL; ++p) a[i & 1][p] = __builtin_bit_cast(V, w[512 * p + at]);
+            };
+            fetch(0);
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                V a[PL];
-#pragma unroll
-                for (int p = 0; p < PL; ++p) a[p] = __builtin_bit_cast(V, w[512 * p + 64 * s]);
-                v = Ops::mma(a, xb[s], v);
+                fetch(s + 1);
+                v = Ops::mma(a[s & 1], xb[s], v);
+                ring.pass(ht & 1, s);
+                __builtin_amdgcn_sched_barrier(0);  // or the loads, and their waits, are moved together
             }
             V vb[2][PL];
 #pragma unroll
@@ -398,17 +485,15 @@ __device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const Lan
                 for (int j = 0; j < 8; ++j) t[j] = v[8 * b + j];
                 Ops::pack_hidden(t, vb[b]);
             }
-            w += 512 * PL;
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt) {
-                    V a[PL];
-#pragma unroll
-                    for (int p = 0; p < PL; ++p) a[p] = __builtin_bit_cast(V, w[512 * p + 128 * mt + 64 * b]);
-                    R.h[mt] = Ops::mma(a, vb[b], R.h[mt]);
-                }
-            ring.advance(ht & 1);
+            for (int i = 0; i < 8; ++i) {
+                if (i < 7) fetch(i + 9);
+                R.h[i & 3] = Ops::mma(a[i & 1], vb[i >> 2], R.h[i & 3]);
+            }
+            ring.finish();
+        }
+        if constexpr (HS > 1) {
+            LaneEx<PREC>::join(R, LaneEx<PREC>::at(ring, wave % LaneShape<HS>::RG), half, lane);
         }
     }
     float mean, rstd;
@@ -560,20 +645,20 @@ __device__ __forceinline__ void tile_row_head(const mg_policy_view& pv, const fl
 }
 
 // A workgroup's LDS, in floats: the ring, the small parameters (W_in where
-// win), then io floats per wave.
+// win), then io floats per row group.
 struct LaneLds {
     uint32_t ln, bin, scale, wh, win, io, total;
 };
-template <int PREC, int HC>
+template <int PREC, int HC, int HS>
 __host__ __device__ __forceinline__ LaneLds lane_lds(uint32_t layers, uint32_t win, uint32_t io_per_wave) {
     LaneLds L;
-    uint32_t o = 2u * LaneRing<PREC>::F4 * 4u;
+    uint32_t o = 2u * LaneRing<PREC, HS>::F4 * 4u;
     L.ln = o, o += (layers + 1) * 2 * kEmbed;
     L.bin = o, o += kEmbed;
     L.scale = o, o += 2 * MG_MAX_LAYERS;
     L.wh = o, o += kEmbed * HC;
     L.win = o, o += win;
-    L.io = o, o += kLaneWaves * ((io_per_wave + 3u) & ~3u);
+    L.io = o, o += LaneShape<HS>::RG * ((io_per_wave + 3u) & ~3u);
     L.total = o;
     return L;
 }
@@ -581,9 +666,9 @@ __host__ __device__ __forceinline__ LaneLds lane_lds(uint32_t layers, uint32_t w
 // Stages the small parameters (the blocks' gamma and beta scaled) and starts
 // the ring. Ends with a barrier. win: floats of W_in to stage (0: read from
 // the arena).
-template <int PREC, int HC>
+template <int PREC, int HC, int HS>
 __device__ __forceinline__ void lane_start(const mg_policy_view& pv, float* lds, const LaneLds& L, uint32_t win,
-                                           LaneParams<HC>& P, LaneRing<PREC>& ring) {
+                                           LaneParams<HC>& P, LaneRing<PREC, HS>& ring) {
     const int tid = threadIdx.x;
     ring.start(pv, reinterpret_cast<f32x4*>(lds));
     const float* lnp = pv.params + pv.off_ln_gamma[0];

@@ -46,9 +46,9 @@ __global__ void __launch_bounds__(kLaneNT, 2) forward_lane_kernel(const mg_polic
                                                                   const float* __restrict__ obs, uint32_t rows,
                                                                   float* __restrict__ head) {
     extern __shared__ __align__(16) float lane_lds_f[];
-    const LaneLds L = lane_lds<PREC, HC>(pv.layers, 0, 0);
+    const LaneLds L = lane_lds<PREC, HC, 1>(pv.layers, 0, 0);
     LaneParams<HC> P;
-    LaneRing<PREC> ring;
+    LaneRing<PREC, 1> ring;
     const int O = (int)pv.obs_dim, HD = (int)pv.head_dim;
     const int lane = threadIdx.x & 63, q = lane >> 5;
     const uint32_t r = blockIdx.x * kLaneTile + (uint32_t)(kLaneRows * (threadIdx.x >> 6) + (lane & 31));
@@ -214,28 +214,27 @@ namespace {
 template <int PREC, int HC, int OC>
 bool try_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
     if (pv.head_dim > (uint32_t)HC || pv.obs_dim > (uint32_t)OC) return false;
-    const size_t lds = (size_t)dev::lane_lds<PREC, HC>(pv.layers, 0, 0).total * 4;
+    const size_t lds = (size_t)dev::lane_lds<PREC, HC, 1>(pv.layers, 0, 0).total * 4;
     if (lds > 163840 / 2) return false;
     hipLaunchKernelGGL((dev::forward_lane_kernel<PREC, HC, OC>), dim3((rows + dev::kLaneTile - 1) / dev::kLaneTile),
                        dim3(dev::kLaneNT), lds, st, pv, obs, rows, head);
     return true;
 }
-// From 12288 rows in fp32 and 16384 in bf16 (96 and 128 workgroups): a
-// workgroup takes the time of its chain of stages however few there are, so
-// smaller tiles are as fast where they fit the GPU once. us a call, CartPole:
-// fp32, forward_kernel / this, 97.6 / 61.9 at 16384 rows, 544 / 189 at 100003
-// (forward_pair_kernel below 12288); bf16 31.2 / 33.8 at 8192, 38.1 / 34.4 at
-// 16384, 162 / 82 at 100003.
+// Over 8192 rows (65 workgroups): a workgroup takes the time of its chain of
+// stages however few there are, so smaller tiles are as fast where they fit the
+// GPU once. us a call, CartPole: fp32, forward_kernel / this, 92 / 56 at 8193
+// rows, 98 / 56 at 16384, 544 / 176 at 100003 (forward_pair_kernel 44 at 8192);
+// bf16 29.8 at 8192, 35.9 / 32 at 8193, 38 / 32 at 16384, 162 / 77 at 100003.
 template <int PREC>
 bool launch_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
-    if (rows < (PREC == MG_PRECISION_BF16 ? 16384u : 12288u) || !pv.frag_fwd32_bf) return false;
+    if (rows <= 8192u || !pv.frag_fwd32_bf) return false;
     return try_forward_lane<PREC, 4, 4>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 8, 32>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 16, 64>(st, pv, obs, rows, head);
 }
 // An fp32 forward of fewer rows, in the place of forward_kernel's 32-row tiles.
 bool launch_forward_pair(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
-    if (pv.precision != MG_PRECISION_FP32 || rows >= 12288u || !pv.frag_fwd16_bf) return false;
+    if (pv.precision != MG_PRECISION_FP32 || !pv.frag_fwd16_bf) return false;
     const size_t lds = (size_t)dev::forward_pair_floats(pv.obs_dim, pv.head_dim, pv.layers) * 4;
     if (lds + sizeof(dev::PairFwdSmem) > 163840) return false;
     hipLaunchKernelGGL(dev::forward_pair_kernel, dim3((rows + dev::kSplitRows - 1) / dev::kSplitRows),

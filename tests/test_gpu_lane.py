@@ -32,8 +32,8 @@ def network64(pv, P, obs):
 
 
 @pytest.mark.parametrize("env,rows,layers,scale,how", [
-    ("cartpole", 12288, 2, 4, "init"),        # the first row count of the path
-    ("cartpole", 12289, 2, 4, "init"),         # one row in the last workgroup
+    ("cartpole", 8193, 2, 4, "init"),          # the first row count of the path: one row in the last workgroup
+    ("cartpole", 12288, 2, 4, "init"),
     ("cartpole", 128 * 97 + 33, 1, 1, "init"),  # a wave and a row; the least hidden width
     ("cartpole_continuous", 12300, 4, 8, "init"),
     ("voxelnav16", 12416, 2, 4, "init"),
@@ -45,7 +45,7 @@ def network64(pv, P, obs):
     ("cartpole", 12300, 2, 4, "far"),          # observations of 1e6
     # 16-row tiles on pairs (policy_pair.h)
     ("cartpole", 1, 2, 4, "init"),
-    ("cartpole", 12287, 2, 4, "init"),
+    ("cartpole", 8192, 2, 4, "init"),
     ("voxelnav16", 17, 3, 3, "init"),          # groups of hidden units uneven over the waves
     ("voxelnav", 1000, 8, 8, "init"),          # the largest policy
     ("cartpole_continuous", 100, 1, 1, "init"),  # waves without a group
@@ -96,13 +96,17 @@ def test_forward_lane(mg, orc, env, rows, layers, scale, how):
 
 
 @pytest.mark.parametrize("env,n,T,layers,scale,bf16", [
-    ("cartpole", 16384, 2, 2, 4, False),             # the last env count of the 16-row tiles on pairs
-    ("cartpole", 16384 + 64, 3, 2, 4, False),        # lane pairs: half a workgroup at the end
+    ("cartpole", 8192, 2, 2, 4, False),              # the last env count of the 16-row tiles on pairs
+    ("cartpole", 8192 + 64, 3, 2, 4, False),         # two shares of the hidden units
+    ("cartpole", 16384, 2, 2, 4, False),
+    ("cartpole_continuous", 10240, 2, 1, 1, False),  # two stages per share, one block
+    ("voxelnav16", 8192, 2, 8, 1, False),            # the deepest: W_in's place in LDS
+    ("cartpole", 16384 + 64, 3, 2, 4, False),        # one share: half a workgroup at the end
     ("cartpole_continuous", 16448, 2, 1, 8, False),
     ("cartpole_continuous_clamp", 16384, 2, 8, 1, False),
     ("voxelnav16", 16448, 2, 2, 4, False),
-    ("voxelnav", 16448, 2, 2, 4, False),
-    ("cartpole", 32832, 2, 2, 4, True),
+    ("voxelnav", 32832, 2, 2, 4, False),
+    ("cartpole", 16448, 2, 2, 4, True),
     ("voxelnav16", 32832, 2, 1, 2, True),
 ])
 def test_collect_lane(mg, orc, env, n, T, layers, scale, bf16):
@@ -121,8 +125,9 @@ def test_collect_lane(mg, orc, env, n, T, layers, scale, bf16):
 
 
 @pytest.mark.parametrize("env,n0,n1,T", [
-    ("voxelnav16", 8192, 16384, 32),   # 32-row tiles against lane pairs, both in the 32-row tiles' arithmetic
-    ("cartpole", 8192, 16448, 96),     # 16-row tiles on pairs against lane pairs, the same
+    ("voxelnav16", 8192, 16448, 32),   # two shares against one, both in the 32-row tiles' arithmetic
+    ("cartpole", 8192, 16384, 96),     # 16-row tiles on pairs against two shares, the same
+    ("cartpole", 12288, 16448, 96),    # two shares against one
 ])
 def test_collects_take_the_same_actions(mg, env, n0, n1, T):
     """The first n0 of n1 envs and n0 envs alone start from the same seeds. Draws
