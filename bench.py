@@ -18,7 +18,8 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-PEAK_FP32_MFMA = 157.3e12  # FLOP/s, MI355X dense fp32 matrix
+# FLOP/s of an fp32 product as three binary16 products (MI355X dense binary16 matrix: 2.5e15)
+PEAK_PAIR_MFMA = 2.5e15 / 3
 PEAK_HBM = 8.0e12          # B/s
 E, H, L = 128, 512, 2
 
@@ -509,8 +510,8 @@ def main():
         "data": "synthetic (seeded envs and weights)",
         "config": {"workload": "cartpole_collect_with_policy", "envs": n, "horizon": T, "embed": E, "hidden": H,
                    "layers": L, "head": "softmax(2)+value", "parallelism": "single-gpu"},
-        "roofline": {"bound": "mfma", "kernel": "collect_kernel<CartPole,64,false,false>", "achieved": achieved / 1e12,
-                     "peak": PEAK_FP32_MFMA / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_MFMA,
+        "roofline": {"bound": "mfma", "kernel": "collect_lane_kernel<CartPole,0,1>", "achieved": achieved / 1e12,
+                     "peak": PEAK_PAIR_MFMA / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_PAIR_MFMA,
                      "traffic": pmc_traffic(),
                      "traffic_source": "profiles/collect_cartpole_262144_pmc.json: rocprofv3 --pmc FETCH_SIZE and "
                                        "WRITE_SIZE of this kernel (a committed profile, not measured in this run)",
@@ -538,13 +539,13 @@ def main():
         _, _, dtc, tc = bench_collect("rollout_cartpole_continuous", 262144, 32, 3, 1, 4, 1)
         kc = kernel_avg_ms(tc, "collect")
         extra["continuous_collect_262144"] = {"env_steps_per_s": 3 * 262144 * 32 / dtc, "collect_ms": kc,
-                                              "mfma_frac": 33 * 262144 * fwd_flop(4, 1) / (kc * 1e-3) / PEAK_FP32_MFMA}
+                                              "mfma_frac": 33 * 262144 * fwd_flop(4, 1) / (kc * 1e-3) / PEAK_PAIR_MFMA}
         extra["continuous_full_ppo_65536"] = bench_full("rollout_cartpole_continuous", 65536, 32, 2, 4, 1)
         extra["continuous_full_ppo_262144"] = bench_full("rollout_cartpole_continuous", 262144, 32, 1, 4, 1)
         _, _, dtv, tv = bench_collect("rollout_voxelnav16", 262144, 32, 3, 1, 30, 6)
         kv = kernel_avg_ms(tv, "collect")
         extra["voxelnav16_collect_262144"] = {"env_steps_per_s": 3 * 262144 * 32 / dtv, "collect_ms": kv,
-                                              "mfma_frac": 33 * 262144 * fwd_flop(30, 6) / (kv * 1e-3) / PEAK_FP32_MFMA}
+                                              "mfma_frac": 33 * 262144 * fwd_flop(30, 6) / (kv * 1e-3) / PEAK_PAIR_MFMA}
         extra["voxelnav16_random_262144"] = bench_random(262144, 32, 10, "rollout_voxelnav16")
         extra["voxelnav16_full_ppo_262144"] = bench_full("rollout_voxelnav16", 262144, 32, 1, 30, 6)
         # the reference's heightmap VoxelNav at its README configuration (4096 envs,

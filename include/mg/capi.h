@@ -109,15 +109,19 @@ typedef struct mg_rollout_args {
  * MG_PRECISION_BF16, frag_fwd32_bf and frag_fwd16_bf hold up^T and down^T and
  * frag_bwd16_bf up and down, rounded to bfloat16 (16-bit patterns), in the
  * operand order of the bf16 instructions (32x32x16 and 16x16x32: k-groups of
- * 16 and 32, each lane 8 consecutive k). With MG_PRECISION_FP32 frag_fwd32_bf, where it is not
- * NULL, holds up^T and down^T in that order as pairs of binary16 values, each element times a power of two of
- * its matrix: the high halves at the arena offsets, the low halves count elements later, then the exponents
- * of the matrices' largest magnitudes (policy_lane.h); with NULL there, collect takes the fp32 copies.
- * Otherwise they are NULL. The fused kernels read the matrices from them. The library derives all of them from params at creation and in
- * mg_ppo_set_params / mg_ppo_params_updated. A train step (mg_ppo_train, mg_ppo_train_block,
- * mg_ppo_train_block_noalloc) rewrites only the copies its own kernels read next (frag_fwd16
- * and frag_bwd16; in bf16 mode their bf16 versions) and leaves the others (frag_fwd32, frag_fwd32_bf, and in
- * bf16 mode the fp32 copies) behind params until the next mg_ppo_policy,
+ * 16 and 32, each lane 8 consecutive k). With MG_PRECISION_FP32 the three hold
+ * the same matrices in the same orders as pairs of binary16 values, each
+ * element times a power of two of its matrix: the high halves at the arena
+ * offsets, the low halves count elements later, then the matrices' exponents
+ * (behind frag_fwd32_bf: SplitScale, policy_lane.h; behind frag_fwd16_bf, for
+ * both 16-row orders: PairScale, policy_pair.h). Where frag_fwd32_bf or
+ * frag_fwd16_bf is NULL an fp32 collect takes the fp32 copies. The fused
+ * kernels read the matrices from all of these. The library derives them from
+ * params at creation and in mg_ppo_set_params / mg_ppo_params_updated. A train
+ * step (mg_ppo_train, mg_ppo_train_block, mg_ppo_train_block_noalloc) rewrites
+ * only the copies its own kernels read next (frag_fwd16_bf and frag_bwd16_bf; frag_fwd16 and
+ * frag_bwd16 where an fp32 policy's row pass runs on those) and leaves the others behind params
+ * until the next mg_ppo_policy,
  * mg_ppo_collect or mg_ppo_forward re-derives them. The pointers never change, so a view stays
  * valid for the model's life, but its copies are current only after one of those calls: a
  * caller that launches kernels with a view after training (an env's mg_env_desc.collect, say)

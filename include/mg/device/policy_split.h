@@ -1,6 +1,7 @@
 // The hidden-unit split of a 16-row policy tile: the layout of the fp32 row
 // pass of a PPO minibatch (metalgym_amd/csrc/rows_split.h) and of collect's
-// fp32 16-row tiles (split_forward16 below).
+// fp32 16-row tiles (pair_forward, policy_pair.h; split_forward16 below for the
+// envs it does not take).
 //
 // A workgroup owns 16 rows on W waves (W = 4: one per SIMD; W = 8: two). Wave
 // w owns the S = 8 / W 16-unit strips 128 c + 16 (S w + s), s < S, of every

@@ -1,7 +1,8 @@
 // The rollout<Env> kernel: one lane per env, `steps` env steps per launch with
 // the state and RNG held in registers (rollout.h:31-54 runs one step per
 // dispatch and round-trips everything through memory). Envs with a split
-// observation and a large state run rollout_split_kernel instead (below).
+// observation and a large state run rollout_split_kernel instead (below), or a
+// kernel of their own (PackedRollout; rollout_voxelnav16.h).
 //
 // Per env and step: pick the action (given, or drawn from the env's RNG before
 // the reset), reset if the stored done flag is set, Env::step, then coalesced

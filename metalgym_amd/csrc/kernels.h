@@ -56,10 +56,10 @@ int check_matrix_layout(const mg_policy_view& pv);
 int train_ws_bytes(const mg_policy_view& pv, uint32_t rows, size_t* bytes);
 int train_ws_bind(const mg_policy_view& pv, uint32_t rows, void* base, TrainWs* ws);
 // One minibatch: rows pass, weight-gradient pass, reduce + norm, Adam. Adam
-// rewrites only the fragment-tiled copies the row pass reads (frag_fwd16 and
-// frag_bwd16, or their bf16 versions in bf16 mode); the others (frag_fwd32,
-// frag_fwd32_bf and, in bf16 mode, the fp32 copies, read by collect and
-// forward) are stale afterwards until launch_derive_blocks.
+// rewrites only the fragment-tiled copies the row pass reads (frag_fwd16_bf and
+// frag_bwd16_bf: pairs of binary16, or bfloat16 in bf16 mode; frag_fwd16 and
+// frag_bwd16 for fp32 policies whose row pass takes the fp32 copies); the others
+// (read by collect and forward) are stale afterwards until launch_derive_blocks.
 int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hparams& hp, float lr,
                       const TrainWs& ws, const TrainStep& step, const float* obs_slots, const void* action_slots,
                       const float* adv_slots, const float* ret_slots, const float* logp_slots,

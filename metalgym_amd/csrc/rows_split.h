@@ -1,5 +1,6 @@
 // The fp32 row pass of a PPO minibatch (the work of train_rows_kernel<false>:
-// forward recompute with capture, loss, backward dX chain, tile partials) in
+// forward recompute with capture, loss, backward dX chain, tile partials; the
+// block GEMMs on pairs of binary16 values, policy_pair.h, or in fp32) in
 // the hidden-unit split layout of include/mg/device/policy_split.h, so that no
 // chunk GEMM waits on a barrier. Included by train_kernels.hip. The loss
 // reduces over the same TPR lanes as LayerNorm. The captures for the weight
