@@ -36,11 +36,15 @@
 // the weights are stored scaled (SplitScale, from each matrix's largest
 // magnitude), gamma and beta are staged scaled so that no LN output row is
 // longer than 2^15 (a normalised row of 128 is at most sqrt(128) long), hence
-// |V| <= 2^15 sqrt(128) 2^13 < 2^32 whatever the observation, which 2^-17 takes
+// |V| <= 2^15 sqrt(128) 2^13 < 2^31.6 whatever the observation, which 2^-16 takes
 // into range, and the residual stream is kept in the units of the block's
 // product. Weights down to 2^-15 of their matrix's largest and LN outputs and
 // hidden units down to 2^-16 of their bounds keep all 22 bits; below that
 // their error is 2^-38 of the largest.
+// Infinities come out as in fp32: a weight that is not finite is in its low
+// plane alone (pack_weights), so it meets the other operand's high half only,
+// and a hidden unit at infinity, which pack_hidden's clamp holds at 2^32, leaves
+// binary16's range again in the conversion.
 //
 // MG_PRECISION_BF16: one bfloat16 plane, as policy_bf16.h.
 #pragma once
@@ -88,11 +92,11 @@ __device__ __forceinline__ int pow2_above(float m) {
     return (int)((__builtin_bit_cast(uint32_t, m) >> 23) & 0xFFu) - 126;
 }
 // The exponents of a block's powers of two: |up| and |down| < 2^13 after them,
-// an LN output row shorter than 2^15, hidden units times 2^-17. Small matrices
+// an LN output row shorter than 2^15, hidden units times 2^-16. Small matrices
 // are scaled up only so far that the residual stream, in units of the block's
 // product, stays under 2^60 of itself; a down matrix may be as small as its up
 // matrix is large.
-constexpr int kMatTarget = 13, kRowTarget = 15, kHiddenExp = -17;
+constexpr int kMatTarget = 13, kRowTarget = 15, kHiddenExp = -16;
 __host__ __device__ __forceinline__ int split_min(int a, int b) { return a < b ? a : b; }
 __host__ __device__ __forceinline__ int split_exp_up(const SplitScale& s, int l) {
     return split_min(kMatTarget - s.up[l], 49);
@@ -143,9 +147,19 @@ struct LaneOps<MG_PRECISION_FP32> {
             p[1][2 * j] = lo[0], p[1][2 * j + 1] = lo[1];
         }
     }
+    // The planes of weights. inf = inf + (inf - inf) would make every product
+    // NaN, and the relu a 0 of that; as 0 + inf it is infinity times the high
+    // half of the other operand, with the fp32 product's sign (and NaN times 0).
+    __device__ static __forceinline__ void pack_weights(const float (&x)[8], V (&p)[2]) {
+        pack(x, p);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (!(fabsf(x[j]) < 65520.0f)) p[0][j] = (_Float16)0.0f, p[1][j] = (_Float16)x[j];
+    }
     // relu of hidden units, times 2^kHiddenExp: 2^-32 takes them under 1, where
     // the multiplication's own clamp is the relu (0 for NaN, as x > 0 ? x : 0),
-    // and the conversion takes them up again
+    // and the conversion takes them up again (from the clamp's 1, an infinite
+    // unit, to 2^16: infinity in binary16)
     __device__ static __forceinline__ void pack_hidden(const float (&x)[8], V (&p)[2]) {
         const float f = opaque((float)(1 << (32 + kHiddenExp)));
 #pragma unroll

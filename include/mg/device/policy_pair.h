@@ -33,9 +33,9 @@ constexpr int kPairRowTarget = 11;   // |x| < 2^11 in a scaled block input row: 
 constexpr int kPairTiles = 128;      // most 32 x 32 tiles of a block matrix
 
 // The scales of the planes, after frag_fwd16_bf's 2 count halves. A matrix's
-// exponent follows its largest magnitude, which an Adam step changes: Adam
-// writes its planes with `next`, records it in `cur` and leaves each tile's
-// largest magnitude in tilemax; the next row pass makes `next` from those and
+// exponent follows its largest finite magnitude, which an Adam step changes:
+// Adam writes its planes with `next`, records it in `cur` and leaves each tile's
+// largest finite magnitude in tilemax; the next row pass makes `next` from those and
 // from what one more Adam step can add. |m| <= 7.27 sqrt(v) for Adam's moments
 // (Cauchy-Schwarz over their weights, beta 0.9 and 0.999, both from 0) and the
 // bias corrections only shrink that ratio, so a step moves no weight by more

@@ -1288,7 +1288,7 @@ __device__ __forceinline__ void store_tile_split(const MatTile& m, const float* 
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[j] = scale * lds[(kb + j) * kTileLd + nb];
     f16x8 p[2];
-    LaneOps<MG_PRECISION_FP32>::pack(x, p);
+    LaneOps<MG_PRECISION_FP32>::pack_weights(x, p);
     uint16_t* at = planes + m.base + frag_index_b<32>(m.c0 + nb, m.r0 + kb, m.rows);
     *reinterpret_cast<f16x8*>(at) = p[0];
     *reinterpret_cast<f16x8*>(at + count) = p[1];
@@ -1319,7 +1319,7 @@ __device__ __forceinline__ void store_tile_pair(const MatTile& m, const float* l
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[j] = f * lds[(r0 + j * dr) * kTileLd + c0 + j * dc];
     f16x8 p[2];
-    LaneOps<MG_PRECISION_FP32>::pack(x, p);
+    LaneOps<MG_PRECISION_FP32>::pack_weights(x, p);
     uint16_t* out = (half == (down ? 1 : 0) ? fwd : bwd) + 2 * (size_t)m.base + at;
     *reinterpret_cast<f16x8*>(out) = p[0];
     *reinterpret_cast<f16x8*>(out + 512) = p[1];
@@ -1468,7 +1468,7 @@ __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
             const int r = (256 / kTT) * e + t / kTT;
             const float p = adam_elem(a, idx[e], in[e], scale);
             lds[r * kTileLd + c] = p;
-            if (PAIRS) most = fmaxf(most, fabsf(p));
+            if (PAIRS && fabsf(p) < __builtin_huge_valf()) most = fmaxf(most, fabsf(p));
         }
         if constexpr (PAIRS) {  // this tile's planes, and what the next step's exponent needs (PairScale)
             most = group_max<64>(most);
