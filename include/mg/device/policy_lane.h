@@ -290,14 +290,18 @@ struct LaneParams {
 };
 
 // The exponent of the power of two for an LN's gamma and beta, from their 128
-// values each: a wave-wide computation.
-__device__ __forceinline__ int lane_row_exp(const float* gamma, const float* beta) {
+// values each: a wave-wide computation. poison: an element is infinite and none
+// is NaN, so that fp32 arithmetic has infinite inputs of every row (a NaN makes
+// every hidden unit of the block NaN, and the relu a 0 of it, in both).
+__device__ __forceinline__ int lane_row_exp(const float* gamma, const float* beta, bool& poison) {
     const int lane = threadIdx.x & 63;
     const float g0 = gamma[lane], g1 = gamma[lane + 64], b0 = beta[lane], b1 = beta[lane + 64];
     const float g = group_max<64>(fmaxf(fabsf(g0), fabsf(g1)));
     const float b = group_max<64>(fmaxf(fabsf(b0), fabsf(b1)));
-    const float len = 11.4f * (g + b);  // sqrt(128) (max |gamma| + max |beta|), rounded up
-    return len < __builtin_huge_valf() ? split_min(kRowTarget - pow2_above(len), 28) : 0;
+    // sqrt(128) (max |gamma| + max |beta|), rounded up, times 2^-8 against overflow
+    const float len = 11.4f * (0x1p-8f * g + 0x1p-8f * b);
+    poison = len == __builtin_huge_valf() && !__any(g0 != g0 || g1 != g1 || b0 != b0 || b1 != b1);
+    return split_min(kRowTarget - 8 - pow2_above(len), 28);
 }
 
 // Row sums over the lane pair.
@@ -699,12 +703,17 @@ __device__ __forceinline__ void lane_start(const mg_policy_view& pv, float* lds,
         if constexpr (PREC == MG_PRECISION_FP32) {
             if (l < nl) {
                 const SplitScale& ss = *split_scale(pv.frag_fwd32_bf, pv.count);
-                const int ex = lane_row_exp(lnp + 2 * kEmbed * l, lnp + 2 * kEmbed * l + kEmbed);
+                bool poison;
+                const int ex = lane_row_exp(lnp + 2 * kEmbed * l, lnp + 2 * kEmbed * l + kEmbed, poison);
                 xs = pow2i(ex);
                 // the unit of block l's product (at 2^-126 the products are past fp32's range)
                 int e = ex + split_exp_up(ss, l) + kHiddenExp + split_exp_down(ss, l);
                 e = e < -126 ? -126 : e;
-                if (tid == 0) lds[L.scale + 2 * l] = pow2i(e), lds[L.scale + 2 * l + 1] = pow2i(-e);
+                // poison: an infinite input's planes are inf and NaN, which the relu would
+                // turn into a block output of 0
+                if (tid == 0)
+                    lds[L.scale + 2 * l] = pow2i(e),
+                    lds[L.scale + 2 * l + 1] = poison ? __builtin_nanf("") : pow2i(-e);
             }
         }
         if (tid < 2 * kEmbed) lds[L.ln + 2 * kEmbed * l + tid] = xs * lnp[2 * kEmbed * l + tid];

@@ -161,7 +161,8 @@ struct alignas(16) PairInput {
 };
 
 // A row's block input (NV float4s per thread, TPR threads) to planes, scaled
-// by the row's own power of two; returns its exponent.
+// by the row's own power of two; returns its exponent. An infinite element is in
+// the low plane alone, as an infinite weight (LaneOps::pack_weights).
 template <int TPR, int NV>
 __device__ __forceinline__ int pair_store_input(PairInput& in, const RowVec<NV>& x, int row, int lk, int e0) {
     static_assert(NV == 1, "four columns per thread");
@@ -174,8 +175,15 @@ __device__ __forceinline__ int pair_store_input(PairInput& in, const RowVec<NV>&
     split_f16_scaled(x[0], x[1], opaque_v(f), h0, l0);
     split_f16_scaled(x[2], x[3], opaque_v(f), h1, l1);
     typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<f16x4*>(&in.x[0][row * kPairLd + 4 * lk]) = f16x4{h0[0], h0[1], h1[0], h1[1]};
-    *reinterpret_cast<f16x4*>(&in.x[1][row * kPairLd + 4 * lk]) = f16x4{l0[0], l0[1], l1[0], l1[1]};
+    f16x4 hi = {h0[0], h0[1], h1[0], h1[1]}, lo = {l0[0], l0[1], l1[0], l1[1]};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const bool inf = __builtin_isinf((float)hi[c]);
+        lo[c] = inf ? hi[c] : lo[c];
+        hi[c] = inf ? (_Float16)0.0f : hi[c];
+    }
+    *reinterpret_cast<f16x4*>(&in.x[0][row * kPairLd + 4 * lk]) = hi;
+    *reinterpret_cast<f16x4*>(&in.x[1][row * kPairLd + 4 * lk]) = lo;
     if (lk == 0) in.unit[row] = e + e0;
     return e;
 }

@@ -39,6 +39,10 @@ def spoil(pv, P, how):
         "up nan": (pv.off_up[0] + 79, np.nan),
         "down inf": (pv.off_down[0] + 80, np.inf),
         "down nan": (pv.off_down[1] + 81, np.nan),
+        "gamma inf": (pv.off_ln_gamma[0] + 7, np.inf),
+        "gamma nan": (pv.off_ln_gamma[1] + 7, np.nan),
+        "beta -inf": (pv.off_ln_beta[1] + 8, -np.inf),
+        "final gamma inf": (pv.off_ln_gamma[2] + 9, np.inf),
     }[how]
     P[at] = value
     return P
@@ -54,10 +58,10 @@ def check_heads(pv, P, obs, got):
     return finite
 
 
-WEIGHTS = ["up inf", "up -inf", "up nan", "down inf", "down nan"]
+HOW = ["up inf", "up -inf", "up nan", "down inf", "down nan", "gamma inf", "gamma nan", "beta -inf", "final gamma inf"]
 
 
-@pytest.mark.parametrize("how", WEIGHTS)
+@pytest.mark.parametrize("how", HOW)
 @pytest.mark.parametrize("rows", [1000, 8200])  # 16-row tiles on pairs, row per lane pair
 def test_forward(mg, rows, how):
     gym = mg.Gym(ENVS["cartpole"][1], 64, 0)
@@ -70,7 +74,7 @@ def test_forward(mg, rows, how):
         assert 0.2 < finite.mean() < 0.8
 
 
-@pytest.mark.parametrize("how", WEIGHTS)
+@pytest.mark.parametrize("how", HOW)
 @pytest.mark.parametrize("n", [64, 8256, 16448])  # 16-row tiles on pairs, two shares, one
 def test_collect(mg, n, how):
     gym = mg.Gym(ENVS["cartpole"][1], n, 0)
@@ -81,7 +85,7 @@ def test_collect(mg, n, how):
     check_heads(model.pv, P, model.download_slots()["obs"][2], model.head())
 
 
-@pytest.mark.parametrize("how", WEIGHTS)
+@pytest.mark.parametrize("how", HOW)
 def test_minibatch(mg, how):
     """The row pass computes the same heads, and a loss that is not finite
     reaches the gradient's norm."""
