@@ -286,7 +286,7 @@ struct LaneParams {
     const float* bin;
     const float* wh;
     const float* win;  // LDS, or the arena
-    const float* scale;  // per block: the residual stream's unit, then its inverse
+    const float* scale;  // per block: the exponent (int) of the residual stream's unit, then the unit's inverse
 };
 
 // The exponent of the power of two for an LN's gamma and beta, from their 128
@@ -447,6 +447,8 @@ __device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const Lan
     }
     if constexpr (HS > 1) Ring::barrier();  // the observations' LDS is read
     float inv = 1.0f;
+    float near = 1.0f;  // fp32: 0 for a row too large for the units of a block, NaN for one that is not finite
+    int exp = 0;        // of the stream's unit
     for (uint32_t l = 0; l < pv.layers; ++l) {
         float mean, rstd;
         lane_stats(R, inv, mean, rstd);
@@ -463,14 +465,18 @@ __device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const Lan
             Ops::pack(x, xb[s]);
         }
         if constexpr (PREC == MG_PRECISION_FP32) {
-            // the stream to this block's units
-            // (in share 0's sum)
-            const float f = half ? 0.0f : P.scale[2 * l] * inv;
-            inv = P.scale[2 * l + 1];
+            // the stream to this block's units (in share 0's sum). They hold rows
+            // under 2^67; larger ones have a deviation of infinity, so LN gives
+            // them beta, here and in all that follows: as it does a stream of 0.
+            if (!(rstd > 0.0f && fabsf(mean) <= 0x1p66f)) near = 0.0f * rstd;
+            const int e = __builtin_bit_cast(int, P.scale[2 * l]);
+            const int by = half || near == 0.0f ? -1000 : e - exp;
+            exp = e;
+            inv = P.scale[2 * l + 1] * near;
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) R.h[mt][r] *= f;
+                for (int r = 0; r < 16; ++r) R.h[mt][r] = __builtin_ldexpf(R.h[mt][r], by);
         } else if constexpr (HS > 1) {
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
@@ -712,7 +718,7 @@ __device__ __forceinline__ void lane_start(const mg_policy_view& pv, float* lds,
                 // poison: an infinite input's planes are inf and NaN, which the relu would
                 // turn into a block output of 0
                 if (tid == 0)
-                    lds[L.scale + 2 * l] = pow2i(e),
+                    lds[L.scale + 2 * l] = __builtin_bit_cast(float, e),
                     lds[L.scale + 2 * l + 1] = poison ? __builtin_nanf("") : pow2i(-e);
             }
         }

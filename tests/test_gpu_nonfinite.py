@@ -1,4 +1,4 @@
-"""Parameters that are not finite, in the kernels that split fp32 operands
+"""Parameters that are not finite, or near the end of fp32's range, in the kernels that split fp32 operands
 (policy_lane.h, policy_pair.h): a head is finite exactly where the float64
 network's is, with its relu (0 for NaN), and as close as elsewhere; a diverged
 policy is not taken for a healthy one."""
@@ -10,9 +10,9 @@ from parity import ENVS
 pytestmark = pytest.mark.gpu
 
 
-def network64(pv, P, obs):
-    """model/ppo.h:575-626 in float64, the relu 0 for NaN as in the kernels."""
-    P = P.astype(np.float64)
+def network(pv, P, obs, dtype):
+    """model/ppo.h:575-626 in dtype, the relu 0 for NaN as in the kernels."""
+    P = P.astype(dtype)
     E, H, O, HD = 128, pv.hidden, pv.obs_dim, pv.head_dim
 
     def mat(off, r, c):
@@ -20,10 +20,10 @@ def network64(pv, P, obs):
 
     def ln(h, l):
         d = h - h.mean(1, keepdims=True)
-        xn = d / np.sqrt((d * d).mean(1, keepdims=True) + 1e-5)
+        xn = d * (1 / np.sqrt((d * d).mean(1, keepdims=True) + dtype(1e-5)))
         return xn * mat(pv.off_ln_gamma[l], 1, E) + mat(pv.off_ln_beta[l], 1, E)
 
-    h = obs.astype(np.float64) @ mat(pv.off_in_w, O, E) + mat(pv.off_in_b, 1, E)
+    h = obs.astype(dtype) @ mat(pv.off_in_w, O, E) + mat(pv.off_in_b, 1, E)
     for l in range(pv.layers):
         v = ln(h, l) @ mat(pv.off_up[l], E, H)
         h = h + np.where(v > 0, v, 0) @ mat(pv.off_down[l], H, E)
@@ -50,7 +50,7 @@ def spoil(pv, P, how):
 
 def check_heads(pv, P, obs, got):
     with np.errstate(all="ignore"):
-        want = network64(pv, P, obs)
+        want = network(pv, P, obs, np.float64)
     finite = np.isfinite(want).all(1)
     np.testing.assert_array_equal(np.isfinite(got).all(1), finite)
     assert not np.isfinite(got[~finite]).any(), "every column of such a row goes through the final LayerNorm"
@@ -98,3 +98,61 @@ def test_minibatch(mg, how):
     model.train_block(1)
     finite = check_heads(model.pv, P, model.download_slots()["obs"][1], model.head())
     assert finite.all() or not np.isfinite(model.last_stats().grad_norm)
+
+
+def shifted(pv, P):
+    """P with betas, which rows too long for fp32's squares come down to."""
+    P = P.copy()
+    for l in range(pv.layers + 1):
+        P[pv.off_ln_beta[l]:pv.off_ln_beta[l] + 128] = np.random.default_rng(l).normal(0, 0.5, 128)
+    return P
+
+
+@pytest.mark.parametrize("rows", [1000, 8200])
+def test_forward_of_huge_rows(mg, rows):
+    """Observations to 1e35: past about 1e19 the squares of a row's deviations
+    overflow, LayerNorm divides by infinity and leaves beta."""
+    gym = mg.Gym(ENVS["cartpole"][1], 64, 0)
+    model = mg.PPOModel(gym, horizon=1)
+    P = shifted(model.pv, model.params())
+    model.set_params(P)
+    obs = np.random.default_rng(3).normal(0, 1.5, (rows, 4)).astype(np.float32)
+    obs *= np.float32(10.0) ** np.array([0, 10, 17, 21, 25, 30, 35], np.float32)[np.arange(rows) % 7, None]
+    with np.errstate(over="ignore"):
+        want = network(model.pv, P, obs, np.float32)
+    np.testing.assert_allclose(model.forward(obs), want, rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("n", [64, 8256, 16448])
+def test_collect_of_huge_rows(mg, n):
+    gym = mg.Gym(ENVS["cartpole"][1], n, 0)
+    model = mg.PPOModel(gym, horizon=2, minibatch=64)
+    pv = model.pv
+    P = shifted(pv, model.params())
+    P[pv.off_in_w:pv.off_in_w + 4 * 128] *= np.float32(1e33)
+    model.set_params(P)
+    model.collect()
+    with np.errstate(over="ignore"):
+        want = network(pv, P, model.download_slots()["obs"][2], np.float32)
+    np.testing.assert_allclose(model.head(), want, rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("rows", [1000, 8200])
+def test_blocks_with_units_far_apart(mg, rows):
+    """One up weight of 1e36: the first block's unit is 2^-100 of the second's."""
+    gym = mg.Gym(ENVS["cartpole"][1], 64, 0)
+    model = mg.PPOModel(gym, horizon=1)
+    P = shifted(model.pv, model.params())
+    P[model.pv.off_up[0] + 77] = 1e36
+    model.set_params(P)
+    obs = np.random.default_rng(3).normal(0, 1.5, (rows, 4)).astype(np.float32)
+    with np.errstate(over="ignore"):
+        want = network(model.pv, P, obs, np.float32)
+    got = model.forward(obs)
+    assert np.isfinite(got).all()
+    # where the unit is on, the row is too long for fp32's squares
+    pv = model.pv
+    beta, head = P[pv.off_ln_beta[2]:pv.off_ln_beta[2] + 128], P[pv.off_head:pv.off_head + 384].reshape(128, 3)
+    on = np.abs(want - beta @ head).max(1) < 1e-5
+    assert 0.2 < on.mean() < 0.8
+    np.testing.assert_allclose(got[on], want[on], rtol=0, atol=1e-4)
