@@ -169,18 +169,18 @@ __device__ __forceinline__ int pair_store_input(PairInput& in, const RowVec<NV>&
     float m = 0.0f;
 #pragma unroll
     for (int c = 0; c < 4; ++c) m = fmaxf(m, fabsf(x[c]));
-    const int e = split_min(kPairRowTarget - pow2_above(group_max<TPR>(m)), 40);
+    m = group_max<TPR>(m);
+    const int e = split_min(kPairRowTarget - pow2_above(m), 40);
     const float f = pow2i(e < -126 ? -126 : e);
     f16x2 h0, l0, h1, l1;
     split_f16_scaled(x[0], x[1], opaque_v(f), h0, l0);
     split_f16_scaled(x[2], x[3], opaque_v(f), h1, l1);
     typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
     f16x4 hi = {h0[0], h0[1], h1[0], h1[1]}, lo = {l0[0], l0[1], l1[0], l1[1]};
+    if (__any(m == __builtin_huge_valf())) {  // one branch in the chain from LN to the products: the selects alone took 0.1 us
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const bool inf = __builtin_isinf((float)hi[c]);
-        lo[c] = inf ? hi[c] : lo[c];
-        hi[c] = inf ? (_Float16)0.0f : hi[c];
+        for (int c = 0; c < 4; ++c)
+            if (__builtin_isinf((float)hi[c])) lo[c] = hi[c], hi[c] = (_Float16)0.0f;
     }
     *reinterpret_cast<f16x4*>(&in.x[0][row * kPairLd + 4 * lk]) = hi;
     *reinterpret_cast<f16x4*>(&in.x[1][row * kPairLd + 4 * lk]) = lo;
