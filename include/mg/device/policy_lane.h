@@ -98,11 +98,9 @@ __device__ __forceinline__ int pow2_above(float m) {
 // matrix is large.
 constexpr int kMatTarget = 13, kRowTarget = 15, kHiddenExp = -16;
 __host__ __device__ __forceinline__ int split_min(int a, int b) { return a < b ? a : b; }
-__host__ __device__ __forceinline__ int split_exp_up(const SplitScale& s, int l) {
-    return split_min(kMatTarget - s.up[l], 49);
-}
-__host__ __device__ __forceinline__ int split_exp_down(const SplitScale& s, int l) {
-    return split_min(split_min(kMatTarget - s.down[l], 49 - split_exp_up(s, l)), 126);
+__host__ __device__ __forceinline__ int split_exp_up(int up) { return split_min(kMatTarget - up, 49); }
+__host__ __device__ __forceinline__ int split_exp_down(int up, int down) {
+    return split_min(split_min(kMatTarget - down, 49 - split_exp_up(up)), 126);
 }
 
 // x = hi + lo in binary16, both rounded to nearest even; the remainder x - hi
@@ -713,7 +711,7 @@ __device__ __forceinline__ void lane_start(const mg_policy_view& pv, float* lds,
                 const int ex = lane_row_exp(lnp + 2 * kEmbed * l, lnp + 2 * kEmbed * l + kEmbed, poison);
                 xs = pow2i(ex);
                 // the unit of block l's product (at 2^-126 the products are past fp32's range)
-                int e = ex + split_exp_up(ss, l) + kHiddenExp + split_exp_down(ss, l);
+                int e = ex + split_exp_up(ss.up[l]) + kHiddenExp + split_exp_down(ss.up[l], ss.down[l]);
                 e = e < -126 ? -126 : e;
                 // poison: an infinite input's planes are inf and NaN, which the relu would
                 // turn into a block output of 0

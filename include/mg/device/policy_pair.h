@@ -40,7 +40,8 @@ constexpr int kPairTiles = 128;      // most 32 x 32 tiles of a block matrix
 // (Cauchy-Schwarz over their weights, beta 0.9 and 0.999, both from 0) and the
 // bias corrections only shrink that ratio, so a step moves no weight by more
 // than 7.27 lr. All of it stays on the device, in stream order, so a captured
-// train step replays correctly.
+// train step replays correctly. tilemax also gives the collects' exponents
+// after a train call (derive_blocks_kernel).
 constexpr float kAdamReach = 7.3f;
 struct PairScale {
     int cur[2 * MG_MAX_LAYERS];  // per block matrix (up, down per layer): the planes' exponent

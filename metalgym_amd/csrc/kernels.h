@@ -47,8 +47,9 @@ struct TrainStep {
 };
 
 // All fragment-tiled copies of the block matrices (frag_fwd32, frag_fwd16,
-// frag_bwd16 and the bf16 ones that exist) from params.
-int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv);
+// frag_bwd16 and the 16-bit ones) from params. trained: params were last
+// written by launch_train_step.
+int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv, bool trained);
 // MG_OK if the block matrices sit contiguously from float_group (the layout
 // the Adam and derive kernels tile).
 int check_matrix_layout(const mg_policy_view& pv);

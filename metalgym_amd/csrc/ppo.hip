@@ -194,7 +194,7 @@ int enqueue_minibatch(mg_ppo* p, uint32_t block, uint32_t mb_index, const TrainW
 // kernel that reads them.
 int sync_tiles(mg_ppo* p) {
     if (!p->tiles_stale) return MG_OK;
-    int rc = launch_derive_blocks(p->gym->stream, p->pv);
+    int rc = launch_derive_blocks(p->gym->stream, p->pv, true);
     if (rc) return rc;
     p->tiles_stale = false;
     return MG_OK;
@@ -387,7 +387,7 @@ int mg_ppo_create(mg_gym* gym, const mg_ppo_config* c, mg_ppo** out) {
         hipMemsetAsync(p->slots, 0, slot_bytes, st) != hipSuccess ||
         hipMemsetAsync(p->head, 0, (size_t)p->head_cap * pv.head_dim * 4, st) != hipSuccess)
         return fail(set_error(MG_ERR_HIP, "PPOModel: initialisation upload failed"));
-    if ((rc = launch_derive_blocks(st, pv))) return fail(rc);
+    if ((rc = launch_derive_blocks(st, pv, false))) return fail(rc);
     if (hipStreamSynchronize(st) != hipSuccess)
         return fail(set_error(MG_ERR_HIP, "PPOModel: initialisation upload failed"));
     p->order.resize(p->blocks);
@@ -595,7 +595,7 @@ int mg_ppo_set_params(mg_ppo* p, const float* host, uint32_t count) {
 
 int mg_ppo_params_updated(mg_ppo* p) {
     MG_CHECK(p, MG_ERR_INVALID, "params_updated: null model");
-    int rc = launch_derive_blocks(p->gym->stream, p->pv);
+    int rc = launch_derive_blocks(p->gym->stream, p->pv, false);
     if (rc) return rc;
     p->tiles_stale = false;
     MG_HIP(hipStreamSynchronize(p->gym->stream), "params_updated synchronize");

@@ -1325,48 +1325,62 @@ __device__ __forceinline__ void store_tile_pair(const MatTile& m, const float* l
     *reinterpret_cast<f16x8*>(out + 512) = p[1];
 }
 
-// SplitScale from params: per block matrix (128 hidden floats each, contiguous
-// from float_group), one per workgroup, the exponent of its largest finite
-// magnitude. pairs: also the pair planes' exponents and their tiles' magnitudes
-// (the matrix's for each), one entry per workgroup.
-__global__ void __launch_bounds__(1024) split_scale_kernel(const float* __restrict__ param, uint32_t float_group,
-                                                           uint32_t EH, SplitScale* out, PairScale* pairs) {
-    __shared__ float red[16];
-    const f32x4* p = reinterpret_cast<const f32x4*>(param + float_group + (size_t)blockIdx.x * EH);
-    float m = 0.0f;
-#pragma unroll 8
-    for (uint32_t k = threadIdx.x; k < EH / 4; k += 1024) {
-        const f32x4 v = p[k];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float x = fabsf(v[j]);
-            m = x < __builtin_huge_valf() && x > m ? x : m;
-        }
-    }
+// The largest of f over a workgroup of 256, in thread 0, after a barrier; wmax
+// holds 4.
+__device__ __forceinline__ float wg_max(float m, float* wmax) {
     m = group_max<64>(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x < kPairTiles) {
-        m = group_max<16>(red[threadIdx.x & 15]);
-        if (threadIdx.x == 0) {
-            ((blockIdx.x & 1) ? out->down : out->up)[blockIdx.x >> 1] = pow2_above(m);
-            if (pairs) pairs->cur[blockIdx.x] = pairs->next[blockIdx.x] = pair_exp(m);
-        }
-        if (pairs) pairs->tilemax[blockIdx.x][threadIdx.x] = m;
+    return fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+}
+__device__ __forceinline__ float finite_magnitude(float x) {
+    const float m = fabsf(x);
+    return m < __builtin_huge_valf() ? m : 0.0f;
+}
+
+// PairScale.tilemax from params, one tile per workgroup.
+__global__ void __launch_bounds__(256) tile_max_kernel(const float* __restrict__ param, uint32_t float_group,
+                                                       uint32_t H, PairScale* pairs) {
+    __shared__ float wmax[4];
+    const MatTile m = mat_tile(blockIdx.x, float_group, H);
+    const uint32_t per = H * kEmbed / (kTT * kTT);
+    float most = 0.0f;
+#pragma unroll
+    for (int e = 0; e < kTT * kTT / 256; ++e) {
+        const int r = (256 / kTT) * e + threadIdx.x / kTT;
+        most = fmaxf(most, finite_magnitude(param[m.base + (size_t)(m.r0 + r) * m.cols + m.c0 + (threadIdx.x & (kTT - 1))]));
     }
+    most = wg_max(most, wmax);
+    if (threadIdx.x == 0) pairs->tilemax[blockIdx.x / per][blockIdx.x % per] = most;
 }
 
 // The fragment-tiled copies from params, one tile per workgroup. split: an
 // fp32 policy's planes, which take fwd32b's place, pfwd and pbwd: its pair
-// planes, in fwd16b's and bwd16b's (the scales after them are current).
+// planes, in fwd16b's and bwd16b's, with their scales, whose tilemax is
+// current. Each workgroup takes its block's exponents from that (a kernel of
+// one workgroup per matrix before this one took 8 us of every collect after a
+// train call); the first of a matrix records them. adam: an Adam step has just
+// written the pair planes, with `next`, which serve unless the magnitudes ask
+// for another exponent.
 __global__ void __launch_bounds__(256) derive_blocks_kernel(const float* __restrict__ param, float* __restrict__ fwd32,
                                                             float* __restrict__ fwd16, float* __restrict__ bwd16,
                                                             uint16_t* fwd32b, uint16_t* fwd16b, uint16_t* bwd16b,
-                                                            uint16_t* split, uint16_t* pfwd, uint16_t* pbwd,
+                                                            uint16_t* split, uint16_t* pfwd, uint16_t* pbwd, bool adam,
                                                             uint32_t count, uint32_t float_group, uint32_t H) {
     __shared__ float lds[kTT * kTileLd];
     const MatTile m = mat_tile(blockIdx.x, float_group, H);
     const int t = threadIdx.x, c = t & (kTT - 1);
+    const uint32_t per = H * kEmbed / (kTT * kTT), mat = blockIdx.x / per;  // at most kPairTiles tiles a matrix
+    PairScale* const pairs = split ? pair_scale(pfwd, count) : nullptr;
+    float most[2] = {};  // of the block's up and down
+    if (split) {
+        const uint32_t lane = t & 63;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float* tm = pairs->tilemax[(mat & ~1u) + k];
+            most[k] = fmaxf(lane < per ? tm[lane] : 0.0f, lane + 64 < per ? tm[lane + 64] : 0.0f);
+        }
+    }
 #pragma unroll
     for (int e = 0; e < kTT * kTT / 256; ++e) {
         const int r = (256 / kTT) * e + t / kTT;
@@ -1374,10 +1388,16 @@ __global__ void __launch_bounds__(256) derive_blocks_kernel(const float* __restr
     }
     store_tile_frags(m, lds, fwd32, fwd16, bwd16, fwd32b, fwd16b, bwd16b);
     if (split) {
-        const SplitScale& ss = *split_scale(split, count);
-        const int mat = (int)((m.base - float_group) / (kEmbed * H)), l = mat >> 1;
-        store_tile_split(m, lds, split, count, pow2i((mat & 1) ? split_exp_down(ss, l) : split_exp_up(ss, l)));
-        if (pfwd) store_tile_pair(m, lds, pfwd, pbwd, mat & 1, pair_scale(pfwd, count)->cur[mat]);
+        const float up = group_max<64>(most[0]), down = group_max<64>(most[1]);
+        const bool is_down = mat & 1;
+        const int eu = pow2_above(up), ed = pow2_above(down), pe = pair_exp(is_down ? down : up);
+        store_tile_split(m, lds, split, count, pow2i(is_down ? split_exp_down(eu, ed) : split_exp_up(eu)));
+        if (!adam || pe != pairs->next[mat]) store_tile_pair(m, lds, pfwd, pbwd, is_down, pe);
+        if (blockIdx.x % per == 0 && t == 0) {
+            SplitScale& ss = *const_cast<SplitScale*>(split_scale(split, count));
+            (is_down ? ss.down : ss.up)[mat >> 1] = is_down ? ed : eu;
+            pairs->cur[mat] = pe;
+        }
     }
 }
 
@@ -1391,6 +1411,7 @@ struct AdamArgs {
     uint16_t* frag_bwd16_bf;
     uint16_t* pair_fwd;  // the pair planes in the place of frag_fwd16 / frag_bwd16, or NULL
     uint16_t* pair_bwd;
+    PairScale* pairs;  // fp32
     const float* grad;
     float* mom;
     float* var;
@@ -1440,11 +1461,12 @@ __device__ __forceinline__ float adam_clip_scale(const AdamArgs& a) {
 // Workgroups [0, mat_tiles) update one 32 x 32 block-matrix tile each and
 // write it to the fragment-tiled copies as well; the rest update the vector
 // group and the head elementwise. Workgroup 0 also records the pre-clip norm.
-// PAIRS: the tiles go to the pair planes instead (policy_pair.h).
-template <bool PAIRS>
+// FP32: each tile's largest magnitude goes to PairScale.tilemax; PAIRS: the
+// tiles go to the pair planes instead of the copies (policy_pair.h).
+template <bool FP32, bool PAIRS>
 __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
     __shared__ float lds[kTT * kTileLd];
-    __shared__ float wmax[PAIRS ? 4 : 1];
+    __shared__ float wmax[FP32 ? 4 : 1];
     constexpr int PER = kTT * kTT / 256;  // tile elements per thread
     const int t = threadIdx.x;
     if (blockIdx.x < a.mat_tiles) {
@@ -1459,8 +1481,7 @@ __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
             in[e] = adam_load(a, idx[e]);
         }
         const uint32_t per = a.hidden * kEmbed / (kTT * kTT), mat = blockIdx.x / per;
-        PairScale* const pairs = PAIRS ? pair_scale(a.pair_fwd, a.count) : nullptr;
-        const int exp = PAIRS ? pairs->next[mat] : 0;
+        const int exp = PAIRS ? a.pairs->next[mat] : 0;
         const float scale = adam_clip_scale(a);
         float most = 0.0f;
 #pragma unroll
@@ -1468,21 +1489,20 @@ __global__ void __launch_bounds__(256) adam_kernel(const AdamArgs a) {
             const int r = (256 / kTT) * e + t / kTT;
             const float p = adam_elem(a, idx[e], in[e], scale);
             lds[r * kTileLd + c] = p;
-            if (PAIRS && fabsf(p) < __builtin_huge_valf()) most = fmaxf(most, fabsf(p));
+            if (FP32) most = fmaxf(most, finite_magnitude(p));
         }
-        if constexpr (PAIRS) {  // this tile's planes, and what the next step's exponent needs (PairScale)
-            most = group_max<64>(most);
-            if ((t & 63) == 0) wmax[t >> 6] = most;
-            __syncthreads();
+        if constexpr (FP32) {
+            most = wg_max(most, wmax);
             if (t == 0) {
-                pairs->tilemax[mat][blockIdx.x % per] = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-                if (blockIdx.x % per == 0) pairs->cur[mat] = exp;
+                a.pairs->tilemax[mat][blockIdx.x % per] = most;
+                if (PAIRS && blockIdx.x % per == 0) a.pairs->cur[mat] = exp;
             }
-            store_tile_pair(m, lds, a.pair_fwd, a.pair_bwd, mat & 1, exp);
-            return;
         }
-        store_tile_frags(m, lds, a.frag_fwd32, a.frag_fwd16, a.frag_bwd16, a.frag_fwd32_bf, a.frag_fwd16_bf,
-                         a.frag_bwd16_bf);
+        if constexpr (PAIRS)
+            store_tile_pair(m, lds, a.pair_fwd, a.pair_bwd, mat & 1, exp);
+        else
+            store_tile_frags(m, lds, a.frag_fwd32, a.frag_fwd16, a.frag_bwd16, a.frag_fwd32_bf, a.frag_fwd16_bf,
+                             a.frag_bwd16_bf);
         return;
     }
     const uint32_t j = (blockIdx.x - a.mat_tiles) * 256 + t;
@@ -1573,23 +1593,20 @@ bool rows_on_pairs(const mg_policy_view& pv) {
 }
 }  // namespace
 
-int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv) {
+int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv, bool trained) {
     int rc = check_matrix_layout(pv);
     if (rc) return rc;
-    const bool bf = pv.precision == MG_PRECISION_BF16, pairs = !bf && pv.frag_fwd16_bf && pv.frag_bwd16_bf;
-    uint16_t* split = bf ? nullptr : pv.frag_fwd32_bf;
-    if (split) {
-        hipLaunchKernelGGL(dev::split_scale_kernel, dim3(2 * pv.layers), dim3(1024), 0, st, pv.params, pv.float_group,
-                           (uint32_t)MG_EMBED * pv.hidden,
-                           const_cast<dev::SplitScale*>(dev::split_scale(split, pv.count)),
-                           pairs ? dev::pair_scale(pv.frag_fwd16_bf, pv.count) : nullptr);
-        MG_HIP(hipGetLastError(), "split scale launch");
+    const bool bf = pv.precision == MG_PRECISION_BF16;
+    if (!bf && !trained) {  // Adam leaves the tiles' magnitudes current
+        hipLaunchKernelGGL(dev::tile_max_kernel, dim3(mat_tiles(pv)), dim3(256), 0, st, pv.params, pv.float_group,
+                           pv.hidden, dev::pair_scale(pv.frag_fwd16_bf, pv.count));
+        MG_HIP(hipGetLastError(), "tile magnitudes launch");
     }
+    uint16_t* const none = nullptr;
     hipLaunchKernelGGL(dev::derive_blocks_kernel, dim3(mat_tiles(pv)), dim3(256), 0, st, pv.params, pv.frag_fwd32,
-                       pv.frag_fwd16, pv.frag_bwd16, bf ? pv.frag_fwd32_bf : nullptr,
-                       bf ? pv.frag_fwd16_bf : nullptr, bf ? pv.frag_bwd16_bf : nullptr, split,
-                       pairs ? pv.frag_fwd16_bf : nullptr, pairs ? pv.frag_bwd16_bf : nullptr, pv.count,
-                       pv.float_group, pv.hidden);
+                       pv.frag_fwd16, pv.frag_bwd16, bf ? pv.frag_fwd32_bf : none, bf ? pv.frag_fwd16_bf : none,
+                       bf ? pv.frag_bwd16_bf : none, bf ? none : pv.frag_fwd32_bf, bf ? none : pv.frag_fwd16_bf,
+                       bf ? none : pv.frag_bwd16_bf, trained && rows_on_pairs(pv), pv.count, pv.float_group, pv.hidden);
     MG_HIP(hipGetLastError(), "derive blocks launch");
     return MG_OK;
 }
@@ -1773,6 +1790,7 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         aa.frag_bwd16 = bf || pairs ? nullptr : pv.frag_bwd16;
         aa.pair_fwd = pairs ? pv.frag_fwd16_bf : nullptr;
         aa.pair_bwd = pairs ? pv.frag_bwd16_bf : nullptr;
+        aa.pairs = bf ? nullptr : dev::pair_scale(pv.frag_fwd16_bf, pv.count);
         aa.frag_fwd32_bf = nullptr;
         aa.frag_fwd16_bf = bf ? pv.frag_fwd16_bf : nullptr;
         aa.frag_bwd16_bf = bf ? pv.frag_bwd16_bf : nullptr;
@@ -1792,10 +1810,12 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         aa.max_grad_norm = hp.max_grad_norm;
         const uint32_t lin = pv.float_group + (pv.count - pv.off_head);
         const dim3 grid(aa.mat_tiles + (lin + 255) / 256);
-        if (pairs)
-            hipLaunchKernelGGL(dev::adam_kernel<true>, grid, dim3(256), 0, st, aa);
+        if (bf)
+            hipLaunchKernelGGL((dev::adam_kernel<false, false>), grid, dim3(256), 0, st, aa);
+        else if (pairs)
+            hipLaunchKernelGGL((dev::adam_kernel<true, true>), grid, dim3(256), 0, st, aa);
         else
-            hipLaunchKernelGGL(dev::adam_kernel<false>, grid, dim3(256), 0, st, aa);
+            hipLaunchKernelGGL((dev::adam_kernel<true, false>), grid, dim3(256), 0, st, aa);
         MG_HIP(hipGetLastError(), "adam launch");
     }
     return MG_OK;

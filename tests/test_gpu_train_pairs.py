@@ -47,3 +47,33 @@ def test_copies_follow_the_parameters(mg, lr, epochs):
     want = network64(model.pv, p, obs[1][256:512])
     err = np.abs(model.head() - want) / np.maximum(1.0, np.abs(want).max(1, keepdims=True))
     assert float(err.max()) <= 1e-4, float(err.max())
+
+
+@pytest.mark.parametrize("layers,lr", [(2, 3e-4), (2, 0.05), (2, 1.0), (5, 0.05)])
+def test_copies_after_training(mg, layers, lr):
+    """What a view hands out after training (exponents from the magnitudes that
+    Adam keeps per tile) is what the same parameters give when they are set:
+    every copy and the collects' exponents, bit for bit. 5 blocks: the fp32 row
+    pass, whose Adam does not write the pair planes."""
+    n = 512
+    gym = mg.Gym(ENVS["cartpole"][1], n, 0)
+    model = mg.PPOModel(gym, horizon=4, minibatch=256, layers=layers, lr=lr)
+    count, halves = model.pv.count, 2 * model.pv.count
+
+    def copies():
+        pv = model.policy()
+        scale = mg.d2h(pv.frag_fwd32_bf, np.uint16, (halves + 32,))[halves:].view(np.int32).reshape(2, 8)[:, :layers]
+        cur = mg.d2h(pv.frag_fwd16_bf, np.uint16, (halves + 32,))[halves:].view(np.int32)[:2 * layers]
+        got = {k: mg.d2h(getattr(pv, k), np.uint32, (count,)) for k in ("frag_fwd32", "frag_fwd16", "frag_bwd16")}
+        got.update({k: mg.d2h(getattr(pv, k), np.uint16, (halves,)) for k in ("frag_fwd32_bf", "frag_fwd16_bf",
+                                                                             "frag_bwd16_bf")})
+        return dict(got, scale=scale, cur=cur)
+
+    model.collect()
+    for _ in range(3):
+        model.train(2)
+        got = copies()
+        model.set_params(model.params())
+        want = copies()
+        for k in want:
+            np.testing.assert_array_equal(got[k], want[k], err_msg=k)
