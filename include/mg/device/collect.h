@@ -674,7 +674,7 @@ __global__ void __launch_bounds__(64 * kPairW, 1) collect_pair_kernel(const mg_c
 // (two workgroups per CU, one after the other) of an env with at most 16
 // observation floats and a register-held State. ms a collect of 32 steps,
 // CartPole, split_forward16 or the 32-row tiles against this: 0.63 / 0.40 at 64
-// envs, 0.65 / 0.46 at 4096, 1.34 / 0.83 at 8192 (collect_lane_kernel 1.06),
+// envs, 0.65 / 0.42 at 4096, 1.34 / 0.83 at 8192 (collect_lane_kernel 1.06),
 // 2.32 / 1.22 at 12288 (1.10). A step takes 14 us at 4096 envs, of
 // which the weights' 1 MB through each CU's L1 is about 11.
 template <typename Env>
@@ -735,13 +735,23 @@ void launch_collect_m(const mg_collect_args* a, hipStream_t st) {
     launch_collect_mw<Env, M, BF16, false>(a, st);
 }
 
+// The LDS bytes of a workgroup of collect_lane_kernel; 0 where that is more than
+// its share of a CU's. In fp32 the small parameters of a deep policy do not fit
+// beside the ring: one share takes up to 4 blocks of CartPole and 2 of VoxelNav
+// and VoxelNav16, two shares 8, and 7 of VoxelNav16.
+template <typename Env, int PREC, int HS>
+size_t collect_lane_bytes(uint32_t layers) {
+    using CL = CollectLane<Env, PREC, HS>;
+    const size_t lds = (size_t)lane_lds<PREC, CL::HC, HS>(layers, CL::WIN, CL::IO).total * 4;
+    return lds > 163840 / LaneShape<HS>::WG ? 0 : lds;
+}
+
 template <typename Env, int PREC, int HS>
 bool launch_collect_lane_as(const mg_collect_args* a, hipStream_t st) {
-    using CL = CollectLane<Env, PREC, HS>;
     using Sh = LaneShape<HS>;
-    if constexpr (CL::OK) {
-        const size_t lds = (size_t)lane_lds<PREC, CL::HC, HS>(a->policy.layers, CL::WIN, CL::IO).total * 4;
-        if (!a->policy.frag_fwd32_bf || lds > 163840 / Sh::WG) return false;
+    if constexpr (CollectLane<Env, PREC, HS>::OK) {
+        const size_t lds = collect_lane_bytes<Env, PREC, HS>(a->policy.layers);
+        if (!a->policy.frag_fwd32_bf || lds == 0) return false;
         hipLaunchKernelGGL((collect_lane_kernel<Env, PREC, HS>), dim3((a->n + Sh::TILE - 1) / Sh::TILE), dim3(kLaneNT),
                            lds, st, *a);
         return true;
@@ -756,14 +766,15 @@ bool launch_collect_lane_as(const mg_collect_args* a, hipStream_t st) {
 // binary16 products from 65536 (what the library's 8192^3 binary16 product
 // reaches here); at 16384 half the CUs have none, so there two shares take 64
 // envs a workgroup. ms a collect of 32 steps, CartPole, fp32, the tiles below (to
-// 8192 envs the 16-row tiles on pairs) / two shares / one: 0.87 / 1.06 / 1.32 at
+// 12288 envs the 16-row tiles on pairs) / two shares / one: 0.83 / 1.06 / 1.32 at
 // 8192 envs, 1.22 / 1.10 / 1.37 at 12288, 2.30 / 1.14 / 1.38 at 16384, 3.26 /
 // 2.08 / 1.43 at 24576, 8.44 / 4.18 / 2.86 at 65536. VoxelNav16, 16 steps: 0.83 /
 // 0.75 / 0.98 at 8192, 1.34 / 0.80 / 1.02 at 16384. bf16, 0.56 / 0.62 / 0.62 at
 // 16384, 0.71 / 1.20 / 0.63 at 20480, 0.87 / 1.21 / 0.68 at 32768: one share only.
 // An env of more than 32 observation floats spends its step on computing them
 // (VoxelNav's 32 ray marches), which the tiles spread over more threads, until
-// the grid is full: 16 steps, tiles / one share, fp32 2.37 / 3.16 at 16384 and 4.09 / 3.32 at 32768;
+// the grid is full. A policy too deep for the LDS (collect_lane_bytes) runs on the
+// tiles at every env count. 16 steps, tiles / one share, fp32 2.37 / 3.16 at 16384 and 4.09 / 3.32 at 32768;
 // bf16 2.34 / 2.93 at 32768, and 8 steps of 65536 2.48 / 1.92.
 template <typename Env, int PREC>
 bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
@@ -772,11 +783,10 @@ bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
         if (a->n < (F32 ? 32768u : 65536u)) return false;
     }
     if (a->n > 16384u) return launch_collect_lane_as<Env, PREC, 1>(a, st);
-    if constexpr (F32) {
-        if (a->n >= 8192u && launch_collect_lane_as<Env, PREC, 2>(a, st)) return true;
-        if (a->n == 16384u) return launch_collect_lane_as<Env, PREC, 1>(a, st);
-    }
-    return false;
+    if constexpr (F32)
+        return a->n >= 8192u && launch_collect_lane_as<Env, PREC, 2>(a, st);
+    else
+        return false;
 }
 
 template <typename Env, bool BF16>
