@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from parity import ENVS, THREADS
+from test_cpu_lane_limits import DEEPEST
 from test_gpu_collect import run_collect_parity
 
 pytestmark = pytest.mark.gpu
@@ -100,7 +101,7 @@ def test_forward_lane(mg, orc, env, rows, layers, scale, how):
     ("cartpole", 8192 + 64, 3, 2, 4, False),         # two shares of the hidden units
     ("cartpole", 16384, 2, 2, 4, False),
     ("cartpole_continuous", 10240, 2, 1, 1, False),  # two stages per share, one block
-    ("voxelnav16", 8192, 2, 8, 1, False),            # the deepest: W_in's place in LDS
+    ("voxelnav16", 8192, 2, 8, 1, False),            # a block too deep for the lane kernel's LDS: the 32-row tiles
     ("cartpole", 16384 + 64, 3, 2, 4, False),        # one share: half a workgroup at the end
     ("cartpole_continuous", 16448, 2, 1, 8, False),
     ("cartpole_continuous_clamp", 16384, 2, 8, 1, False),
@@ -122,6 +123,21 @@ def test_collect_lane(mg, orc, env, n, T, layers, scale, bf16):
         Gym, PPOModel = mg.Gym, Model
 
     run_collect_parity(Mg, orc, env, n, T, layers=layers, scale=scale, bf16=bf16)
+
+
+@pytest.mark.parametrize("env,shares,n,T,over", [
+    ("cartpole", 2, 8256, 2, 0),
+    ("voxelnav16", 2, 8192, 2, 0),   # W_in in LDS beside the deepest policy that leaves it room
+    ("cartpole", 1, 16448, 2, 0),
+    ("cartpole", 1, 16448, 2, 1),    # one block more: the tiles
+    ("voxelnav16", 1, 16448, 1, 0),
+    ("voxelnav16", 1, 16448, 1, 1),
+])
+def test_collect_lane_deepest(mg, orc, env, shares, n, T, over):
+    """The deepest policy on the lane kernel and, over, the first past its LDS."""
+    layers = DEEPEST[env, shares] + over
+    assert 1 <= layers <= 8
+    test_collect_lane(mg, orc, env, n, T, layers, 1, False)
 
 
 @pytest.mark.parametrize("env,n0,n1,T", [
