@@ -13,12 +13,12 @@ namespace dev {
 constexpr int kMaxObs = 64;   // OBS_DIM limit of the staged forward
 constexpr int kMaxHead = 64;  // ACT_DIM + 1 limit (model/ppo.h:117)
 
-// model/ppo.h:575-626 on `rows` obs rows; rows past the end compute on zeros
-// and are not stored.
-template <int M, bool BF16>
+// model/ppo.h:575-626 on `rows` obs rows with bf16 matmuls; rows past the end
+// compute on zeros and are not stored.
+template <int M>
 __global__ void __launch_bounds__(256) forward_kernel(const mg_policy_view pv, const float* __restrict__ obs,
                                                       uint32_t rows, float* __restrict__ head) {
-    __shared__ typename std::conditional<BF16, FwdSmemB<M>, FwdSmem<M>>::type sm;
+    __shared__ FwdSmemB<M> sm;
     __shared__ float obsL[M * kMaxObs];
     __shared__ float headL[M * kMaxHead];
     FwdRegs<M> R;
@@ -29,10 +29,7 @@ __global__ void __launch_bounds__(256) forward_kernel(const mg_policy_view pv, c
         obsL[idx] = r < rows ? obs[(size_t)row0 * O + idx] : 0.0f;
     }
     __syncthreads();
-    if constexpr (BF16)
-        policy_forward_b<M>(pv, small_params(pv), sm, R, obsL, O, headL, HD);
-    else
-        policy_forward<M>(pv, small_params(pv), sm, R, obsL, O, headL, HD);
+    policy_forward_b<M>(pv, small_params(pv), sm, R, obsL, O, headL, HD);
     for (int idx = threadIdx.x; idx < M * HD; idx += 256) {
         const uint32_t r = row0 + idx / HD;
         if (r < rows) head[(size_t)row0 * HD + idx] = headL[idx];
@@ -72,7 +69,7 @@ __global__ void __launch_bounds__(kLaneNT, 2) forward_lane_kernel(const mg_polic
 // The same in 16-row tiles with the fp32 products on pairs (policy_pair.h), one
 // workgroup per CU. Dynamic LDS: the small parameters, the observations and the
 // heads.
-__host__ __device__ __forceinline__ uint32_t forward_pair_floats(uint32_t O, uint32_t HD, uint32_t layers) {
+__host__ __device__ constexpr uint32_t forward_pair_floats(uint32_t O, uint32_t HD, uint32_t layers) {
     return O * kEmbed + kEmbed + (layers + 1) * 2 * kEmbed + kEmbed * HD + kSplitRows * (O + HD);
 }
 __global__ void __launch_bounds__(64 * kPairW, 1) forward_pair_kernel(const mg_policy_view pv,
@@ -227,19 +224,18 @@ bool try_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs
 // bf16 29.8 at 8192, 35.9 / 32 at 8193, 38 / 32 at 16384, 162 / 77 at 100003.
 template <int PREC>
 bool launch_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
-    if (rows <= 8192u || !pv.frag_fwd32_bf) return false;
+    if (rows <= 8192u) return false;
     return try_forward_lane<PREC, 4, 4>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 8, 32>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 16, 64>(st, pv, obs, rows, head);
 }
-// An fp32 forward of fewer rows, in the place of forward_kernel's 32-row tiles.
-bool launch_forward_pair(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
-    if (pv.precision != MG_PRECISION_FP32 || !pv.frag_fwd16_bf) return false;
+// An fp32 forward of fewer rows, or of a policy that the lane kernel does not take.
+void launch_forward_pair(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
+    static_assert(dev::forward_pair_floats(dev::kMaxObs, dev::kMaxHead, MG_MAX_LAYERS) * 4 + sizeof(dev::PairFwdSmem) <=
+                      163840, "the largest policy fits");
     const size_t lds = (size_t)dev::forward_pair_floats(pv.obs_dim, pv.head_dim, pv.layers) * 4;
-    if (lds + sizeof(dev::PairFwdSmem) > 163840) return false;
     hipLaunchKernelGGL(dev::forward_pair_kernel, dim3((rows + dev::kSplitRows - 1) / dev::kSplitRows),
                        dim3(64 * dev::kPairW), lds, st, pv, obs, rows, head);
-    return true;
 }
 }  // namespace
 
@@ -247,15 +243,12 @@ int launch_forward(hipStream_t st, const mg_policy_view& pv, const float* obs, u
     MG_CHECK(pv.obs_dim <= (uint32_t)dev::kMaxObs && pv.head_dim <= (uint32_t)dev::kMaxHead, MG_ERR_INVALID,
              "forward: OBS_DIM must be <= %d and ACT_DIM + 1 <= %d", dev::kMaxObs, dev::kMaxHead);
     if (rows == 0) return MG_OK;
-    if (pv.precision == MG_PRECISION_BF16 ? launch_forward_lane<MG_PRECISION_BF16>(st, pv, obs, rows, head)
-                                          : launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head) ||
-                                                launch_forward_pair(st, pv, obs, rows, head)) {
-    } else if (pv.precision == MG_PRECISION_BF16)
-        hipLaunchKernelGGL((dev::forward_kernel<32, true>), dim3((rows + 31) / 32), dim3(256), 0, st, pv, obs, rows,
-                           head);
-    else
-        hipLaunchKernelGGL((dev::forward_kernel<32, false>), dim3((rows + 31) / 32), dim3(256), 0, st, pv, obs, rows,
-                           head);
+    if (pv.precision == MG_PRECISION_BF16) {
+        if (!launch_forward_lane<MG_PRECISION_BF16>(st, pv, obs, rows, head))
+            hipLaunchKernelGGL(dev::forward_kernel<32>, dim3((rows + 31) / 32), dim3(256), 0, st, pv, obs, rows, head);
+    } else if (!launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head)) {
+        launch_forward_pair(st, pv, obs, rows, head);
+    }
     MG_HIP(hipGetLastError(), "forward launch");
     return MG_OK;
 }

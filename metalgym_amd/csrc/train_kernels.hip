@@ -1586,10 +1586,9 @@ int check_matrix_layout(const mg_policy_view& pv) {
 
 namespace {
 // Whether the fp32 row pass runs on binary16 pairs: wherever the 8-wave split
-// layout holds the policy and the planes are there.
+// layout holds the policy.
 bool rows_on_pairs(const mg_policy_view& pv) {
-    return pv.precision == MG_PRECISION_FP32 && pv.frag_fwd16_bf && pv.frag_bwd16_bf &&
-           dev::rows_split_waves(pv) == dev::kPairW;
+    return pv.precision == MG_PRECISION_FP32 && dev::rows_split_waves(pv) == dev::kPairW;
 }
 }  // namespace
 
@@ -1614,9 +1613,7 @@ int launch_derive_blocks(hipStream_t st, const mg_policy_view& pv, bool trained)
 // The weight-gradient jobs of one minibatch: per block, dUp and dDown from
 // the captures (T: their element type); tile x tile tiles.
 template <class T>
-dev::DwArgsT<T> dw_args(const mg_policy_view& pv, const TrainWs& ws, uint32_t B, uint32_t splits, uint32_t tile,
-                        uint32_t tile_n = 0) {
-    if (!tile_n) tile_n = tile;
+dev::DwArgsT<T> dw_args(const mg_policy_view& pv, const TrainWs& ws, uint32_t B, uint32_t splits, uint32_t tile) {
     const uint32_t E = MG_EMBED, H = pv.hidden;
     const T* x = reinterpret_cast<const T*>(ws.x);
     const T* v = reinterpret_cast<const T*>(ws.v);
@@ -1632,11 +1629,11 @@ dev::DwArgsT<T> dw_args(const mg_policy_view& pv, const TrainWs& ws, uint32_t B,
     for (uint32_t l = 0; l < pv.layers; ++l) {
         // dUp_l[k][j] = sum_r x_l[r][k] dV_l[r][j]  (model/mlp.metal:201-203)
         da.big[nb] = {x + (size_t)l * B * E, dv + (size_t)l * B * H, E, H, E, H, pv.off_up[l], 0};
-        da.tiles_per_big[nb] = (E / tile) * (H / tile_n);
+        da.tiles_per_big[nb] = (E / tile) * (H / tile);
         tiles += da.tiles_per_big[nb++];
         // dDown_l[j][c] = sum_r V_l[r][j] dh_l[r][c]  (model/mlp.metal:205-207)
         da.big[nb] = {v + (size_t)l * B * H, dh + (size_t)l * B * E, H, E, H, E, pv.off_down[l], 0};
-        da.tiles_per_big[nb] = (H / tile) * (E / tile_n);
+        da.tiles_per_big[nb] = (H / tile) * (E / tile);
         tiles += da.tiles_per_big[nb++];
     }
     da.nbig = nb;
@@ -1644,8 +1641,9 @@ dev::DwArgsT<T> dw_args(const mg_policy_view& pv, const TrainWs& ws, uint32_t B,
     return da;
 }
 
-// The split row pass with the head width's compile-time bound.
-template <int W, bool F16 = false>
+// The split row pass with the head width's compile-time bound: on pairs with
+// eight waves, in fp32 with four.
+template <int W, bool F16 = W == dev::kPairW>
 void launch_rows_split(hipStream_t st, uint32_t B, const mg_policy_view& pv, const dev::RowsArgs& ra) {
     if (pv.head_dim <= 4)
         hipLaunchKernelGGL((dev::train_rows_split_kernel<W, 4, F16>), dim3(B / dev::kTR), dim3(64 * W), 0, st, ra);
@@ -1696,9 +1694,7 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         if (bf)
             hipLaunchKernelGGL(dev::train_rows_kernel<true>, dim3(B / dev::kTR), dim3(dev::kTNT), 0, st, ra);
         else if (rows_on_pairs(pv))
-            launch_rows_split<dev::kPairW, true>(st, B, pv, ra);
-        else if (dev::rows_split_waves(pv) == 8)
-            launch_rows_split<8>(st, B, pv, ra);
+            launch_rows_split<dev::kPairW>(st, B, pv, ra);
         else if (dev::rows_split_waves(pv) == 4)
             launch_rows_split<4>(st, B, pv, ra);
         else
