@@ -549,16 +549,19 @@ __device__ __forceinline__ void lane_forward(const mg_policy_view& pv, const Lan
 // The split product's head differs from the fp32 tiles' (policy.h) in its last
 // bits, so a draw that falls within rounding of an edge of the CDF could pick
 // another action, and the env's rollout would go its own way from there. Such
-// draws (edge <= kLaneEdge, about one in 2^17 per edge) are decided by the row's
-// head as the tiles compute it, bit for bit: a seeded rollout takes the same
-// actions whichever kernel runs it. One wave recomputes one row, weights from
+// draws (edge <= kLaneEdge, one in 2^18 per edge) are decided by the row's
+// head as the tiles compute it, bit for bit: a seeded fp32 collect of a
+// categorical policy takes the same actions whichever kernel runs it, as long as
+// the two heads' edges are that close. Of a policy whose logits have a standard
+// deviation of 1 they are: the logits differ by at most 5.5e-6 over 2^21 rows,
+// an edge by a quarter of that. That grows with the head's weights: at 20, 2 of
+// 2^21 draws were decided otherwise. Gaussian and bfloat16 collects, and samples
+// of a forward's head, follow their own kernel's rounding. One wave recomputes one row, weights from
 // the arena, every sum in the tiles' order: an MFMA adds its k in order with
 // one rounding each (v_mfma_f32_32x32x2_f32 equals the chain of FMAs, checked
 // on 65536 sums of 128), the k of a group of 8 in the order 0, 4, 1, 5, 2, 6, 3,
 // 7 (policy.h's K-order permutation), a row's LN and head sums as trees over
 // CPT columns (32 in a 64-row tile, 16 in a 32-row tile), then over its threads.
-// The fp32 head of an initial policy moves a draw's edge by about 2^-25 of the
-// whole, of a trained one by 2^-21.
 constexpr float kLaneEdge = 0x1p-19f;
 constexpr int kLaneRowLds = 2 * kEmbed + 16;  // floats of scratch per wave
 
