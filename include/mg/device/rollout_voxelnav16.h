@@ -200,11 +200,13 @@ __global__ void __launch_bounds__(64) rollout_voxelnav16_kernel(const mg_rollout
                     r[p] = mine.row(((y | z) & ~15) == 0 ? (uint32_t)(16 * z + y) : 0u);
                 }
                 float o[kVnObs];
+                // an agent that the caller put outside the grid may be anywhere
+                const int sh = (px < -2 ? -2 : px > 17 ? 17 : px) + 2;
 #pragma unroll
                 for (int p = 0; p < 9; ++p) {
                     const int y = py + p % 3 - 1, z = pz + p / 3 - 1;
                     const uint32_t row = ((y | z) & ~15) == 0 ? r[p] : 0xFFFFu;
-                    const uint32_t c = ((row << 1) | 0x20001u) >> px;  // cells px - 1 .. px + 1, out-of-grid ones set
+                    const uint32_t c = ((row << 3) | 0xFFF80007u) >> sh;  // cells px - 1 .. px + 1, out-of-grid ones set
 #pragma unroll
                     for (int d = 0; d < 3; ++d) o[3 * p + d] = (float)((c >> d) & 1u);
                 }

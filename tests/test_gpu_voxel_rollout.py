@@ -56,3 +56,24 @@ def test_no_outputs(mg, orc):
     mg._capi.check(mg.lib().mg_gym_rollout_random(gym.h, 9, None, None, None, None))
     orc.rollout(g, 9, random=True, threads=THREADS)
     compare_gym(gym, g, "no outputs")
+
+
+def test_agents_outside_the_grid(mg, orc):
+    """Positions that the caller wrote, on the grid's sides and far off them:
+    every cell out there is occupied, and a step into the grid is allowed."""
+    eid, kernel = ENVS["voxelnav16"]
+    n, steps = 4096, 6
+    gym, g = mg.Gym(kernel, n, 5), orc.GymState(eid, n, 5)
+    gym.rollout_random(2)
+    orc.rollout(g, 2, random=True, threads=THREADS)
+    rs = np.random.default_rng(2)
+    position = g.state.reshape(n, -1)[:, :12].view(np.int32)
+    position[:] = np.where(rs.random((n, 3)) < 0.5, position,
+                           rs.choice(np.array([-33, -3, -2, -1, 0, 15, 16, 17, 18, 31, 32, 48], np.int32), (n, 3)))
+    mg.h2d(gym.buf.state, g.state)
+    bufs = gym.rollout_random(steps)
+    acts, obs, rew, dn = gym.download_slots(bufs, steps)
+    oa, oo, orw, od = orc.rollout(g, steps, random=True, threads=THREADS)
+    for got, want, what in ((acts, oa, "actions"), (obs, oo, "obs"), (rew, orw, "reward"), (dn, od, "done")):
+        assert_bit_exact(got, want, what)
+    compare_gym(gym, g, "after")
