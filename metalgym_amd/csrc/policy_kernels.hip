@@ -13,12 +13,12 @@ namespace dev {
 constexpr int kMaxObs = 64;   // OBS_DIM limit of the staged forward
 constexpr int kMaxHead = 64;  // ACT_DIM + 1 limit (model/ppo.h:117)
 
-// model/ppo.h:575-626 on `rows` obs rows with bf16 matmuls; rows past the end
-// compute on zeros and are not stored.
-template <int M>
+// model/ppo.h:575-626 on `rows` obs rows; rows past the end compute on zeros
+// and are not stored.
+template <int M, bool BF16>
 __global__ void __launch_bounds__(256) forward_kernel(const mg_policy_view pv, const float* __restrict__ obs,
                                                       uint32_t rows, float* __restrict__ head) {
-    __shared__ FwdSmemB<M> sm;
+    __shared__ typename std::conditional<BF16, FwdSmemB<M>, FwdSmem<M>>::type sm;
     __shared__ float obsL[M * kMaxObs];
     __shared__ float headL[M * kMaxHead];
     FwdRegs<M> R;
@@ -29,7 +29,10 @@ __global__ void __launch_bounds__(256) forward_kernel(const mg_policy_view pv, c
         obsL[idx] = r < rows ? obs[(size_t)row0 * O + idx] : 0.0f;
     }
     __syncthreads();
-    policy_forward_b<M>(pv, small_params(pv), sm, R, obsL, O, headL, HD);
+    if constexpr (BF16)
+        policy_forward_b<M>(pv, small_params(pv), sm, R, obsL, O, headL, HD);
+    else
+        policy_forward<M>(pv, small_params(pv), sm, R, obsL, O, headL, HD);
     for (int idx = threadIdx.x; idx < M * HD; idx += 256) {
         const uint32_t r = row0 + idx / HD;
         if (r < rows) head[(size_t)row0 * HD + idx] = headL[idx];
@@ -229,13 +232,21 @@ bool launch_forward_lane(hipStream_t st, const mg_policy_view& pv, const float* 
            try_forward_lane<PREC, 8, 32>(st, pv, obs, rows, head) ||
            try_forward_lane<PREC, 16, 64>(st, pv, obs, rows, head);
 }
-// An fp32 forward of fewer rows, or of a policy that the lane kernel does not take.
-void launch_forward_pair(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
+// An fp32 forward of fewer rows, or of a policy that the lane kernel does not
+// take, in the place of forward_kernel's 32-row tiles. Past 4096 rows (a
+// workgroup of 16 per CU) only for heads up to 8 columns: the head's columns are
+// added one after the other, twice there. us a call, forward_kernel / this, at
+// 4096 and 8192 rows, 1 block of hidden 128: 16 / 10 and 16 / 15 (3 columns), 22
+// / 12 and 22 / 19 (7), 28 / 23 and 29 / 43 (16), 75 / 68 and 77 / 132 (64); 8
+// blocks, at 100003 rows, 646 / 550 (7 columns) and 716 / 830 (16).
+bool launch_forward_pair(hipStream_t st, const mg_policy_view& pv, const float* obs, uint32_t rows, float* head) {
+    if (rows > 4096u && pv.head_dim > 8) return false;
     static_assert(dev::forward_pair_floats(dev::kMaxObs, dev::kMaxHead, MG_MAX_LAYERS) * 4 + sizeof(dev::PairFwdSmem) <=
                       163840, "the largest policy fits");
     const size_t lds = (size_t)dev::forward_pair_floats(pv.obs_dim, pv.head_dim, pv.layers) * 4;
     hipLaunchKernelGGL(dev::forward_pair_kernel, dim3((rows + dev::kSplitRows - 1) / dev::kSplitRows),
                        dim3(64 * dev::kPairW), lds, st, pv, obs, rows, head);
+    return true;
 }
 }  // namespace
 
@@ -243,11 +254,13 @@ int launch_forward(hipStream_t st, const mg_policy_view& pv, const float* obs, u
     MG_CHECK(pv.obs_dim <= (uint32_t)dev::kMaxObs && pv.head_dim <= (uint32_t)dev::kMaxHead, MG_ERR_INVALID,
              "forward: OBS_DIM must be <= %d and ACT_DIM + 1 <= %d", dev::kMaxObs, dev::kMaxHead);
     if (rows == 0) return MG_OK;
+    const dim3 tiles((rows + 31) / 32);
     if (pv.precision == MG_PRECISION_BF16) {
         if (!launch_forward_lane<MG_PRECISION_BF16>(st, pv, obs, rows, head))
-            hipLaunchKernelGGL(dev::forward_kernel<32>, dim3((rows + 31) / 32), dim3(256), 0, st, pv, obs, rows, head);
-    } else if (!launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head)) {
-        launch_forward_pair(st, pv, obs, rows, head);
+            hipLaunchKernelGGL((dev::forward_kernel<32, true>), tiles, dim3(256), 0, st, pv, obs, rows, head);
+    } else if (!launch_forward_lane<MG_PRECISION_FP32>(st, pv, obs, rows, head) &&
+               !launch_forward_pair(st, pv, obs, rows, head)) {
+        hipLaunchKernelGGL((dev::forward_kernel<32, false>), tiles, dim3(256), 0, st, pv, obs, rows, head);
     }
     MG_HIP(hipGetLastError(), "forward launch");
     return MG_OK;
