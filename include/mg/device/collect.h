@@ -676,12 +676,20 @@ __global__ void __launch_bounds__(64 * kPairW, 1) collect_pair_kernel(const mg_c
 // CartPole, split_forward16 or the 32-row tiles against this: 0.63 / 0.40 at 64
 // envs, 0.65 / 0.42 at 4096, 1.34 / 0.83 at 8192 (collect_lane_kernel 1.06),
 // 2.32 / 1.22 at 12288 (1.10). A step takes 14 us at 4096 envs, of
-// which the weights' 1 MB through each CU's L1 is about 11.
+// which the weights' 1 MB through each CU's L1 is about 11. At exactly 8192 a wide
+// head's env lanes (16 to a workgroup, a column after the other) cost more than
+// the products gain: 15 floats and 16 columns, 8 steps, 32-row tiles / this /
+// two shares 463 / 627 / 414 us; 3 and 5: 373 / 266 / 345. So do the steps
+// between the products of the smallest network, one block of 128 units: CartPole
+// 80 / 86 us.
 template <typename Env>
 bool launch_collect_pair(const mg_collect_args* a, hipStream_t st) {
     using CP = CollectPair<Env>;
     if constexpr (CP::OK) {
-        if (a->policy.precision != MG_PRECISION_FP32 || a->n > 8192u || !a->policy.frag_fwd16_bf) return false;
+        const bool least = a->policy.layers * a->policy.hidden <= 128u;
+        if (a->policy.precision != MG_PRECISION_FP32 || a->n > (CP::HD > 8 || least ? 8191u : 8192u) ||
+            !a->policy.frag_fwd16_bf)
+            return false;
         hipLaunchKernelGGL((collect_pair_kernel<Env>), dim3(a->n / kSplitRows), dim3(64 * kPairW),
                            CP::small(a->policy.layers) * 4, st, *a);
         return true;
@@ -776,17 +784,28 @@ bool launch_collect_lane_as(const mg_collect_args* a, hipStream_t st) {
 // the grid is full. A policy too deep for the LDS (collect_lane_bytes) runs on the
 // tiles at every env count. 16 steps, tiles / one share, fp32 2.37 / 3.16 at 16384 and 4.09 / 3.32 at 32768;
 // bf16 2.34 / 2.93 at 32768, and 8 steps of 65536 2.48 / 1.92.
+// Small networks stay on the tiles where those fill the GPU evenly (8192 envs are
+// one 32-row workgroup per CU, 16384 two, 32768 two of 64 rows) and the products
+// are too few to pay for the observations' slower way. us a collect of 8 steps,
+// tiles / lanes: VoxelNav16 at 8192 149 / 180 (1 block of 128), 275 / 288 (2 of
+// 256), 353 / 356 (2 of 384), 433 / 404 (2 of 512), but 402 / 289 (2 of 256) at
+// 8256; at 16384 189 / 198 (1 of 128), 261 / 224 (1 of 256); 4 steps of VoxelNav at
+// 32768 817 / 889 (1 of 128), 891 / 900 (1 of 256).
 template <typename Env, int PREC>
 bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
     constexpr bool F32 = PREC == MG_PRECISION_FP32;
+    const bool least = a->policy.layers * a->policy.hidden <= 128u;
     if constexpr (Env::OBS_DIM > 32) {
-        if (a->n < (F32 ? 32768u : 65536u)) return false;
+        if (a->n < (F32 ? (least ? 32769u : 32768u) : 65536u)) return false;
     }
     if (a->n > 16384u) return launch_collect_lane_as<Env, PREC, 1>(a, st);
-    if constexpr (F32)
-        return a->n >= 8192u && launch_collect_lane_as<Env, PREC, 2>(a, st);
-    else
+    if constexpr (F32) {
+        const uint32_t first = a->policy.hidden >= 512u ? 8192u : 8193u;
+        const uint32_t last = Env::OBS_DIM > 16 && least ? 16383u : 16384u;
+        return a->n >= first && a->n <= last && launch_collect_lane_as<Env, PREC, 2>(a, st);
+    } else {
         return false;
+    }
 }
 
 template <typename Env, bool BF16>

@@ -140,6 +140,21 @@ def test_collect_lane_deepest(mg, orc, env, shares, n, T, over):
     test_collect_lane(mg, orc, env, n, T, layers, 1, False)
 
 
+@pytest.mark.parametrize("env,n,T,layers,scale", [
+    # the tiles, where they fill the GPU evenly, and the lane kernels an env count on
+    ("cartpole", 8192, 3, 1, 1),
+    ("cartpole_continuous", 8192, 2, 1, 1),
+    ("voxelnav16", 8192, 2, 2, 3),
+    ("voxelnav16", 8256, 2, 2, 3),
+    ("voxelnav16", 16320, 2, 1, 1),
+    ("voxelnav16", 16384, 2, 1, 1),
+    ("voxelnav", 32768, 1, 1, 1),
+    ("voxelnav", 32832, 1, 1, 1),
+])
+def test_collect_small_networks(mg, orc, env, n, T, layers, scale):
+    test_collect_lane(mg, orc, env, n, T, layers, scale, False)
+
+
 @pytest.mark.parametrize("env,n0,n1,T", [
     ("voxelnav16", 8192, 16448, 32),   # two shares against one, both in the 32-row tiles' arithmetic
     ("cartpole", 8192, 16384, 96),     # 16-row tiles on pairs against two shares, the same
