@@ -169,7 +169,8 @@ void launch_split_rollout(const mg_rollout_args* a, hipStream_t st) {
 }
 
 // An env may bring a rollout kernel of its own (a specialisation with OK true,
-// seen before MG_DEFINE_ENV) that gives the same results as rollout_kernel.
+// seen before MG_DEFINE_ENV) that gives the same results as rollout_kernel, for
+// the launches that its takes() names.
 template <typename Env>
 struct PackedRollout {
     static constexpr bool OK = false;
@@ -185,8 +186,12 @@ int launch_rollout(const mg_rollout_args* a) {
     // over more CUs (4096 envs are 64 waves: 64 CUs instead of 16)
     hipStream_t st = static_cast<hipStream_t>(a->stream);
     if constexpr (PackedRollout<Env>::OK) {
-        PackedRollout<Env>::launch(a, st);
-    } else if constexpr (SplitRollout<Env>::OK) {
+        if (PackedRollout<Env>::takes(a)) {
+            PackedRollout<Env>::launch(a, st);
+            return (int)hipGetLastError();
+        }
+    }
+    if constexpr (SplitRollout<Env>::OK) {
         if (a->mode == MG_ACTIONS_RANDOM)
             launch_split_rollout<Env, MG_ACTIONS_RANDOM>(a, st);
         else

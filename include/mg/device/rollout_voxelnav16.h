@@ -2,8 +2,9 @@
 // one per lane, their grids in LDS as 256 rows of 16 bits (516 bytes an env in
 // the place of 4 KB).
 //
-// rollout_split_kernel stages the grids as bytes, of which LDS holds 36 to 38
-// per CU, and spreads a step's 27 gathers over threads behind two barriers. As
+// rollout_split_kernel, still the faster for what takes() leaves to it, stages
+// the grids as bytes, of which LDS holds 36 to 38 per CU, and spreads a step's 27
+// gathers over threads behind two barriers. As
 // bits, 256 envs fit a CU: a step is a lane's own (nine 16-bit row reads give
 // its 27 cells) and needs no barrier, and the observations leave through a
 // wave's LDS tile as 16-byte stores. A reset's 256 draws are spread over the
@@ -259,6 +260,16 @@ __global__ void __launch_bounds__(64) rollout_voxelnav16_kernel(const mg_rollout
 template <>
 struct PackedRollout<VoxelNav16> {
     static constexpr bool OK = true;
+    // Not the observations of a few envs, which the split kernel computes on more
+    // lanes: us a launch of 32 random steps, it against this, 24 / 29 for one env,
+    // 27 / 29.5 for 4, 32 / 30 for 8. Nor few steps of very many envs, which are the
+    // stream of their grids alone: one step 121 / 120 at 131072 envs, 147 / 152 at
+    // 163840, 229 / 241 at 262144; two 190 / 190 at 196544, 248 / 254 at 262144;
+    // four 208 / 208 and 270 / 274; eight 317 / 311.
+    static bool takes(const mg_rollout_args* a) {
+        const uint32_t many = a->steps == 1u ? 131073u : a->steps <= 4u ? 196608u : 0xFFFFFFFFu;
+        return !(a->n < 8u && a->obs_out) && a->n < many;
+    }
     template <int E>
     static void launch_e(const mg_rollout_args* a, hipStream_t st) {
         const dim3 grid((a->n + E - 1) / E), block(64);

@@ -10,7 +10,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,steps", [
-    (1, 300),       # one env
+    (1, 300),       # one env: the split kernel, as to 7
+    (7, 70),
+    (8, 70),
     (1027, 40),     # 8 envs per wave, the last partial (three of them)
     (9001, 12),     # 16 per wave, one in the last; rows that start off 16 bytes
     (32769, 5),     # 32 per wave, one in the last
@@ -76,4 +78,18 @@ def test_agents_outside_the_grid(mg, orc):
     oa, oo, orw, od = orc.rollout(g, steps, random=True, threads=THREADS)
     for got, want, what in ((acts, oa, "actions"), (obs, oo, "obs"), (rew, orw, "reward"), (dn, od, "done")):
         assert_bit_exact(got, want, what)
+    compare_gym(gym, g, "after")
+
+
+@pytest.mark.parametrize("n,lengths", [(131072, (1, 2)), (131073, (1, 2)), (196608, (4, 5))])
+def test_few_steps_of_many_envs(mg, orc, n, lengths):
+    """Either side of the split kernel's lines."""
+    eid, kernel = ENVS["voxelnav16"]
+    gym, g = mg.Gym(kernel, n, 3), orc.GymState(eid, n, 3)
+    for steps in lengths:
+        bufs = gym.rollout_random(steps)
+        got = gym.download_slots(bufs, steps)
+        want = orc.rollout(g, steps, random=True, threads=THREADS)
+        for x, y, what in zip(got, want, ("actions", "obs", "reward", "done")):
+            assert_bit_exact(x, y, f"{steps} steps {what}")
     compare_gym(gym, g, "after")
