@@ -509,7 +509,8 @@ def main():
         "dtype": "fp32",
         "data": "synthetic (seeded envs and weights)",
         "config": {"workload": "cartpole_collect_with_policy", "envs": n, "horizon": T, "embed": E, "hidden": H,
-                   "layers": L, "head": "softmax(2)+value", "parallelism": "single-gpu"},
+                   "layers": L, "head": "softmax(2)+value", "parallelism": "single-gpu",
+                   "block_products": "fp32 operands as two binary16 halves, three products, fp32 accumulation"},
         "roofline": {"bound": "mfma", "kernel": "collect_lane_kernel<CartPole,0,1>", "achieved": achieved / 1e12,
                      "peak": PEAK_PAIR_MFMA / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_PAIR_MFMA,
                      "traffic": pmc_traffic(),

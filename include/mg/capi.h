@@ -110,12 +110,13 @@ typedef struct mg_rollout_args {
  * frag_bwd16_bf up and down, rounded to bfloat16 (16-bit patterns), in the
  * operand order of the bf16 instructions (32x32x16 and 16x16x32: k-groups of
  * 16 and 32, each lane 8 consecutive k). With MG_PRECISION_FP32 the three hold
- * the same matrices in the same orders as pairs of binary16 values, each
- * element times a power of two of its matrix: the high halves at the arena
- * offsets, the low halves count elements later, then the matrices' exponents
- * (behind frag_fwd32_bf: SplitScale, policy_lane.h; behind frag_fwd16_bf, for
- * both 16-row orders: PairScale, policy_pair.h). Where frag_fwd32_bf or
- * frag_fwd16_bf is NULL an fp32 collect takes the fp32 copies. The fused
+ * the same matrices as pairs of binary16 values, each element times a power of
+ * two of its matrix: frag_fwd32_bf in its bf16 order, the high halves at the
+ * arena offsets, the low halves count elements later, then the exponents
+ * (SplitScale, policy_lane.h); frag_fwd16_bf and frag_bwd16_bf at twice the
+ * offsets, in groups of 32 hidden units with both halves (policy_pair.h), the
+ * exponents of both after frag_fwd16_bf's 2 count halves (PairScale). Where
+ * frag_fwd32_bf or frag_fwd16_bf is NULL an fp32 collect takes the fp32 copies. The fused
  * kernels read the matrices from all of these. The library derives them from
  * params at creation and in mg_ppo_set_params / mg_ppo_params_updated. A train
  * step (mg_ppo_train, mg_ppo_train_block, mg_ppo_train_block_noalloc) rewrites
@@ -255,7 +256,13 @@ typedef struct mg_ppo_config {
     uint32_t minibatch;
     uint32_t seed;
     float lr;
-    /* MG_PRECISION_FP32 (default), or MG_PRECISION_BF16: the block matmuls of
+    /* MG_PRECISION_FP32 (default): fp32 operands and results. The block matmuls'
+     * operands go through the matrix units as two binary16 halves (22 bits and
+     * the low half's sign; a weight under 2^-15 of its matrix's largest, or an
+     * activation as small beside its row's bound, keeps fewer), three products
+     * accumulated in fp32; the weight gradients of large minibatches as three
+     * bfloat16 parts (all 24 bits), six products. Against 64 bits both are as
+     * close as fp32 matrix instructions. MG_PRECISION_BF16: the block matmuls of
      * the forward, the backward and the weight gradients multiply bfloat16
      * operands (weights, LN outputs, hidden activations and their gradients)
      * with fp32 accumulation, as the reference's matmuls do; master weights,
@@ -338,7 +345,9 @@ int mg_ppo_train_block(mg_ppo* model, uint32_t block);
  * mg_ppo_train or mg_ppo_train_block, or MG_ERR_STATE if there was none). */
 int mg_ppo_train_block_noalloc(mg_ppo* model, uint32_t block, float* stats_out);
 /* model/ppo.h:628-634: policy forward on `rows` obs rows (device pointer) into
- * the model's head buffer. Blocking. */
+ * the model's head buffer. Blocking. The row count chooses the kernel (its
+ * lines: 4096 and 8192 rows), and each sums in its own order, so a row's head
+ * may differ in its last bits between calls of different row counts. */
 int mg_ppo_forward(mg_ppo* model, const float* obs, uint32_t rows);
 /* model/ppo.h:925-943 */
 int mg_ppo_last_stats(mg_ppo* model, mg_loss_stats* out);

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("env,n,T", [
     ("cartpole", 1024, 8),           # 16-row tiles, 8 waves
     ("cartpole", 8192, 4),           # 32-row tiles
-    ("cartpole", 64 * 576, 2),       # 64-row tiles
+    ("cartpole", 64 * 576, 2),       # row per lane pair
     ("cartpole_continuous", 2048, 4),
     ("voxelnav16", 1024, 4),         # 16-row tiles, 4 waves
     ("voxelnav", 1024, 4),           # heightmaps staged in LDS beside the bf16 tiles

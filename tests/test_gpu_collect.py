@@ -56,14 +56,14 @@ def run_collect_parity(mg, orc, env, n, T, layers=2, scale=4, seed=0, collects=2
     ("cartpole", 4096, 8),
     ("cartpole", 64, 1),         # the fewest envs (four 16-row tiles), one step
     ("cartpole", 192, 3),
-    ("cartpole", 64 * 576, 2),   # 64-row tiles (n >= 64 * 512)
+    ("cartpole", 64 * 576, 2),   # row per lane pair, one share
     ("cartpole_continuous", 2048, 8),
     ("cartpole_continuous_clamp", 2048, 8),
     ("voxelnav16", 1024, 8),
     ("voxelnav", 1024, 8),       # heightmaps staged in LDS: 16-row tiles
     ("voxelnav", 8192, 2),       # 32-row tiles, heightmaps in LDS (256 workgroups)
     ("voxelnav", 16384, 2),      # 32-row tiles, heightmaps in device memory, two workgroups per CU
-    ("voxelnav", 32768, 2),      # 64-row tiles, the same
+    ("voxelnav", 32768, 2),      # row per lane pair, heightmaps in device memory
 ])
 def test_collect_teacher_forced(mg, orc, env, n, T):
     run_collect_parity(mg, orc, env, n, T)
@@ -128,7 +128,7 @@ def test_collect_full_size_subset(mg, orc, env, n, block):
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
 def test_collect_and_forward_after_train(mg, orc, precision):
     """train() rewrites only the weight copies its own row pass reads; collect
-    (64-row tiles here, which read the 32-wide copies) and forward() after it
+    (here the row per lane pair, which reads the 32-wide 16-bit copies) and forward() after it
     must see the trained weights. The oracle continues from the GPU's env
     state after the first collect and replays the second one teacher-forced
     with the post-train parameters."""
@@ -170,7 +170,7 @@ def test_collect_and_forward_after_train(mg, orc, precision):
     (1024, 4, 3, 2),
     (1024, 2, 8, 1),     # the most blocks (MG_MAX_LAYERS), 16-row tiles
     (1024, 2, 2, 8),     # the widest hidden layer (1024), 16-row tiles
-    (8192, 2, 2, 8),     # 32-row tiles
+    (8192, 2, 2, 8),     # 16-row tiles, two workgroups a CU one after the other
     (32768, 2, 8, 1),    # 64-row tiles; 9 LNs: small parameters read from the arena, not LDS
 ])
 def test_collect_other_shapes(mg, orc, n, T, layers, scale):

@@ -2,8 +2,8 @@
 env's fused collect kernel launched through its descriptor
 (mg_env_desc.collect) with the view. A train step rewrites only the
 fragment-tiled copies that the next minibatch reads, so after training the
-copy that collect reads (frag_fwd32) lags the parameters until mg_ppo_policy
-re-derives it; a view taken after that call, or one held from before training
+copies that collect reads (frag_fwd32_bf, or frag_fwd32) lag the parameters
+until mg_ppo_policy re-derives them; a view taken after that call, or one held from before training
 (the pointers never change), collects exactly what mg_ppo_collect collects
 from the same env state."""
 import ctypes as C
@@ -52,8 +52,8 @@ def collect_with_view(mg, gym, pv, T, last_obs):
     }, bufs["head"].download(np.float32, (n, HD))
 
 
-@pytest.mark.parametrize("kernel,n", [("rollout_cartpole", 16384),                # 32-row tiles
-                                      ("rollout_cartpole_continuous", 65536)])   # 64-row tiles
+@pytest.mark.parametrize("kernel,n", [("rollout_cartpole", 16384),                # two shares of the hidden units
+                                      ("rollout_cartpole_continuous", 65536)])   # one
 def test_view_collect_after_training(mg, kernel, n):
     T = 4
     gym = mg.Gym(kernel, n, 2)
@@ -63,8 +63,10 @@ def test_view_collect_after_training(mg, kernel, n):
     model.train(1)
     count = model.pv.count
     frag_before = mg.d2h(held.frag_fwd32, np.float32, (count,))
+    pair_before = mg.d2h(held.frag_fwd32_bf, np.uint16, (count,))
     pv = model.policy()  # re-derives the copies that training left behind
     frag_after = mg.d2h(pv.frag_fwd32, np.float32, (count,))
+    assert not np.array_equal(pair_before, mg.d2h(pv.frag_fwd32_bf, np.uint16, (count,)))
     for f in ("params", "frag_fwd32", "frag_fwd16", "frag_bwd16"):
         assert getattr(pv, f) == getattr(held, f), f"{f} moved"
     assert not np.array_equal(frag_before, frag_after), "training left frag_fwd32 current: the test shows nothing"

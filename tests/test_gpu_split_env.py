@@ -57,13 +57,13 @@ def test_split_rollout_matches_step(envs, n, pair):
 @pytest.mark.parametrize("pair", ["raygrid", "rayfield"])
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("n", [
-    1024,    # 16-row tiles, states in LDS for both
+    1024,    # 16-row tiles, states in LDS for both (RayField in fp32: on pairs)
     8192,    # 32-row tiles, 256 workgroups: states in LDS for both
-    16384,   # 32-row tiles, 512 workgroups: the split env's states in device memory, two workgroups per CU
-    32768,   # 64-row tiles: both envs' states in device memory
+    16384,   # fp32 two shares of the hidden units; bf16 32-row tiles, the split env's states in device memory, two workgroups per CU
+    32768,   # row per lane pair, one share: states in device memory
 ])
 def test_split_collect_matches_step(envs, n, bf16, pair):
-    """RayField at 16384 and 32768 envs: the two-workgroup layout whose split
+    """RayField at 16384 and 32768 envs: the layouts whose split
     parts would read the states from device memory, where a register-held
     State is not written until the collect ends."""
     mg = envs
