@@ -676,20 +676,24 @@ __global__ void __launch_bounds__(64 * kPairW, 1) collect_pair_kernel(const mg_c
 // CartPole, split_forward16 or the 32-row tiles against this: 0.63 / 0.40 at 64
 // envs, 0.65 / 0.42 at 4096, 1.34 / 0.83 at 8192 (collect_lane_kernel 1.06),
 // 2.32 / 1.22 at 12288 (1.10). A step takes 14 us at 4096 envs, of
-// which the weights' 1 MB through each CU's L1 is about 11. At exactly 8192 a wide
-// head's env lanes (16 to a workgroup, a column after the other) cost more than
-// the products gain: 15 floats and 16 columns, 8 steps, 32-row tiles / this /
-// two shares 463 / 627 / 414 us; 3 and 5: 373 / 266 / 345. So do the steps
-// between the products of the smallest network, one block of 128 units: CartPole
-// 80 / 86 us.
+// which the weights' 1 MB through each CU's L1 is about 11. At exactly 8192 the
+// steps between the products of the smallest network, one block of 128 units,
+// cost more than the products gain: 8 steps of CartPole 80 us on the tiles, 86 here.
+// So does a wide head, whose columns the 16 env lanes of a workgroup take one after
+// the other: past 8 columns only networks of 1024 hidden units and more come
+// here, and fewer than 8192 envs. us a collect of 3 steps of 15 floats and 16
+// columns, tiles / this, at 64, 4096, 6144 and 8192 envs: 94 / 100, 98 / 114, 187 /
+// 199 and 83 / 145 (1 block of 128), 149 / 129, 160 / 150, 301 / 267 and 215 /
+// 320 (2 of 512); 16 steps of 4096 envs, 5 columns, 1 of 128, 103 / 107.
 template <typename Env>
 bool launch_collect_pair(const mg_collect_args* a, hipStream_t st) {
     using CP = CollectPair<Env>;
     if constexpr (CP::OK) {
-        const bool least = a->policy.layers * a->policy.hidden <= 128u;
-        if (a->policy.precision != MG_PRECISION_FP32 || a->n > (CP::HD > 8 || least ? 8191u : 8192u) ||
-            !a->policy.frag_fwd16_bf)
-            return false;
+        const uint32_t units = a->policy.layers * a->policy.hidden;
+        if (a->policy.precision != MG_PRECISION_FP32 || !a->policy.frag_fwd16_bf) return false;
+        if (a->n > (CP::HD > 8 || units <= 128u ? 8191u : 8192u)) return false;
+        if (CP::HD > 4 && units <= 128u) return false;
+        if (CP::HD > 8 && (units < 1024u || a->policy.hidden < 512u)) return false;
         hipLaunchKernelGGL((collect_pair_kernel<Env>), dim3(a->n / kSplitRows), dim3(64 * kPairW),
                            CP::small(a->policy.layers) * 4, st, *a);
         return true;
@@ -789,8 +793,10 @@ bool launch_collect_lane_as(const mg_collect_args* a, hipStream_t st) {
 // are too few to pay for the observations' slower way. us a collect of 8 steps,
 // tiles / lanes: VoxelNav16 at 8192 149 / 180 (1 block of 128), 275 / 288 (2 of
 // 256), 353 / 356 (2 of 384), 433 / 404 (2 of 512), but 402 / 289 (2 of 256) at
-// 8256; at 16384 189 / 198 (1 of 128), 261 / 224 (1 of 256); 4 steps of VoxelNav at
-// 32768 817 / 889 (1 of 128), 891 / 900 (1 of 256).
+// 8256; 1 of 128 at 8256 181 / 182 (one step 44 / 50), at 12288 199 / 193, at 16384
+// 189 / 198; 4 steps of VoxelNav at 32768 817 / 889 (1 of 128), 891 / 900 (1 of
+// 256). Heads of more than 8 columns likewise at 8192: 16 columns, 2 of 512, 215 /
+// 223 for 3 steps and 463 / 414 for 8.
 template <typename Env, int PREC>
 bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
     constexpr bool F32 = PREC == MG_PRECISION_FP32;
@@ -800,9 +806,9 @@ bool launch_collect_lane(const mg_collect_args* a, hipStream_t st) {
     }
     if (a->n > 16384u) return launch_collect_lane_as<Env, PREC, 1>(a, st);
     if constexpr (F32) {
-        const uint32_t first = a->policy.hidden >= 512u ? 8192u : 8193u;
-        const uint32_t last = Env::OBS_DIM > 16 && least ? 16383u : 16384u;
-        return a->n >= first && a->n <= last && launch_collect_lane_as<Env, PREC, 2>(a, st);
+        if (Env::OBS_DIM > 16 && least) return false;
+        const bool even = a->policy.hidden >= 512u && Env::ACT_DIM + 1 <= 8;
+        return a->n >= (even ? 8192u : 8193u) && launch_collect_lane_as<Env, PREC, 2>(a, st);
     } else {
         return false;
     }

@@ -34,13 +34,14 @@ def policy(mg, gym, T, layers, scale):
 
 
 @pytest.mark.parametrize("env", sorted(WIDTHS))
-# 16-row tiles, two shares (8192: of wide heads), one, and past 32 floats
+# 16-row tiles, 32-row ones (ramp15: its head is wide), two shares, one, and past 32 floats
 @pytest.mark.parametrize("n", [64, 8192, 8256, 16448, 32832])
-def test_collect(ramps, env, n):
+@pytest.mark.parametrize("layers,scale", [(2, 2), (2, 4), (1, 1)])
+def test_collect(ramps, env, n, layers, scale):
     mg, (O, A), T = ramps, WIDTHS[env], 3
     gym, twin = (mg.Gym("rollout_test_" + env, n, 2) for _ in range(2))
     assert (gym.obs_dim, gym.act_dim) == (O, A)
-    model, P = policy(mg, gym, T, 2, 2)
+    model, P = policy(mg, gym, T, layers, scale)
     model.collect()
     s = model.download_slots()
     # the first collect steps every env once with action 0 before the horizon
