@@ -150,6 +150,10 @@ struct LaneOps<MG_PRECISION_FP32> {
     // half of the other operand, with the fp32 product's sign (and NaN times 0).
     __device__ static __forceinline__ void pack_weights(const float (&x)[8], V (&p)[2]) {
         pack(x, p);
+        float m = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(x[j]));
+        if (m < 65520.0f) return;  // a NaN stays in both
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             if (!(fabsf(x[j]) < 65520.0f)) p[0][j] = (_Float16)0.0f, p[1][j] = (_Float16)x[j];
