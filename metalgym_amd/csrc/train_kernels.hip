@@ -1023,7 +1023,9 @@ constexpr int kDwf32Waves = 8, kDwf32U = 8, kDwf32Sets = 2;
 // overflows; the rest is exact in fp32): no scale is needed whatever the
 // gradients' range. Six products, hi hi + hi mid + mid hi + hi lo + lo hi + mid
 // mid, leave out terms of at most 2^-24 of a product, and a sum is rounded 6
-// times per 16 rows instead of 16 times (v_mfma_f32_32x32x2_f32).
+// times per 16 rows instead of 16 times (v_mfma_f32_32x32x2_f32). An infinite
+// operand gives NaN; the captures hold none without a NaN beside it (an
+// infinity in the row pass is NaN after its next LayerNorm, forward or backward).
 struct Planes3 {
     bf16x8 p[3];
 };
@@ -1064,6 +1066,13 @@ __device__ __forceinline__ void mma3(const Planes3 (&a)[2], const Planes3 (&b)[2
 // .. + 7 of its columns i and i + 32 of both operands as dwords straight from
 // the row-major captures (a half-wave reads one row's 128 bytes), one step
 // ahead.
+// The matrix unit's sums of a bfloat16 product come out a little short, each
+// time they are added up: in one chain over 16384 rows (128 steps of 6 products
+// a wave) a gradient's norm by 6.6e-7, which the clip passes on to every
+// gradient, where fp32 MFMA is 3e-8 off. So a chain is 2 kDw3Chain steps, added up in fp32:
+// norm 3.8e-8 off, a block's gradients 2.9e-7 (one chain 4.5e-7, fp32 MFMA 3.2e-7),
+// at the same 194 us (4 blocks of 1024; chains of 4 steps 197).
+constexpr uint32_t kDw3Chain = 4;
 template <int NW>
 __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, uint32_t tn, uint32_t rb,
                                          uint32_t steps, float* red) {
@@ -1080,7 +1089,7 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
                 y[h][j] = buffer_load4(bm.y, yv + 128 * h, 4 * (r + j) * bm.ldy);
             }
     };
-    f32x16 acc[2][2] = {};
+    f32x16 acc[2][2], sum[2][2] = {};
     float x[2][2][8], y[2][2][8];
     auto step = [&](int b) {
         Planes3 px[2], py[2];
@@ -1091,17 +1100,27 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
         mma3(px, py, acc);
     };
     load(x[0], y[0], w);
-    for (uint32_t s = w; s < steps; s += 2 * NW) {
-        load(x[1], y[1], s + NW);
-        __builtin_amdgcn_sched_barrier(0);
-        step(0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + NW < steps) {
-            load(x[0], y[0], s + 2 * NW);
+    for (uint32_t s = w; s < steps;) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[m][n] = f32x16{};
+        for (uint32_t end = s + 2 * kDw3Chain * NW; s < steps && s < end; s += 2 * NW) {
+            load(x[1], y[1], s + NW);
             __builtin_amdgcn_sched_barrier(0);
-            step(1);
+            step(0);
             __builtin_amdgcn_sched_barrier(0);
+            if (s + NW < steps) {
+                load(x[0], y[0], s + 2 * NW);
+                __builtin_amdgcn_sched_barrier(0);
+                step(1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) sum[m][n] += acc[m][n];
     }
     float* rw = red + w * 4096;
 #pragma unroll
@@ -1109,7 +1128,7 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) rw[(32 * m + c32_row(r, lane)) * 64 + 32 * n + i] = acc[m][n][r];
+            for (int r = 0; r < 16; ++r) rw[(32 * m + c32_row(r, lane)) * 64 + 32 * n + i] = sum[m][n][r];
     __syncthreads();
 }
 

@@ -77,3 +77,32 @@ def test_copies_after_training(mg, layers, lr):
         want = copies()
         for k in want:
             np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+
+
+@pytest.mark.parametrize("env,n,layers,scale", [
+    ("cartpole_continuous", 16384, 4, 8),  # all rows in one workgroup: 128 steps a wave
+    ("cartpole", 16384, 2, 4),             # row splits: 32
+    ("cartpole", 1088, 4, 8),              # 68 steps over 8 waves: chains that end short
+])
+def test_block_gradients_are_not_short(mg, env, n, layers, scale):
+    """The block matrices' gradients against float64 sums of the captures they are
+    made of: as close as fp32 sums, and not all a little too small, which the
+    norm and the clip would pass on to every parameter. The first moment is
+    fp32(1 - 0.9f) g clip; three roundings, the clip's two, common to all elements,
+    are up to 1.2e-7 (2^-24 each) together."""
+    gym = mg.Gym(ENVS[env][1], n, 0)
+    model = mg.PPOModel(gym, horizon=1, minibatch=n, layers=layers, scale=scale)
+    model.collect()
+    model.train_block(0)
+    pv, m = model.pv, model.adam_state()[0].astype(np.float64)
+    norm = np.float32(model.last_stats().grad_norm)
+    factor = float(np.float32(1) - np.float32(0.9)) * (float(np.float32(0.5) / (norm + np.float32(1e-6))) if norm > 0.5 else 1)
+    x, v, dh, dv = (model.train_capture(k) for k in range(4))
+    for l in (0, layers - 1):
+        for off, a, b in ((pv.off_up[l], x[l], dv[l]), (pv.off_down[l], v[l], dh[l])):
+            want = (a.astype(np.float64).T @ b.astype(np.float64)).ravel()
+            got = m[off:off + want.size] / factor
+            short = float(got @ want / (want @ want) - 1)
+            err = float(np.linalg.norm(got - want) / np.linalg.norm(want))
+            print(f"layer {l}: short by {short:.2e}, error {err:.2e}")
+            assert abs(short) <= 2e-7 and err <= 4e-7
