@@ -785,9 +785,9 @@ bool launch_collect_lane_as(const mg_collect_args* a, hipStream_t st) {
 // 16384, 0.71 / 1.20 / 0.63 at 20480, 0.87 / 1.21 / 0.68 at 32768: one share only.
 // An env of more than 32 observation floats spends its step on computing them
 // (VoxelNav's 32 ray marches), which the tiles spread over more threads, until
-// the grid is full. A policy too deep for the LDS (collect_lane_bytes) runs on the
-// tiles at every env count. 16 steps, tiles / one share, fp32 2.37 / 3.16 at 16384 and 4.09 / 3.32 at 32768;
-// bf16 2.34 / 2.93 at 32768, and 8 steps of 65536 2.48 / 1.92.
+// the grid is full: 16 steps, tiles / one share, fp32 2.37 / 3.16 at 16384 and
+// 4.09 / 3.32 at 32768; bf16 2.34 / 2.93 at 32768, and 8 steps of 65536 2.48 /
+// 1.92. A policy too deep for the LDS (collect_lane_bytes) runs on the tiles.
 // Small networks stay on the tiles where those fill the GPU evenly (8192 envs are
 // one 32-row workgroup per CU, 16384 two, 32768 two of 64 rows) and the products
 // are too few to pay for the observations' slower way. us a collect of 8 steps,

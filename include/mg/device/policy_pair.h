@@ -178,7 +178,8 @@ __device__ __forceinline__ int pair_store_input(PairInput& in, const RowVec<NV>&
     split_f16_scaled(x[2], x[3], opaque_v(f), h1, l1);
     typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
     f16x4 hi = {h0[0], h0[1], h1[0], h1[1]}, lo = {l0[0], l0[1], l1[0], l1[1]};
-    if (__any(m == __builtin_huge_valf())) {  // one branch in the chain from LN to the products: the selects alone took 0.1 us
+    // one branch in the chain from LN to the products: the selects alone took 0.1 us
+    if (__any(m == __builtin_huge_valf())) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             if (__builtin_isinf((float)hi[c])) lo[c] = hi[c], hi[c] = (_Float16)0.0f;

@@ -1344,7 +1344,7 @@ __device__ __forceinline__ void store_tile_pair(const MatTile& m, const float* l
     *reinterpret_cast<f16x8*>(out + 512) = p[1];
 }
 
-// The largest of f over a workgroup of 256, in thread 0, after a barrier; wmax
+// The largest m of a workgroup of 256, in every thread, after a barrier. wmax
 // holds 4.
 __device__ __forceinline__ float wg_max(float m, float* wmax) {
     m = group_max<64>(m);
@@ -1366,8 +1366,8 @@ __global__ void __launch_bounds__(256) tile_max_kernel(const float* __restrict__
     float most = 0.0f;
 #pragma unroll
     for (int e = 0; e < kTT * kTT / 256; ++e) {
-        const int r = (256 / kTT) * e + threadIdx.x / kTT;
-        most = fmaxf(most, finite_magnitude(param[m.base + (size_t)(m.r0 + r) * m.cols + m.c0 + (threadIdx.x & (kTT - 1))]));
+        const int r = (256 / kTT) * e + threadIdx.x / kTT, c = threadIdx.x & (kTT - 1);
+        most = fmaxf(most, finite_magnitude(param[m.base + (size_t)(m.r0 + r) * m.cols + m.c0 + c]));
     }
     most = wg_max(most, wmax);
     if (threadIdx.x == 0) pairs->tilemax[blockIdx.x / per][blockIdx.x % per] = most;
