@@ -1069,11 +1069,14 @@ __device__ __forceinline__ void mma3(const Planes3 (&a)[2], const Planes3 (&b)[2
 // The matrix unit's sums of a bfloat16 product come out a little short, each
 // time they are added up: in one chain over 16384 rows (128 steps of 6 products
 // a wave) a gradient's norm by 6.6e-7, which the clip passes on to every
-// gradient, where fp32 MFMA is 3e-8 off. So a chain is 2 kDw3Chain steps, added up in fp32:
-// norm 3.8e-8 off, a block's gradients 2.9e-7 (one chain 4.5e-7, fp32 MFMA 3.2e-7),
-// at the same 194 us (4 blocks of 1024; chains of 4 steps 197).
-constexpr uint32_t kDw3Chain = 4;
-template <int NW>
+// gradient, where fp32 MFMA is 3e-8 off. So past 32 steps (LONG) a chain is 16 of
+// them, added up in fp32: norm 3.8e-8 off, a block's gradients against float64
+// sums of their captures 6.7e-8 (one chain 4.2e-7, chains of 32 8.3e-8), at the
+// same time (4 blocks of 1024: 196.2 us, one chain 197.8). Up to 32 steps the
+// second set of sums costs time for little: 2 blocks of 512 (4096 rows a split)
+// 50.8 -> 52.2 us, from 8.0e-8 off to 6.4e-8.
+constexpr uint32_t kDw3Steps = 32, kDw3Chain = 16;
+template <int NW, bool LONG>
 __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, uint32_t tn, uint32_t rb,
                                          uint32_t steps, float* red) {
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
@@ -1089,7 +1092,7 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
                 y[h][j] = buffer_load4(bm.y, yv + 128 * h, 4 * (r + j) * bm.ldy);
             }
     };
-    f32x16 acc[2][2], sum[2][2] = {};
+    f32x16 acc[2][2] = {}, sum[2][2] = {};
     float x[2][2][8], y[2][2][8];
     auto step = [&](int b) {
         Planes3 px[2], py[2];
@@ -1101,11 +1104,8 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
     };
     load(x[0], y[0], w);
     for (uint32_t s = w; s < steps;) {
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int n = 0; n < 2; ++n) acc[m][n] = f32x16{};
-        for (uint32_t end = s + 2 * kDw3Chain * NW; s < steps && s < end; s += 2 * NW) {
+        const uint32_t end = LONG ? s + kDw3Chain * NW : steps;
+        for (; s < steps && s < end; s += 2 * NW) {
             load(x[1], y[1], s + NW);
             __builtin_amdgcn_sched_barrier(0);
             step(0);
@@ -1117,10 +1117,11 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (LONG)
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+            for (int m = 0; m < 2; ++m)
 #pragma unroll
-            for (int n = 0; n < 2; ++n) sum[m][n] += acc[m][n];
+                for (int n = 0; n < 2; ++n) sum[m][n] += acc[m][n], acc[m][n] = f32x16{};
     }
     float* rw = red + w * 4096;
 #pragma unroll
@@ -1128,7 +1129,7 @@ __device__ __forceinline__ void dw3_tile(const BigMatT<float>& bm, uint32_t tm, 
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) rw[(32 * m + c32_row(r, lane)) * 64 + 32 * n + i] = sum[m][n][r];
+            for (int r = 0; r < 16; ++r) rw[(32 * m + c32_row(r, lane)) * 64 + 32 * n + i] = (LONG ? sum : acc)[m][n][r];
     __syncthreads();
 }
 
@@ -1150,7 +1151,7 @@ __device__ __forceinline__ void dw3_locate(uint32_t t, uint32_t per, uint32_t& m
 // 512, 53.0 + 8.8 against 71.7 with 2 blocks at 16384 rows, 30.2 + 6.5 against
 // 44.5 with 4 at 4096, 19.1 + 6.4 against 21.5 with 2 at 4096; hence the line at
 // twice the work of 2 blocks at 4096 rows (launch_train_step).
-template <int NW>
+template <int NW, bool LONG>
 __global__ void __launch_bounds__(64 * NW) train_dw3_kernel(const DwArgsT<float> a) {
     __shared__ float red[NW * 4096];
     const uint32_t item = xcd_item(blockIdx.x, gridDim.x), split = item / a.big_tiles, t = item % a.big_tiles;
@@ -1159,7 +1160,7 @@ __global__ void __launch_bounds__(64 * NW) train_dw3_kernel(const DwArgsT<float>
     const BigMatT<float>& bm = a.big[mi];
     const bool up = bm.mdim == (uint32_t)kEmbed;
     const uint32_t tm = up ? eb : hb, tn = up ? hb : eb, per = a.rows / a.splits;
-    dw3_tile<NW>(bm, tm, tn, split * per, per / 16, red);
+    dw3_tile<NW, LONG>(bm, tm, tn, split * per, per / 16, red);
     float* out = a.partial + (size_t)split * a.count + bm.off + (size_t)tm * 64 * bm.ndim + tn * 64;
     for (int e = threadIdx.x; e < 4096; e += 64 * NW) {
         float v = red[e];
@@ -1174,7 +1175,7 @@ __global__ void __launch_bounds__(64 * NW) train_dw3_kernel(const DwArgsT<float>
 // 1024, 16384 rows: 368 -> 190 us. The captures' 604 MB take 116 us from HBM and
 // the products 85 us; a wave's splits (176 vector instructions per 24 MFMAs)
 // overlap its SIMD's other wave's MFMAs only in part.
-template <int NW>
+template <int NW, bool LONG>
 __global__ void __launch_bounds__(64 * NW) train_dw3_fused_kernel(const DwFusedArgs<float> a) {
     __shared__ float red[NW * 4096];
     float sq = 0.0f;
@@ -1187,7 +1188,7 @@ __global__ void __launch_bounds__(64 * NW) train_dw3_fused_kernel(const DwFusedA
         const BigMatT<float>& bm = a.dw.big[mi];
         const bool up = bm.mdim == (uint32_t)kEmbed;
         const uint32_t tm = up ? eb : hb, tn = up ? hb : eb;
-        dw3_tile<NW>(bm, tm, tn, 0, a.dw.rows / 16, red);
+        dw3_tile<NW, LONG>(bm, tm, tn, 0, a.dw.rows / 16, red);
         float* out = a.red.grad + bm.off + (size_t)tm * 64 * bm.ndim + tn * 64;
         for (int e = threadIdx.x; e < 4096; e += 64 * NW) {
             float v = red[e];
@@ -1749,8 +1750,11 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
         fa.dw = dw_args<float>(pv, ws, B, 1, 64);
         fa.red = ga;
         const uint32_t grid = tiles64 + ga.small_wgs <= (uint32_t)kReduceBlocks ? tiles64 + ga.small_wgs : tiles64;
-        hipLaunchKernelGGL((dev::train_dw3_fused_kernel<dev::kDw3Waves>), dim3(grid), dim3(64 * dev::kDw3Waves), 0, st,
-                           fa);
+        const dim3 threads(64 * dev::kDw3Waves);
+        if (B > 16 * dev::kDw3Waves * dev::kDw3Steps)
+            hipLaunchKernelGGL((dev::train_dw3_fused_kernel<dev::kDw3Waves, true>), dim3(grid), threads, 0, st, fa);
+        else
+            hipLaunchKernelGGL((dev::train_dw3_fused_kernel<dev::kDw3Waves, false>), dim3(grid), threads, 0, st, fa);
         MG_HIP(hipGetLastError(), "train dW launch");
     } else if (bf && tiles32 >= 128 && tiles32 <= (uint32_t)kReduceBlocks && B % (16 * dev::kDwfWaves) == 0) {
         TimedLaunch tl(MG_K_TRAIN_DW, st);
@@ -1782,8 +1786,13 @@ int launch_train_step(hipStream_t st, const mg_policy_view& pv, const mg_ppo_hpa
                                    dim3(64 * dev::kDwbWaves), 0, st, da);
             } else {
                 const auto da = dw_args<float>(pv, ws, B, splits, 64);
-                hipLaunchKernelGGL((dev::train_dw3_kernel<dev::kDw3Waves>), dim3(dw_tiles * splits),
-                                   dim3(64 * dev::kDw3Waves), 0, st, da);
+                const dim3 threads(64 * dev::kDw3Waves);
+                if (B / splits > 16 * dev::kDw3Waves * dev::kDw3Steps)
+                    hipLaunchKernelGGL((dev::train_dw3_kernel<dev::kDw3Waves, true>), dim3(dw_tiles * splits), threads,
+                                       0, st, da);
+                else
+                    hipLaunchKernelGGL((dev::train_dw3_kernel<dev::kDw3Waves, false>), dim3(dw_tiles * splits), threads,
+                                       0, st, da);
             }
             MG_HIP(hipGetLastError(), "train dW launch");
         }

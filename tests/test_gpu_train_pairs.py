@@ -81,8 +81,10 @@ def test_copies_after_training(mg, layers, lr):
 
 @pytest.mark.parametrize("env,n,layers,scale", [
     ("cartpole_continuous", 16384, 4, 8),  # all rows in one workgroup: 128 steps a wave
-    ("cartpole", 16384, 2, 4),             # row splits: 32
-    ("cartpole", 1088, 4, 8),              # 68 steps over 8 waves: chains that end short
+    ("cartpole", 16384, 2, 4),             # row splits: 32, the most in one chain
+    ("cartpole", 4160, 4, 8),              # 260 steps over 8 waves: chains that end short
+    ("cartpole", 81920, 2, 4),             # row splits past it
+    ("cartpole", 1088, 4, 8),              # 68 steps over 8 waves
 ])
 def test_block_gradients_are_not_short(mg, env, n, layers, scale):
     """The block matrices' gradients against float64 sums of the captures they are
